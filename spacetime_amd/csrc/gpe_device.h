@@ -4,6 +4,7 @@
 
 #include "gpe_internal.h"
 
+#include <cstddef>
 #include <type_traits>
 
 namespace gpe {
@@ -65,6 +66,28 @@ __device__ __forceinline__ int sweep_order(const Geometry &g, int b, int nb, int
 {
     if (!order) return b;
     return g.xcd_remap ? reverse_in_xcd(b, nb) : nb - 1 - b;
+}
+
+// Wave-uniform read-only data through scalar loads that the compiler neither hoists out of a loop
+// nor keeps: the pointer passes through an empty asm, so every call's loads are its own.
+template <typename T>
+using const_ptr = const __attribute__((address_space(4))) T *;
+
+template <typename T>
+__device__ __forceinline__ const_ptr<T> fresh(const T *p)
+{
+    const_ptr<T> q = (const_ptr<T>)(unsigned long long)p;
+    asm volatile("" : "+s"(q));
+    return q;
+}
+
+// A member of the kernel's argument (its only one, a struct) at `offset`.
+template <typename T>
+__device__ __forceinline__ const_ptr<T> fresh_args(unsigned offset)
+{
+    const_ptr<char> q = (const_ptr<char>)__builtin_amdgcn_kernarg_segment_ptr() + offset;
+    asm volatile("" : "+s"(q));
+    return (const_ptr<T>)q;
 }
 
 struct WaveCoord {
@@ -225,11 +248,27 @@ __device__ __forceinline__ void spin_dot(R wx, R wy, R wz, const R *pr, const R 
         spin2_dot<R>(wx, wy, wz, pr, pi, orr, oi);
 }
 
-struct LocalCoef {
-    double vtrap;
-    double Bx, By, Bz;
-    double Qx, Qy, Qz;
-};
+// Spin density psi^dag f psi (not divided by n).
+template <typename R, int C>
+__device__ __forceinline__ void spin_density(const R *pr, const R *pi, R &Fx, R &Fy, R &Fz)
+{
+    if constexpr (C == 3) {
+        // F+ = sqrt2 (conj(psi1) psi0 + conj(psi0) psi-1), Fz = |psi1|^2 - |psi-1|^2
+        const R s2 = (R)1.41421356237309504880;
+        Fx = s2 * (pr[0] * pr[1] + pi[0] * pi[1] + pr[1] * pr[2] + pi[1] * pi[2]);
+        Fy = s2 * (pr[0] * pi[1] - pi[0] * pr[1] + pr[1] * pi[2] - pi[1] * pr[2]);
+        Fz = pr[0] * pr[0] + pi[0] * pi[0] - pr[2] * pr[2] - pi[2] * pi[2];
+    } else {
+        const R s6 = (R)2.44948974278317809820;
+        // F+ = 2 c(psi2) psi1 + s6 c(psi1) psi0 + s6 c(psi0) psi-1 + 2 c(psi-1) psi-2
+        Fx = 2 * (pr[0] * pr[1] + pi[0] * pi[1]) + s6 * (pr[1] * pr[2] + pi[1] * pi[2]) +
+             s6 * (pr[2] * pr[3] + pi[2] * pi[3]) + 2 * (pr[3] * pr[4] + pi[3] * pi[4]);
+        Fy = 2 * (pr[0] * pi[1] - pi[0] * pr[1]) + s6 * (pr[1] * pi[2] - pi[1] * pr[2]) +
+             s6 * (pr[2] * pi[3] - pi[2] * pr[3]) + 2 * (pr[3] * pi[4] - pi[3] * pr[4]);
+        Fz = 2 * (pr[0] * pr[0] + pi[0] * pi[0]) + pr[1] * pr[1] + pi[1] * pi[1] - pr[3] * pr[3] -
+             pi[3] * pi[3] - 2 * (pr[4] * pr[4] + pi[4] * pi[4]);
+    }
+}
 
 // hr/hi += local part of H psi at one unknown.
 template <typename R, int C>
@@ -250,24 +289,12 @@ __device__ __forceinline__ void add_local_h(const R *pr, const R *pi, R vtrap, R
     }
     if constexpr (C > 1) {
         R Fx, Fy, Fz, wx, wy, wz;
+        spin_density<R, C>(pr, pi, Fx, Fy, Fz);
         if constexpr (C == 3) {
-            // F+ = sqrt2 (conj(psi1) psi0 + conj(psi0) psi-1), Fz = |psi1|^2 - |psi-1|^2
-            const R s2 = (R)1.41421356237309504880;
-            Fx = s2 * (pr[0] * pr[1] + pi[0] * pi[1] + pr[1] * pr[2] + pi[1] * pi[2]);
-            Fy = s2 * (pr[0] * pi[1] - pi[0] * pr[1] + pr[1] * pi[2] - pi[1] * pr[2]);
-            Fz = pr[0] * pr[0] + pi[0] * pi[0] - pr[2] * pr[2] - pi[2] * pi[2];
             wx = Bx + c1 * Fx;
             wy = By + c1 * Fy;
             wz = Bz + c1 * Fz;
         } else {
-            const R s6 = (R)2.44948974278317809820;
-            // F+ = 2 c(psi2) psi1 + s6 c(psi1) psi0 + s6 c(psi0) psi-1 + 2 c(psi-1) psi-2
-            Fx = 2 * (pr[0] * pr[1] + pi[0] * pi[1]) + s6 * (pr[1] * pr[2] + pi[1] * pi[2]) +
-                 s6 * (pr[2] * pr[3] + pi[2] * pi[3]) + 2 * (pr[3] * pr[4] + pi[3] * pi[4]);
-            Fy = 2 * (pr[0] * pi[1] - pi[0] * pr[1]) + s6 * (pr[1] * pi[2] - pi[1] * pr[2]) +
-                 s6 * (pr[2] * pi[3] - pi[2] * pr[3]) + 2 * (pr[3] * pi[4] - pi[3] * pr[4]);
-            Fz = 2 * (pr[0] * pr[0] + pi[0] * pi[0]) + pr[1] * pr[1] + pi[1] * pi[1] - pr[3] * pr[3] -
-                 pi[3] * pi[3] - 2 * (pr[4] * pr[4] + pi[4] * pi[4]);
             // spin-2 linear Zeeman enters with -B (Spin2GpeBCC.cu:942-957)
             wx = c1 * Fx - Bx;
             wy = c1 * Fy - By;

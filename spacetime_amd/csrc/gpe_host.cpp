@@ -67,6 +67,9 @@ struct gpe_ctx {
     const LatticeTable *lat = nullptr;
     Geometry g{};    // one x per lane: observables, packing, adjoint
     Geometry gs{};   // the sweep's geometry (1 or 2 x per lane)
+    Geometry gr{};   // the reductions' geometry (one x per lane over row groups)
+    int gr_segs = 1;    // 64-slot segments of a row group that a wave of it takes
+    int red_blocks = 1; // workgroups of a reduction: as many as run at once
     Physics ph{};
     int fp64 = 0;
     size_t elem_bytes = 0;   // bytes of one complex element
@@ -76,6 +79,8 @@ struct gpe_ctx {
     void *level[2] = {nullptr, nullptr};
     // tables
     int *d_face = nullptr, *d_nface = nullptr, *d_facex = nullptr;
+    int *d_oface = nullptr, *d_nfwd = nullptr;  // the observables' faces (ObsArgs)
+    double *d_ow = nullptr;
     float *d_w32 = nullptr, *d_wsum32 = nullptr, *d_pos32 = nullptr;
     double *d_w64 = nullptr, *d_wsum64 = nullptr, *d_pos64 = nullptr, *d_dv = nullptr;
     // fields per sweep
@@ -86,6 +91,7 @@ struct gpe_ctx {
     double *d_partials = nullptr;
     double *d_scalars = nullptr;   // [0..15] results / scales
     double *d_red = nullptr;       // FIN_SCRATCH doubles: first-stage results of launch_finalize
+    double *h_red = nullptr;       // pinned: results the host reads (FIN_WIDTH_MAX doubles)
     // static field and ramp
     double bq = 0, bb[3] = {0, 0, 0}, bqq = 0, bbq[3] = {0, 0, 0};
     Ramp ramp;
@@ -299,6 +305,42 @@ bool finish_geometry(Geometry &g)
     return true;
 }
 
+// Traversal of a reduction over a level: one x per lane, the rows of a tile as one group whose
+// slots (row, x) fill whole waves.  The tile is the lowest of 8-32 rows whose waves carry within
+// 3% of the most values (57-value lines, 57 rows: 19 rows 99% against 8 rows 87%, and one row
+// a wave 89%; 16-value lines one row a wave 25%).  A wave takes a chunk of the group's segments:
+// all of them where the groups alone give every wave of the launch one, fewer in smaller boxes.
+// Needs a finished g; its waves are never more than g's.
+Geometry reduce_geometry(const Geometry &g, int blocks, int *segs)
+{
+    Geometry r = g;
+    r.xpl = 1;
+    r.v_inner = 0;
+    r.pairs = g.nx;
+    const auto segments = [&](int rows) { return ((long long)rows * g.nx + 63) / 64; };
+    const auto use = [&](int ty) {  // values per lane slot of the waves that hold any
+        const long long waves = (g.ny / ty) * segments(ty) + (g.ny % ty ? segments(g.ny % ty) : 0);
+        return (double)g.ny * g.nx / (64.0 * waves);
+    };
+    const int lo = std::min(8, g.ny), hi = std::min(32, g.ny);
+    double best = 0.0;
+    for (int ty = lo; ty <= hi; ++ty) best = std::max(best, use(ty));
+    for (r.ty = lo; use(r.ty) < best - 0.03;) ++r.ty;
+    r.rows = r.ty;
+    r.tyr = 1;
+    r.ntile = (g.ny + r.ty - 1) / r.ty;
+    const long long groups = (long long)r.ntile * g.nz * g.V, each = segments(r.ty);
+    const long long parts = std::min(each, std::max(1ll, 4 * blocks / groups));
+    *segs = (int)((each + parts - 1) / parts);
+    r.nseg = (int)((each + *segs - 1) / *segs);
+    r.waves = groups * r.nseg;
+    r.blocks = (int)((r.waves + 3) / 4);
+    r.f_nseg = make_fast_div((unsigned)r.nseg);
+    r.f_ty = make_fast_div(1u);
+    r.f_pairs = make_fast_div((unsigned)g.nx);
+    return r;
+}
+
 // Layout of a configuration's levels and its default traversal (one x per lane, tiles of 8 rows,
 // XCD remap), before finish_geometry.
 Geometry base_geometry(const gpe_config &cfg)
@@ -360,6 +402,59 @@ SweepArgs sweep_args(gpe_ctx *c, int mode_coef_sweep, const void *cur, void *nex
     a.scale_in = nullptr;
     a.partials = c->d_partials;
     return a;
+}
+
+// Reduction partials: AUX_COUNT doubles a workgroup of the one-x-per-lane traversal, one of the
+// sweep's (norm partials), OBS_COUNT of a reduction's.
+size_t partials_bytes(const gpe_ctx *c)
+{
+    const size_t per_block = sizeof(double) * AUX_COUNT * (size_t)std::max(c->g.blocks, c->gs.blocks);
+    return std::max(per_block, sizeof(double) * OBS_COUNT * RED_BLOCKS_MAX);
+}
+
+// Sums over a level (gpe_observables_t) into d_scalars[8...] and the pinned h_red.
+hipError_t reduce_observables(gpe_ctx *c, int level, double t)
+{
+    const FieldRec f = field_at(c, t);
+    const Physics &ph = c->ph;
+    ObsArgs oa;
+    oa.g = c->gr;
+    oa.tb = tables(c);
+    oa.face = c->d_oface;
+    oa.w = c->d_ow;
+    oa.nfwd = c->d_nfwd;
+    oa.psi = c->level[level];
+    oa.quad = quad_active(c);
+    ObsConsts &k = oa.k;
+    const bool trap_on = t < ph.trap_off_time;
+    const double sign = c->cfg.ncomp == 5 ? -1.0 : 1.0;
+    k.sig = f.sigma;
+    k.ik = -1.0 / (f.sigma * f.sigma);
+    k.off = trap_on ? ph.trap_offset : 0.0;
+    k.bq = sign * f.bq;
+    k.bqq = f.bqq;
+    for (int a = 0; a < 3; ++a) {
+        k.p0[a] = ph.p0[a];
+        k.cell[a] = f.sigma * ph.cell[a];
+        k.ht[a] = trap_on ? 0.5 * ph.trap2[a] : 0.0;
+        k.center[a] = ph.center[a];
+        k.bb[a] = sign * f.bb[a];
+        k.bbq[a] = f.bbq[a];
+    }
+    k.quad_sign = ph.quad_sign;
+    k.q = ph.q;
+    k.hc0 = 0.5 * ph.c0;
+    k.hc1 = 0.5 * ph.c1;
+    k.c2_10 = ph.c2 / 10.0;
+    oa.segs = c->gr_segs;
+    oa.per = (c->gr.blocks + c->red_blocks - 1) / c->red_blocks;
+    oa.blocks = ((c->gr.blocks + oa.per - 1) / oa.per + 7) / 8 * 8;
+    oa.partials = c->d_partials;
+    hipError_t e = launch_observables(c->fp64, c->cfg.ncomp, oa, c->stream);
+    if (e == hipSuccess)
+        e = launch_finalize_few(c->d_partials, oa.blocks, OBS_COUNT, OBS_MAXDENS, c->d_scalars + 8, c->h_red,
+                                c->stream);
+    return e;
 }
 
 int check_level(gpe_ctx *c, int level)
@@ -461,6 +556,9 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     if ((e = hipGetDevice(&c->device)) != hipSuccess) rc = hip_fail(c, e, "hipGetDevice");
     if (!rc && (e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess)
         rc = hip_fail(c, e, "hipStreamCreate");
+    if (!rc && (e = observables_resident(c->fp64, cfg->ncomp, c->device, &c->red_blocks)) != hipSuccess)
+        rc = hip_fail(c, e, "occupancy");
+    c->gr = reduce_geometry(g, c->red_blocks, &c->gr_segs);
     const size_t lbytes = (size_t)c->level_elems * c->elem_bytes;
     for (int l = 0; l < 2 && !rc; ++l) {
         if ((e = hipMalloc(&c->level[l], lbytes)) != hipSuccess)
@@ -473,7 +571,8 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     const double s = cfg->block_scale;
     std::vector<double> w64(V * deg), wsum64(V, 0.0), pos64(3 * V), dv(V);
     std::vector<float> w32(V * deg), wsum32(V), pos32(3 * V);
-    std::vector<int> nface(V), facex(2 * V * deg);
+    std::vector<int> nface(V), facex(2 * V * deg), oface(2 * V * deg), nfwd(V);
+    std::vector<double> ow(V * deg);
     for (int v = 0; v < V; ++v) {
         for (int f = 0; f < deg; ++f) {
             const int pk = c->lat->face[v * deg + f];
@@ -492,6 +591,20 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
             wsum64[v] += w;
         }
         wsum32[v] = (float)wsum64[v];
+        // the observables' order: faces to a higher address (offset between the two unknowns, dx
+        // included), the others, then the pad faces
+        int o = v * deg;
+        for (int pass = 0; pass < 3; ++pass) {
+            for (int f = 0; f < deg; ++f) {
+                const int pk = facex[2 * (v * deg + f)], off = facex[2 * (v * deg + f) + 1];
+                const int kind = f >= nf ? 2 : (off + (pk & 3) - 1 > 0 ? 0 : 1);
+                if (kind != pass) continue;
+                oface[2 * o] = pk;
+                oface[2 * o + 1] = off;
+                ow[o++] = w64[v * deg + f];
+            }
+            if (pass == 0) nfwd[v] = o - v * deg;
+        }
         for (int k = 0; k < 3; ++k) {
             pos64[3 * v + k] = s * c->lat->pos[3 * v + k];
             pos32[3 * v + k] = (float)pos64[3 * v + k];
@@ -511,6 +624,9 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     up((void **)&c->d_face, c->lat->face, sizeof(int) * V * deg);
     up((void **)&c->d_nface, nface.data(), sizeof(int) * V);
     up((void **)&c->d_facex, facex.data(), sizeof(int) * 2 * V * deg);
+    up((void **)&c->d_oface, oface.data(), sizeof(int) * 2 * V * deg);
+    up((void **)&c->d_ow, ow.data(), sizeof(double) * V * deg);
+    up((void **)&c->d_nfwd, nfwd.data(), sizeof(int) * V);
     up((void **)&c->d_w32, w32.data(), sizeof(float) * V * deg);
     up((void **)&c->d_w64, w64.data(), sizeof(double) * V * deg);
     up((void **)&c->d_wsum32, wsum32.data(), sizeof(float) * V);
@@ -518,7 +634,8 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     up((void **)&c->d_pos32, pos32.data(), sizeof(float) * 3 * V);
     up((void **)&c->d_pos64, pos64.data(), sizeof(double) * 3 * V);
     up((void **)&c->d_dv, dv.data(), sizeof(double) * V);
-    if (!rc && hipMalloc((void **)&c->d_partials, sizeof(double) * OBS_COUNT * (size_t)g.blocks) != hipSuccess)
+    if (!rc && hipMalloc((void **)&c->d_partials, partials_bytes(c)) != hipSuccess) rc = GPE_ENOMEM;
+    if (!rc && hipHostMalloc((void **)&c->h_red, sizeof(double) * FIN_WIDTH_MAX, hipHostMallocDefault) != hipSuccess)
         rc = GPE_ENOMEM;
     if (!rc && hipMalloc((void **)&c->d_scalars, sizeof(double) * 64) != hipSuccess) rc = GPE_ENOMEM;
     if (!rc && hipMalloc((void **)&c->d_red, sizeof(double) * FIN_SCRATCH) != hipSuccess) rc = GPE_ENOMEM;
@@ -540,11 +657,12 @@ int gpe_destroy(gpe_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (int l = 0; l < 2; ++l)
         if (c->level[l]) (void)hipFree(c->level[l]);
-    void *ptrs[] = {c->d_face, c->d_nface, c->d_facex, c->d_w32, c->d_w64, c->d_wsum32, c->d_wsum64, c->d_pos32,
+    void *ptrs[] = {c->d_face, c->d_nface, c->d_facex, c->d_oface, c->d_ow, c->d_nfwd, c->d_w32, c->d_w64, c->d_wsum32, c->d_wsum64, c->d_pos32,
                     c->d_pos64, c->d_dv, c->d_fields, c->d_partials, c->d_scalars, c->d_red};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_fields) (void)hipHostFree(c->h_fields);
+    if (c->h_red) (void)hipHostFree(c->h_red);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -734,16 +852,7 @@ int gpe_itp(gpe_ctx *c, int nsteps, double dt_itp)
     double *norm = c->d_scalars + 0;
     double *scale[2] = {c->d_scalars + 1, c->d_scalars + 2};
     // initial scale from the norm of level 0
-    ObsArgs oa;
-    oa.g = c->g;
-    oa.tb = tables(c);
-    oa.ph = c->ph;
-    oa.psi = c->level[0];
-    oa.field = field_at(c, c->t0 + c->sweeps * sweep_dt(c));
-    oa.quad = quad_active(c);
-    oa.partials = c->d_partials;
-    hipError_t e = launch_observables(c->fp64, c->cfg.ncomp, oa, c->stream);
-    if (e == hipSuccess) e = launch_finalize(c->d_partials, c->g.blocks, OBS_COUNT, OBS_MAXDENS, c->d_scalars + 8, c->d_red, c->stream);
+    hipError_t e = reduce_observables(c, 0, c->t0 + c->sweeps * sweep_dt(c));
     if (e == hipSuccess) e = launch_norm_to_scale(c->d_scalars + 8 + OBS_NORM, 1.0, scale[0], c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "ITP initial norm");
     for (int i = 0; i < nsteps; ++i) {
@@ -770,20 +879,10 @@ int gpe_observables(gpe_ctx *c, int level, gpe_observables_t *out)
     int rc = check_level(c, level);
     if (rc) return rc;
     const double t = c->t0 + (double)(c->sweeps - level) * sweep_dt(c);
-    ObsArgs oa;
-    oa.g = c->g;
-    oa.tb = tables(c);
-    oa.ph = c->ph;
-    oa.psi = c->level[level];
-    oa.field = field_at(c, t);
-    oa.quad = quad_active(c);
-    oa.partials = c->d_partials;
-    hipError_t e = launch_observables(c->fp64, c->cfg.ncomp, oa, c->stream);
-    if (e == hipSuccess) e = launch_finalize(c->d_partials, c->g.blocks, OBS_COUNT, OBS_MAXDENS, c->d_scalars + 8, c->d_red, c->stream);
+    const hipError_t e = reduce_observables(c, level, t);
     if (e != hipSuccess) return hip_fail(c, e, "observables");
-    double h[OBS_COUNT];
-    HIPCALL(c, hipMemcpyAsync(h, c->d_scalars + 8, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     HIPCALL(c, hipStreamSynchronize(c->stream));
+    const double *h = c->h_red;
     out->norm = h[OBS_NORM];
     out->energy = h[OBS_ENERGY];
     out->expect_h = h[OBS_EXPECT_H];
@@ -1654,14 +1753,14 @@ static bool set_traversal(gpe_ctx *c, int ty, int flags, int xpl)
     return true;
 }
 
-// Reduction partials are sized by the workgroups of the one-x-per-lane traversal.
-static int grow_partials(gpe_ctx *c, int blocks_before)
+// Reduction partials after a change of traversal; `before` their size then.
+static int grow_partials(gpe_ctx *c, size_t before)
 {
-    if (c->g.blocks <= blocks_before) return GPE_OK;
+    if (partials_bytes(c) <= before) return GPE_OK;
     HIPCALL(c, hipStreamSynchronize(c->stream));
     (void)hipFree(c->d_partials);
     c->d_partials = nullptr;
-    if (hipMalloc((void **)&c->d_partials, sizeof(double) * OBS_COUNT * (size_t)c->g.blocks) != hipSuccess)
+    if (hipMalloc((void **)&c->d_partials, partials_bytes(c)) != hipSuccess)
         return fail(c, GPE_ENOMEM, "partials");
     return GPE_OK;
 }
@@ -1673,7 +1772,7 @@ int gpe_set_traversal(gpe_ctx *c, int tile_rows, int xcd_remap, int x_per_lane)
         return fail(c, GPE_EINVAL, "bad traversal");
     if (x_per_lane == 2 && !pair_lanes_ok(c->fp64, c->g.deg, c->cfg.ncomp))
         return fail(c, GPE_EINVAL, "two x per lane needs FP32");
-    const int before = c->g.blocks;
+    const size_t before = partials_bytes(c);
     if (!set_traversal(c, tile_rows, xcd_remap, x_per_lane))
         return fail(c, GPE_EINVAL, "traversal needs more workgroups than the decode supports");
     return grow_partials(c, before);
@@ -1743,7 +1842,7 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
     if (!c) return GPE_EINVAL;
     if (trial_sweeps < 0) return fail(c, GPE_EINVAL, "negative trial sweeps");
     const TuneKey key(c->cfg.lattice, c->cfg.ncomp, c->fp64, c->cfg.nx, c->cfg.ny, c->cfg.nz);
-    const int max_blocks_before = c->g.blocks;
+    const size_t partials_before = partials_bytes(c);
     int best_ty = c->g.ty, best_remap = c->gs.xcd_remap | (c->gs.v_inner << 1), best_xpl = c->gs.xpl;
     double best_ms = -1.0;
     {
@@ -1820,7 +1919,7 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
     }
     if (!set_traversal(c, best_ty, best_remap, best_xpl))
         return fail(c, GPE_EINVAL, "traversal needs more workgroups than the decode supports");
-    int rc = grow_partials(c, max_blocks_before);
+    int rc = grow_partials(c, partials_before);
     if (rc) return rc;
     if (tile_rows) *tile_rows = best_ty;
     if (xcd_remap) *xcd_remap = best_remap;

@@ -150,15 +150,33 @@ enum { FIELD_DENSITY = 0, FIELD_SPIN = 1, FIELD_SPIN_NORM = 2, FIELD_UV_THETA = 
 hipError_t launch_local_fields(int fp64, int ncomp, const Geometry &g, const void *psi, int kind, double *out,
                                hipStream_t s);
 
+// Constants of the observables, combined on the host.
+struct ObsConsts {
+    double p0[3], cell[3], sig;     // cell edges times the grid's scale factor sig
+    double ik;                      // -1 / sig^2
+    double ht[3], off;              // half the squared trap frequencies and the offset; 0 once the trap is off
+    double center[3];
+    double bq, bb[3];               // linear Zeeman field with its sign (- for spin-2)
+    double bqq, bbq[3], quad_sign, q;
+    double hc0, hc1, c2_10;         // c0 / 2, c1 / 2, c2 / 10
+};
+
 struct ObsArgs {
     Geometry g;
     Tables tb;
-    Physics ph;
+    ObsConsts k;
+    const int *face;          // V*deg pairs (packed face, line offset) as Tables::facex, the faces to a
+    const double *w;          // higher address first (nfwd[v] of them), pad faces last; weights likewise
+    const int *nfwd;
     const void *psi;
-    FieldRec field;
     int quad;
+    int segs;                 // 64-slot segments of a wave's chunk
+    int blocks, per;          // workgroups, and chunks each of their waves takes
     double *partials;         // OBS_COUNT per workgroup
 };
+
+// Most workgroups of a reduction whose waves keep their sums over many unknowns: 8 a CU.
+constexpr int RED_BLOCKS_MAX = 2048;
 
 // Per-unknown bound of the local Hamiltonian (maxHamilton) and the weighted distance to a
 // reference state (weightedDiff), reduced per workgroup: partials[2 b] = max, [2 b + 1] = sum.
@@ -258,6 +276,8 @@ hipError_t launch_fill_tf(int fp64, const Geometry &g, const Tables &tb, const P
 hipError_t launch_sweep(int fp64, int ncomp, int mode, const SweepArgs &a, hipStream_t s);
 hipError_t launch_aux(int fp64, int ncomp, const AuxArgs &a, hipStream_t s);
 hipError_t launch_observables(int fp64, int ncomp, const ObsArgs &a, hipStream_t s);
+// workgroups of the observables kernel that the device runs at once (at most RED_BLOCKS_MAX)
+hipError_t observables_resident(int fp64, int ncomp, int device, int *blocks);
 // sum `n` partial records of `width` doubles into out[width] (max for column maxcol, if >= 0)
 // scratch: FIN_SCRATCH doubles of device memory owned by the caller's context.
 constexpr int FIN_WIDTH_MAX = 16;
@@ -268,6 +288,10 @@ hipError_t launch_sum_tables(const double *partials, int nslot, int n, int width
                              hipStream_t s);
 hipError_t launch_finalize(const double *partials, int n, int width, int maxcol, double *out, double *scratch,
                            hipStream_t s);
+// the same for at most RED_BLOCKS_MAX records, in one launch; the results also go to `host` (pinned)
+// unless it is null
+hipError_t launch_finalize_few(const double *partials, int n, int width, int maxcol, double *out, double *host,
+                               hipStream_t s);
 // out = sqrt(target / in[0])
 hipError_t launch_norm_to_scale(const double *in, double target, double *out, hipStream_t s);
 // level *= factor (device scalar if dfactor != nullptr)

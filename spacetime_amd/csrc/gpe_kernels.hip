@@ -590,157 +590,240 @@ __global__ void k_set_base(int *base, int value)
 
 // ------------------------------------------------------------------------ observables --
 
-template <typename R, int C, int DEG>
+// A wave's part of a reduction (reduce_geometry): a chunk of the 64-slot segments of one group of
+// y rows of (z, v); slot p of the group is row p / nx, x = p mod nx.
+struct RedCoord {
+    int v, z, y0, nrow;  // the group's first row and its rows in the box
+    unsigned slot0;      // the chunk's first slot
+};
+
+__device__ __forceinline__ bool decode_reduce(const Geometry &g, int segs, unsigned w, RedCoord &rc)
+{
+    if ((long long)w >= g.waves) return false;
+    int chunk;
+    const unsigned q1 = split_v_seg(g, w, &rc.v, &chunk);
+    const unsigned q2 = fast_div(q1, g.f_nz);
+    rc.z = (int)(q1 - q2 * (unsigned)g.nz);
+    rc.y0 = (int)q2 * g.ty;
+    rc.nrow = g.ny - rc.y0 < g.rows ? g.ny - rc.y0 : g.rows;
+    rc.slot0 = (unsigned)(chunk * segs * 64);
+    return true;
+}
+
+// FP64 observables of a level.  Vector instructions bind it, not bytes: spin-1 128^3 FP32 reads
+// 604 MB (92 us at the copy rate) and issues 98 M of them (159 us at 4 cycles a wave and SIMD), in
+// 241 us of kernel time; 770 us with one unknown a lane and an exchange per wave of 64.  So:
+//   * a lane keeps its 14 sums over all the unknowns it takes and the wave exchanges them once;
+//   * the kinetic energy is summed over the faces, each once: with dv_i w_ij = dv_j w_ji (the dual
+//     volumes are solved from it) Re sum_i dv_i psi_i* sum_j w_ij (psi_j - psi_i) is
+//     -sum over faces of dv_i w_ij |psi_i - psi_j|^2, and -dv_i w_ij |psi_i|^2 for a face at the
+//     box's boundary.  A face belongs to the unknown that finds the other one at a higher address
+//     (the first nfwd[v] of its row of the table), so a lane loads two neighbours, not four;
+//   * the decode serves all segments of the wave's chunk.
+// U segments go together (two for one component, 202 -> 208 us on Cube 293^3 with one; three
+// components lose a wave a SIMD with two, 296 -> 316 us): the own values and the first four faces'
+// neighbours are in flight at once.  Tables, weights and constants are read again in every step
+// (scalar loads, fresh()): kept across the loop they take more scalar registers than there are, and
+// the spills cost more (447 us).
+template <typename R, int C, int U>
 __global__ __launch_bounds__(256) void k_observables(ObsArgs a)
 {
     using V2 = vec2_t<R>;
     const Geometry &g = a.g;
-    const WaveCoord wc = decode(g);
+    const unsigned wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // XCD k (blocks k, k + 8, ...: gridDim.x is a multiple of 8) has a contiguous range of the
+    // traversal, which its workgroups walk side by side: the rows and planes a wave needs are what
+    // the others read at the same time (each workgroup on a range of its own read a level 2.4 times)
+    const unsigned each = gridDim.x >> 3;
+    const unsigned first = ((blockIdx.x & 7u) * each * (unsigned)a.per + (blockIdx.x >> 3)) * 4u + wid;
+    const V2 *__restrict__ psi = (const V2 *)a.psi;
+    const long long cstride = comp_stride(g);
+    const int deg = g.deg;
+    constexpr int FB = 4;
     double acc[OBS_COUNT];
 #pragma unroll
     for (int i = 0; i < OBS_COUNT; ++i) acc[i] = 0.0;
+    bool bad = false;
 
-    if (wc.valid && wc.x < g.nx) {
-        const int x = wc.x, v = wc.v, y = wc.y, z = wc.z;
-        const V2 *__restrict__ psi = (const V2 *)a.psi;
-        double pr[C], pi[C], kr[C], ki[C];
+    for (int j = 0; j < a.per; ++j) {
+        RedCoord rc;
+        if (!decode_reduce(g, a.segs, first + 4u * each * (unsigned)j, rc)) break;
+        const int v = rc.v, z = rc.z;
+        const V2 *base = psi + line_index(g, 0, z, rc.y0, v);  // the group's first row
+        // every y / z neighbour of the group inside the box
+        const bool inner = z >= 1 && z <= g.nz - 2 && rc.y0 >= 1 && rc.y0 + rc.nrow <= g.ny - 1;
+        const int nfwd = fresh(a.nfwd + v)[0], nf = fresh(a.tb.nface + v)[0];
+        const unsigned rows = (unsigned)rc.nrow, slots = rows * (unsigned)g.nx;
+        const unsigned end = rc.slot0 + 64u * (unsigned)a.segs < slots ? rc.slot0 + 64u * (unsigned)a.segs : slots;
+        for (unsigned s = rc.slot0; s < end; s += 64u * U) {
+            int x[U], y[U], at[U];
+            bool live[U];
+            const const_ptr<int2> fx = fresh((const int2 *)a.face + v * deg);
+            int2 face[FB];
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const V2 o = psi[line_index(g, c, z, y, v) + x];
-            pr[c] = o.x;
-            pi[c] = o.y;
-            kr[c] = 0;
-            ki[c] = 0;
-        }
-        const int *face = a.tb.face + v * DEG;
-        const double *wt = a.tb.w64 + v * DEG;
+            for (int f = 0; f < FB; ++f) {
+                face[f].x = fx[f].x;
+                face[f].y = fx[f].y;
+            }
+            V2 own[U][C], nb[U][FB][C];
+            double ekin[U];
+            // whether a face's neighbour is inside the box
+            auto inside = [&](int u, int pk) {
+                const int dx = (pk & 3) - 1, dy = ((pk >> 2) & 3) - 1, dz = ((pk >> 4) & 3) - 1;
+                return (unsigned)(x[u] + dx) < (unsigned)g.nx && (unsigned)(z + dz) < (unsigned)g.nz &&
+                       (unsigned)(y[u] + dy) < (unsigned)g.ny;
+            };
+            // an outside neighbour reads the lane's own value: |psi_i - psi_i|^2 adds nothing
+            auto load = [&](int u, int f, int2 e) {
+                int off = at[u] + e.y + (e.x & 3) - 1;
+                if (!inner || (e.x & 3) != 1) off = inside(u, e.x) ? off : at[u];
 #pragma unroll
-        for (int f = 0; f < DEG; ++f) {
-            const int pk = face[f];
-            const int dx = (pk & 3) - 1, dy = ((pk >> 2) & 3) - 1, dz = ((pk >> 4) & 3) - 1, t = pk >> 8;
-            const int zn = z + dz, yn = y + dy, xn = x + dx;
-            if ((unsigned)zn < (unsigned)g.nz && (unsigned)yn < (unsigned)g.ny && (unsigned)xn < (unsigned)g.nx) {
+                for (int c = 0; c < C; ++c) nb[u][f][c] = base[c * cstride + off];
+            };
+            auto face_energy = [&](int u, int f, double w) {
+                double d2 = 0;
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
-                    const V2 nb = psi[line_index(g, c, zn, yn, t) + xn];
-                    kr[c] += wt[f] * ((double)nb.x - pr[c]);
-                    ki[c] += wt[f] * ((double)nb.y - pi[c]);
+                    const double dr = (double)own[u][c].x - (double)nb[u][f][c].x;
+                    const double di = (double)own[u][c].y - (double)nb[u][f][c].y;
+                    d2 += dr * dr;
+                    d2 += di * di;
                 }
-            } else {
+                ekin[u] += w * d2;
+            };
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const unsigned p = s + 64u * u + (threadIdx.x & 63);
+                const unsigned r = fast_div(p, g.f_pairs);
+                live[u] = p < end;
+                const unsigned rr = live[u] ? r : 0;  // a slot past the group reads the first row
+                x[u] = live[u] ? (int)(p - r * (unsigned)g.nx) : 0;
+                y[u] = rc.y0 + (int)rr;
+                at[u] = (int)rr * (int)g.ys + x[u];
+                ekin[u] = 0;
+#pragma unroll
+                for (int c = 0; c < C; ++c) own[u][c] = base[c * cstride + at[u]];
+            }
+#pragma unroll
+            for (int f = 0; f < FB; ++f) {
+                if (f >= nfwd) break;
+#pragma unroll
+                for (int u = 0; u < U; ++u) load(u, f, face[f]);
+            }
+            const const_ptr<double> wt = fresh(a.w + v * deg);
+#pragma unroll
+            for (int f = 0; f < FB; ++f) {
+                if (f >= nfwd) break;
+#pragma unroll
+                for (int u = 0; u < U; ++u) face_energy(u, f, wt[f]);
+            }
+            for (int f = FB; f < nfwd; ++f) {  // unknowns that own more faces (degree 6 and 8)
+                int2 e;
+                e.x = fx[f].x;
+                e.y = fx[f].y;
+#pragma unroll
+                for (int u = 0; u < U; ++u) load(u, 0, e);
+#pragma unroll
+                for (int u = 0; u < U; ++u) face_energy(u, 0, wt[f]);
+            }
+            const const_ptr<ObsConsts> k = fresh_args<ObsConsts>(offsetof(ObsArgs, k));
+            const const_ptr<double> pos = fresh(a.tb.pos64 + 3 * v);
+            const double dv = fresh(a.tb.dv + v)[0];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                double pr[C], pi[C], q[C], n = 0;
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
-                    kr[c] -= wt[f] * pr[c];
-                    ki[c] -= wt[f] * pi[c];
+                    pr[c] = own[u][c].x;
+                    pi[c] = own[u][c].y;
+                    q[c] = pr[c] * pr[c] + pi[c] * pi[c];
+                    n += q[c];
                 }
-            }
-        }
-        const Physics &ph = a.ph;
-        const double *pos = a.tb.pos64 + 3 * v;
-        const double sig = a.field.sigma, ik = 1.0 / (sig * sig);
-        const double rx = ph.p0[0] + sig * (ph.cell[0] * x + pos[0]);
-        const double ry = ph.p0[1] + sig * (ph.cell[1] * y + pos[1]);
-        const double rz = ph.p0[2] + sig * (ph.cell[2] * z + pos[2]);
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            kr[c] *= ik;
-            ki[c] *= ik;
-        }
-        double vtrap = 0;
-        if (a.field.t < ph.trap_off_time)
-            vtrap = 0.5 * (ph.trap2[0] * rx * rx + ph.trap2[1] * ry * ry + ph.trap2[2] * rz * rz) + ph.trap_offset;
-        double n = 0, ekin = 0;
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            n += pr[c] * pr[c] + pi[c] * pi[c];
-            ekin += pr[c] * kr[c] + pi[c] * ki[c];
-        }
-        double e = ekin + vtrap * n + 0.5 * ph.c0 * n * n;
-        double eh = ekin + vtrap * n + ph.c0 * n * n;
-        double Fx = 0, Fy = 0, Fz = 0;
-        if constexpr (C > 1) {
-            const double dxr = rx - ph.center[0], dyr = ry - ph.center[1], dzr = rz - ph.center[2];
-            const double Bx = a.field.bq * dxr + a.field.bb[0];
-            const double By = a.field.bq * dyr + a.field.bb[1];
-            const double Bz = -2 * a.field.bq * dzr + a.field.bb[2];
-            // F = psi^dag f psi through (e_x . f) psi etc. with the same ladder code
-            double tr[C], ti[C];
-            spin_dot<double, C>(1, 0, 0, pr, pi, tr, ti);
-            for (int c = 0; c < C; ++c) Fx += pr[c] * tr[c] + pi[c] * ti[c];
-            spin_dot<double, C>(0, 1, 0, pr, pi, tr, ti);
-            for (int c = 0; c < C; ++c) Fy += pr[c] * tr[c] + pi[c] * ti[c];
-            spin_dot<double, C>(0, 0, 1, pr, pi, tr, ti);
-            for (int c = 0; c < C; ++c) Fz += pr[c] * tr[c] + pi[c] * ti[c];
-            const double sgn = (C == 3) ? 1.0 : -1.0;
-            const double f2 = Fx * Fx + Fy * Fy + Fz * Fz;
-            const double bf = sgn * (Bx * Fx + By * Fy + Bz * Fz);
-            e += 0.5 * ph.c1 * f2 + bf;
-            eh += ph.c1 * f2 + bf;
-            if constexpr (C == 5) {
-                const double thr = 2 * (pr[0] * pr[4] - pi[0] * pi[4]) - 2 * (pr[1] * pr[3] - pi[1] * pi[3]) +
-                                   (pr[2] * pr[2] - pi[2] * pi[2]);
-                const double thi = 2 * (pr[0] * pi[4] + pi[0] * pr[4]) - 2 * (pr[1] * pi[3] + pi[1] * pr[3]) +
-                                   2 * pr[2] * pi[2];
-                const double th2 = thr * thr + thi * thi;
-                e += ph.c2 / 10.0 * th2;
-                eh += ph.c2 / 5.0 * th2;
-            }
-            if (a.quad) {
-                const double Qx = a.field.bqq * dxr + a.field.bbq[0];
-                const double Qy = a.field.bqq * dyr + a.field.bbq[1];
-                const double Qz = -2 * a.field.bqq * dzr + a.field.bbq[2];
-                spin_dot<double, C>(Qx, Qy, Qz, pr, pi, tr, ti);
-                double m2 = 0;
-                for (int c = 0; c < C; ++c) m2 += tr[c] * tr[c] + ti[c] * ti[c];
-                e += ph.quad_sign * m2;
-                eh += ph.quad_sign * m2;
-            }
-            constexpr int F = (C - 1) / 2;
-            double qz = 0;
-            for (int c = 0; c < C; ++c) qz += (double)((F - c) * (F - c)) * (pr[c] * pr[c] + pi[c] * pi[c]);
-            e += ph.q * qz;
-            eh += ph.q * qz;
-        }
-        const double dv = a.tb.dv[v];
-        acc[OBS_NORM] = n * dv;
-        acc[OBS_ENERGY] = e * dv;
-        acc[OBS_EXPECT_H] = eh * dv;
-        acc[OBS_MX] = Fx * dv;
-        acc[OBS_MY] = Fy * dv;
-        acc[OBS_MZ] = Fz * dv;
-        acc[OBS_MAXDENS] = n;
-        acc[OBS_NONFINITE] = (isfinite(n) && isfinite(e)) ? 0.0 : 1.0;
-        acc[OBS_SPIN] = sqrt(Fx * Fx + Fy * Fy + Fz * Fz) * dv;
-        acc[OBS_RX] = n * rx * dv;
-        acc[OBS_RY] = n * ry * dv;
-        acc[OBS_RZ] = n * rz * dv;
-        if constexpr (C > 1) {
-            // the reference's local spin (localAvgSpinAndDensity, Spin1GpeBCC.cu:235-271; Spin2GpeBCC.cu
-            // 214-262 applies the same spin-1 expressions to m = 1, 0, -1): x, y of the spinor divided
-            // by sqrt(n), z = |psi_1|^2 - |psi_-1|^2 undivided; its integrals weight it by n
-            // (integrateSpinAndDensity, Spin1GpeBCC.cu:992-1020).  Unknowns with n = 0 add nothing.
-            constexpr int o = C == 5 ? 1 : 0;
-            const double zr = (pr[o] * pr[o] + pi[o] * pi[o]) - (pr[o + 2] * pr[o + 2] + pi[o + 2] * pi[o + 2]);
-            double sx = 0, sy = 0;
-            if (n > 0) {
-                const double sq = sqrt(n);
-                double ur[3], ui[3];
-                for (int k = 0; k < 3; ++k) {
-                    ur[k] = pr[o + k] / sq;
-                    ui[k] = pi[o + k] / sq;
+                // faces of the box's boundary, whichever unknown would own them
+                for (int f = 0; f < nf; ++f) {
+                    const int pk = fx[f].x;
+                    if (inner && (pk & 3) == 1) continue;
+                    ekin[u] += (inside(u, pk) ? 0.0 : wt[f]) * n;
                 }
-                // sqrt2 (conj(u1) u0 + conj(u0) u-1)
-                sx = 1.4142135623730951 * ((ur[0] * ur[1] + ui[0] * ui[1]) + (ur[1] * ur[2] + ui[1] * ui[2]));
-                sy = 1.4142135623730951 * ((ur[0] * ui[1] - ui[0] * ur[1]) + (ur[1] * ui[2] - ui[1] * ur[2]));
+                const double rx = k->p0[0] + k->sig * pos[0] + k->cell[0] * x[u];
+                const double ry = k->p0[1] + k->sig * pos[1] + k->cell[1] * y[u];
+                const double rz = k->p0[2] + k->sig * pos[2] + k->cell[2] * z;
+                // e = part + half, <H> density = part + 2 half: interactions count twice
+                double trap = k->off + k->ht[0] * rx * rx;
+                trap += k->ht[1] * ry * ry;
+                trap += k->ht[2] * rz * rz;
+                double part = k->ik * ekin[u] + trap * n;
+                double half = k->hc0 * n * n;
+                if (!live[u]) continue;
+                if constexpr (C > 1) {
+                    const double dxr = rx - k->center[0], dyr = ry - k->center[1], dzr = rz - k->center[2];
+                    double Fx, Fy, Fz;
+                    spin_density<double, C>(pr, pi, Fx, Fy, Fz);
+                    const double fxy = Fx * Fx + Fy * Fy, f2 = fxy + Fz * Fz;
+                    part += (k->bq * dxr + k->bb[0]) * Fx;
+                    part += (k->bq * dyr + k->bb[1]) * Fy;
+                    part += (k->bb[2] - 2 * k->bq * dzr) * Fz;
+                    half += k->hc1 * f2;
+                    if constexpr (C == 5) {
+                        const double thr = 2 * (pr[0] * pr[4] - pi[0] * pi[4]) - 2 * (pr[1] * pr[3] - pi[1] * pi[3]) +
+                                           (pr[2] * pr[2] - pi[2] * pi[2]);
+                        const double thi = 2 * (pr[0] * pi[4] + pi[0] * pr[4]) - 2 * (pr[1] * pi[3] + pi[1] * pr[3]) +
+                                           2 * pr[2] * pi[2];
+                        half += k->c2_10 * (thr * thr + thi * thi);
+                    }
+                    if (a.quad) {
+                        const double Qx = k->bqq * dxr + k->bbq[0], Qy = k->bqq * dyr + k->bbq[1];
+                        const double Qz = -2 * k->bqq * dzr + k->bbq[2];
+                        double tr[C], ti[C], m2 = 0;
+                        spin_dot<double, C>(Qx, Qy, Qz, pr, pi, tr, ti);
+#pragma unroll
+                        for (int c = 0; c < C; ++c) m2 += tr[c] * tr[c] + ti[c] * ti[c];
+                        part += k->quad_sign * m2;
+                    }
+                    if constexpr (C == 3)
+                        part += k->q * (q[0] + q[2]);
+                    else
+                        part += k->q * (4 * (q[0] + q[4]) + (q[1] + q[3]));
+                    // the reference's local spin (localAvgSpinAndDensity, Spin1GpeBCC.cu:235-271;
+                    // Spin2GpeBCC.cu 214-262 applies the same spin-1 expressions to m = 1, 0, -1): x, y of
+                    // the spinor divided by sqrt(n), z = |psi_1|^2 - |psi_-1|^2 undivided; its integrals
+                    // weight it by n (integrateSpinAndDensity, Spin1GpeBCC.cu:992-1020).  n |(sx, sy, z)|
+                    // with sx, sy = (the undivided x, y) / n is |(x, y, n z)|: no division, and unknowns
+                    // with n = 0 add nothing.
+                    double sxy = fxy, zr = n * Fz;
+                    if constexpr (C == 5) {
+                        const double sx = (pr[1] * pr[2] + pi[1] * pi[2]) + (pr[2] * pr[3] + pi[2] * pi[3]);
+                        const double sy = (pr[1] * pi[2] - pi[1] * pr[2]) + (pr[2] * pi[3] - pi[2] * pr[3]);
+                        sxy = 2 * (sx * sx + sy * sy);
+                        zr = n * (q[1] - q[3]);
+                    }
+                    acc[OBS_MX] += Fx * dv;
+                    acc[OBS_MY] += Fy * dv;
+                    acc[OBS_MZ] += Fz * dv;
+                    acc[OBS_SPIN] += sqrt(f2) * dv;
+                    acc[OBS_REF_SPIN] += sqrt(sxy + zr * zr) * dv;
+                    acc[OBS_REF_MZ] += zr * dv;
+                }
+                const double nd = n * dv, e = part + half;
+                bad = bad || !isfinite(e);  // a non-finite n makes e non-finite
+                acc[OBS_NORM] += nd;
+                acc[OBS_ENERGY] += e * dv;
+                acc[OBS_EXPECT_H] += (e + half) * dv;
+                acc[OBS_MAXDENS] = fmax(acc[OBS_MAXDENS], n);
+                acc[OBS_RX] += nd * rx;
+                acc[OBS_RY] += nd * ry;
+                acc[OBS_RZ] += nd * rz;
             }
-            acc[OBS_REF_SPIN] = n * sqrt(sx * sx + sy * sy + zr * zr) * dv;
-            acc[OBS_REF_MZ] = n * zr * dv;
         }
     }
+    acc[OBS_NONFINITE] = bad ? 1.0 : 0.0;
     __shared__ double red[4][OBS_COUNT];
+    const double dens = wave_max(acc[OBS_MAXDENS]);
+    wave_sum_n<OBS_COUNT>(acc);
+    acc[OBS_MAXDENS] = dens;
+    if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-    for (int i = 0; i < OBS_COUNT; ++i) {
-        const double r = (i == OBS_MAXDENS) ? wave_max(acc[i]) : wave_sum(acc[i]);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][i] = r;
+        for (int i = 0; i < OBS_COUNT; ++i) red[threadIdx.x >> 6][i] = acc[i];
     }
     __syncthreads();
     if (threadIdx.x < OBS_COUNT) {
@@ -861,6 +944,26 @@ __global__ __launch_bounds__(256) void k_finalize_stage(const double *partials, 
         }
         if (threadIdx.x == 0) out[(long long)blockIdx.x * width + col] = red[0];
         __syncthreads();
+    }
+}
+
+// The reduction of at most RED_BLOCKS_MAX records in one workgroup, a wave a column: the fixed lane
+// stride and butterfly give the same bits for the same inputs.  The results go to `out` and, for
+// a host that reads them, straight to its pinned buffer (a copy of 112 bytes after the kernel cost
+// 8 us of a 20 us small-box call).
+__global__ __launch_bounds__(1024) void k_finalize_few(const double *partials, int n, int width, int maxcol,
+                                                       double *out, double *host)
+{
+    const int col = threadIdx.x >> 6;
+    if (col >= width) return;
+    const bool is_max = col == maxcol;
+    double acc = is_max ? -INFINITY : 0.0;
+#pragma unroll 8
+    for (int i = threadIdx.x & 63; i < n; i += 64) acc = fin_op(is_max, acc, partials[(long long)i * width + col]);
+    acc = is_max ? wave_max(acc) : wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) {
+        out[col] = acc;
+        if (host) host[col] = acc;
     }
 }
 
@@ -1318,33 +1421,36 @@ hipError_t launch_sweep(int fp64, int ncomp, int mode, const SweepArgs &a, hipSt
     return fp64 ? sweep_comp<double>(ncomp, mode, a, s) : sweep_comp<float>(ncomp, mode, a, s);
 }
 
-template <typename R, int C>
-static hipError_t obs_deg(const ObsArgs &a, hipStream_t s)
-{
-    dim3 grid(a.g.blocks), block(256);
-    switch (a.g.deg) {
-    case 4: hipLaunchKernelGGL((k_observables<R, C, 4>), grid, block, 0, s, a); break;
-    case 6: hipLaunchKernelGGL((k_observables<R, C, 6>), grid, block, 0, s, a); break;
-    case 8: hipLaunchKernelGGL((k_observables<R, C, 8>), grid, block, 0, s, a); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
+typedef void (*ObsKernel)(ObsArgs);
 
-template <typename R>
-static hipError_t obs_comp(int ncomp, const ObsArgs &a, hipStream_t s)
+static ObsKernel observables_kernel(int fp64, int ncomp)
 {
     switch (ncomp) {
-    case 1: return obs_deg<R, 1>(a, s);
-    case 3: return obs_deg<R, 3>(a, s);
-    case 5: return obs_deg<R, 5>(a, s);
-    default: return hipErrorInvalidValue;
+    case 1: return fp64 ? k_observables<double, 1, 2> : k_observables<float, 1, 2>;
+    case 3: return fp64 ? k_observables<double, 3, 1> : k_observables<float, 3, 1>;
+    case 5: return fp64 ? k_observables<double, 5, 1> : k_observables<float, 5, 1>;
+    default: return nullptr;
     }
+}
+
+hipError_t observables_resident(int fp64, int ncomp, int device, int *blocks)
+{
+    int per = 0, cus = 0;
+    const ObsKernel f = observables_kernel(fp64, ncomp);
+    if (!f) return hipErrorInvalidValue;
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void *)f, 256, 0);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+    const int n = per * cus;
+    *blocks = n < 1 ? 1 : (n > RED_BLOCKS_MAX ? RED_BLOCKS_MAX : n);
+    return e;
 }
 
 hipError_t launch_observables(int fp64, int ncomp, const ObsArgs &a, hipStream_t s)
 {
-    return fp64 ? obs_comp<double>(ncomp, a, s) : obs_comp<float>(ncomp, a, s);
+    const ObsKernel f = observables_kernel(fp64, ncomp);
+    if (!f) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(f, dim3(a.blocks), dim3(256), 0, s, a);
+    return hipGetLastError();
 }
 
 template <typename R>
@@ -1442,6 +1548,14 @@ hipError_t launch_finalize(const double *partials, int n, int width, int maxcol,
     hipLaunchKernelGGL(k_finalize_stage, dim3(nb), dim3(256), 0, s, partials, n, width, maxcol, chunk, scratch);
     hipLaunchKernelGGL(k_finalize_stage, dim3(1), dim3(256), 0, s, (const double *)scratch, nb, width, maxcol, nb,
                        out);
+    return hipGetLastError();
+}
+
+hipError_t launch_finalize_few(const double *partials, int n, int width, int maxcol, double *out, double *host,
+                               hipStream_t s)
+{
+    if (n <= 0 || n > RED_BLOCKS_MAX || width <= 0 || width > FIN_WIDTH_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_finalize_few, dim3(1), dim3(64 * FIN_WIDTH_MAX), 0, s, partials, n, width, maxcol, out, host);
     return hipGetLastError();
 }
 
