@@ -277,7 +277,9 @@ int gpe_traversal(const gpe_ctx *ctx, int *tile_rows, int *xcd_remap, int *x_per
  * plan's xcd_remap holds the flags); and the constants of the wave
  * decode's divisions by invariants (d, m, l: n / d = (t + n) >> l for n < 2^31, t the high
  * 32 bits of n m).  No counterpart in the reference, whose
- * launch shape is fixed (Spin1GpeBCC.cu:1376-1380). */
+ * launch shape is fixed (Spin1GpeBCC.cu:1376-1380).  With x_per_lane 1 the plan is the launch
+ * of one row per wave; the FP64 sweeps of lines that leave lanes idle that way walk the same
+ * tiles with the rows of a tile packed into whole waves. */
 typedef struct {
     int nx, ny, nz, V, C;
     int x_per_lane, rows, pairs, nseg, tile_rows, row_groups, ntile, xcd_remap;

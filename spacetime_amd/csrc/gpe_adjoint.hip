@@ -262,21 +262,21 @@ __device__ __forceinline__ void adj_sens32(const float *pr, const float *pi, con
 // One x value per lane (FP64, and FP32 where the pair form is not chosen): the forward sweep's
 // single body on mu_{k+1} -- interior fast path through the per-face line offsets, wave-uniform
 // weights on same-x faces, zero-weight pad faces skipped.
-template <typename R, int C, int DEG>
+template <typename R, int C, int DEG, bool ROWS>
 __device__ __forceinline__ void adjoint_single(const AdjArgs &a, int b, int nb, double *part)
 {
     using V2 = vec2_t<R>;
     const Geometry &g = a.g;
-    const WaveCoord wc = decode(g, b, nb);
-    if (!wc.valid) return;
-    const int x = wc.x, v = wc.v, y = wc.y, z = wc.z;
-    const bool act = x < g.nx;
-    const int xc = act ? x : g.nx - 1;
+    const LaneCoord lc = lane_coord<ROWS>(g, b, nb);
+    if (!lc.valid) return;
+    const int x = lc.x, v = lc.v, y = lc.y, z = lc.z;
+    const bool act = lc.act;
+    const int xc = lc.at;  // the lane's offset from the line of row y0
     const V2 *__restrict__ psi = (const V2 *)a.psi;
     const V2 *__restrict__ mu1 = (const V2 *)a.mu1;
     V2 *__restrict__ mu2 = (V2 *)a.mu2;
     const long long cstride = comp_stride(g);
-    const long long own_line = line_index(g, 0, z, y, v);
+    const long long own_line = line_index(g, 0, z, lc.y0, v);
 
     R pr[C], pi[C], mr[C], mi[C], qr[C], qi[C], ar[C], ai[C];
 #pragma unroll
@@ -306,36 +306,7 @@ __device__ __forceinline__ void adjoint_single(const AdjArgs &a, int b, int nb, 
     bool xok[DEG];
     int dxf[DEG], noff[DEG];
     const V2 *nbase[DEG];
-#pragma unroll
-    for (int f = 0; f < DEG; ++f) {
-        const int dx = (face[f] & 3) - 1;
-        const int xn = xc + dx;
-        xok[f] = (unsigned)xn < (unsigned)g.nx;
-        dxf[f] = dx;
-        noff[f] = xn < 0 ? 0 : (xn >= g.nx ? g.nx - 1 : xn);
-    }
-    if (z >= 1 && z <= g.nz - 2 && y >= 1 && y <= g.ny - 2) {
-        const V2 *own = mu1 + own_line;
-#pragma unroll
-        for (int f = 0; f < DEG; ++f) {
-            wu[f] = wt[f];
-            nbase[f] = own + fd[f];
-        }
-    } else {
-#pragma unroll
-        for (int f = 0; f < DEG; ++f) {
-            const int pk = face[f];
-            const int dy = ((pk >> 2) & 3) - 1, dz = ((pk >> 4) & 3) - 1, t = pk >> 8;
-            int zn = z + dz, yn = y + dy;
-            const bool inside = (unsigned)zn < (unsigned)g.nz && (unsigned)yn < (unsigned)g.ny;
-            if (!inside) {
-                zn = z;
-                yn = y;
-            }
-            wu[f] = inside ? wt[f] : (R)0;
-            nbase[f] = mu1 + line_index(g, 0, zn, yn, t);
-        }
-    }
+    face_lanes<R, DEG, ROWS>(g, lc, mu1 + own_line, face, fd, wt, wu, xok, dxf, nbase, noff);
     const int nf = DEG == 8 ? a.tb.nface[v] : DEG;
     V2 nbv[DEG][C];
 #pragma unroll
@@ -405,7 +376,7 @@ __device__ __forceinline__ void adjoint_pair(const AdjArgs &a, int b, int nb, do
     int x0, v, y0, z, r = 0;
     bool valid;
     if constexpr (ROWS) {
-        const RowCoord rc = decode_rows(g, b, nb);
+        const RowCoord rc = decode_rows<2>(g, b, nb);
         x0 = rc.x, v = rc.v, y0 = rc.y0, z = rc.z, r = rc.r, valid = rc.valid;
     } else {
         const WaveCoord wc = decode(g, b, nb);
@@ -617,8 +588,8 @@ __global__ __launch_bounds__(256) void k_adjoint(AdjArgs a)
     double part[ADJ_COUNT];
 #pragma unroll
     for (int i = 0; i < ADJ_COUNT; ++i) part[i] = 0.0;
-    if constexpr (X == 1)
-        adjoint_single<R, C, DEG>(a, b, gridDim.x, part);
+    if constexpr (X == 1 || X == 4)
+        adjoint_single<R, C, DEG, X == 4>(a, b, gridDim.x, part);
     else
         adjoint_pair<C, DEG, X == 3>(a, b, gridDim.x, part);
     __shared__ double red[4][ADJ_COUNT];
@@ -744,6 +715,12 @@ static hipError_t adj_form(const AdjArgs &a, hipStream_t s)
     if (form == 1) {
         hipLaunchKernelGGL((k_adjoint<R, C, DEG, 1>), grid, block, 0, s, a);
         return hipGetLastError();
+    }
+    if constexpr (std::is_same<R, double>::value) {
+        if (form == 4) {
+            hipLaunchKernelGGL((k_adjoint<R, C, DEG, 4>), grid, block, 0, s, a);
+            return hipGetLastError();
+        }
     }
     if constexpr (pair_lanes_ok(std::is_same<R, double>::value, DEG, C)) {
         if (form == 2) hipLaunchKernelGGL((k_adjoint<R, C, DEG, 2>), grid, block, 0, s, a);

@@ -146,16 +146,17 @@ __device__ __forceinline__ WaveCoord decode(const Geometry &g, int b, int nb)
 
 __device__ __forceinline__ WaveCoord decode(const Geometry &g) { return decode(g, blockIdx.x, gridDim.x); }
 
-// Lane coordinates of a traversal with row groups of g.rows y rows (x pairs on lines that one
-// row per wave would leave partly idle): the group's rows * pairs pair slots, row-major, fill
+// Lane coordinates of a traversal with row groups of g.rows y rows (lines that one row per wave
+// would leave partly idle): the group's rows * pairs slots (XPL x values each), row-major, fill
 // g.nseg waves; lane l of segment s takes slot p = 64 s + l, row r = p / pairs of the group
-// and the pair at x = 2 (p - r pairs).  Order: tile, z, row group, v, segment, as in decode().
+// and x = XPL (p - r pairs).  Order: tile, z, row group, v, segment, as in decode().
 // valid is wave-uniform; lanes with r >= rows or a row past ny are the caller's to mask.
 struct RowCoord {
     int x, v, y0, r, z;
     bool valid;
 };
 
+template <int XPL>
 __device__ __forceinline__ RowCoord decode_rows(const Geometry &g, int b, int nb)
 {
     RowCoord rc;
@@ -172,7 +173,7 @@ __device__ __forceinline__ RowCoord decode_rows(const Geometry &g, int b, int nb
     const unsigned p = (unsigned)(xseg * 64) + (threadIdx.x & 63);
     const unsigned r = fast_div(p, g.f_pairs);
     rc.r = (int)r;
-    rc.x = 2 * (int)(p - r * (unsigned)g.pairs);
+    rc.x = XPL * (int)(p - r * (unsigned)g.pairs);
     return rc;
 }
 
@@ -184,6 +185,104 @@ __device__ __forceinline__ long long line_index(const Geometry &g, int c, int z,
 
 // Elements between the same x of consecutive components of one line.
 __device__ __forceinline__ long long comp_stride(const Geometry &g) { return g.cs; }
+
+// Coordinates of a lane that owns one x (sweep_body_single, adjoint_single), with one y row per
+// wave (ROWS false: y = y0) or a row group.  A lane past the line, the group or the box has act =
+// false and stays in bounds (y, at).
+struct LaneCoord {
+    int x, v, y, z, y0;
+    int at;        // elements from the line of row y0 to the lane's value
+    int ylo, yhi;  // the rows of the wave's lanes
+    bool act, valid;
+};
+
+template <bool ROWS>
+__device__ __forceinline__ LaneCoord lane_coord(const Geometry &g, int b, int nb)
+{
+    LaneCoord lc;
+    if constexpr (ROWS) {
+        const RowCoord rc = decode_rows<1>(g, b, nb);
+        const int nrow = g.ny - rc.y0 < g.rows ? g.ny - rc.y0 : g.rows;  // the group's rows in the box
+        const int rr = rc.r < nrow ? rc.r : nrow - 1;
+        lc.x = rc.x, lc.v = rc.v, lc.z = rc.z, lc.y0 = rc.y0;
+        lc.act = rc.r < nrow;
+        lc.y = rc.y0 + rr;
+        lc.at = rr * (int)g.ys + rc.x;
+        // a lane's row grows with its lane number: lanes 0 and 63 bound the wave's rows; a wave
+        // whose first lane is past the group has nothing to do
+        lc.ylo = rc.y0 + __builtin_amdgcn_readfirstlane(rr);
+        lc.yhi = rc.y0 + __builtin_amdgcn_readlane(rr, 63);
+        lc.valid = rc.valid && __builtin_amdgcn_readfirstlane(rc.r) < nrow;
+    } else {
+        const WaveCoord wc = decode(g, b, nb);
+        lc.x = wc.x, lc.v = wc.v, lc.y = lc.y0 = lc.ylo = lc.yhi = wc.y, lc.z = wc.z, lc.valid = wc.valid;
+        lc.act = wc.x < g.nx;
+        lc.at = lc.act ? wc.x : g.nx - 1;
+    }
+    return lc;
+}
+
+// Addresses and weights of the faces of a lane's unknown: neighbour f at nbase[f][noff[f]] (plus
+// the component's stride) with weight wu[f], and xok[f] false where it is outside the box in x.
+// own: the line of row y0.
+template <typename R, int DEG, bool ROWS>
+__device__ __forceinline__ void face_lanes(const Geometry &g, const LaneCoord &lc, const vec2_t<R> *own,
+                                           const int *face, const int *fd, const R *wt, R *wu, bool *xok, int *dxf,
+                                           const vec2_t<R> **nbase, int *noff)
+{
+    const bool inner = lc.z >= 1 && lc.z <= g.nz - 2 && lc.ylo >= 1 && lc.yhi <= g.ny - 2;
+    if constexpr (ROWS) {
+#pragma unroll
+        for (int f = 0; f < DEG; ++f) {
+            const int dx = (face[f] & 3) - 1;
+            dxf[f] = dx;
+            xok[f] = (unsigned)(lc.x + dx) < (unsigned)g.nx;
+            // an x neighbour outside the box reads the lane's own x of that line
+            noff[f] = lc.at + (xok[f] ? dx : 0);
+        }
+        if (inner) {
+            // every y / z neighbour inside the box: own line plus the table's per-face offsets
+#pragma unroll
+            for (int f = 0; f < DEG; ++f) {
+                wu[f] = wt[f];
+                nbase[f] = own + fd[f];
+            }
+        } else {
+#pragma unroll
+            for (int f = 0; f < DEG; ++f) {
+                const int dy = ((face[f] >> 2) & 3) - 1, dz = ((face[f] >> 4) & 3) - 1;
+                const bool inside = (unsigned)(lc.z + dz) < (unsigned)g.nz && (unsigned)(lc.y + dy) < (unsigned)g.ny;
+                wu[f] = inside ? wt[f] : (R)0;
+                nbase[f] = own;
+                noff[f] += inside ? fd[f] : 0;  // outside: the lane's own line
+            }
+        }
+    } else {
+#pragma unroll
+        for (int f = 0; f < DEG; ++f) {
+            const int dx = (face[f] & 3) - 1;
+            const int xn = lc.at + dx;
+            xok[f] = (unsigned)xn < (unsigned)g.nx;
+            dxf[f] = dx;
+            noff[f] = xn < 0 ? 0 : (xn >= g.nx ? g.nx - 1 : xn);
+        }
+        if (inner) {
+#pragma unroll
+            for (int f = 0; f < DEG; ++f) {
+                wu[f] = wt[f];
+                nbase[f] = own + fd[f];
+            }
+        } else {
+#pragma unroll
+            for (int f = 0; f < DEG; ++f) {
+                const int dy = ((face[f] >> 2) & 3) - 1, dz = ((face[f] >> 4) & 3) - 1;
+                const bool inside = (unsigned)(lc.z + dz) < (unsigned)g.nz && (unsigned)(lc.y + dy) < (unsigned)g.ny;
+                wu[f] = inside ? wt[f] : (R)0;
+                nbase[f] = inside ? own + fd[f] : own;
+            }
+        }
+    }
+}
 
 // ------------------------------------------------------------------ local Hamiltonian --
 

@@ -41,11 +41,12 @@ struct Geometry {
     int nx, ny, nz, V, deg;
     int C;             // complex components (1, 3, 5)
     FastDiv f_nseg, f_V, f_ty, f_nz;  // the decode's divisors (f_ty divides by tyr)
-    FastDiv f_pairs;   // divides a lane's pair slot by `pairs` (rows > 1)
+    FastDiv f_pairs;   // divides a lane's slot by `pairs` (rows > 1)
     int xpl;           // consecutive x values per lane (1, or 2 for the FP32 sweep)
     int rows;          // y rows of a row group (1; 2-8, or the tile's rows in the slab layout
-                       // when they start on 128-byte boundaries: x pairs spread over the rows)
-    int pairs;         // x pairs per row: ceil(nx / 2)
+                       // when they start on 128-byte boundaries: x pairs spread over the rows;
+                       // FP64: the tile's rows where one row a wave would idle lanes)
+    int pairs;         // lane slots per row of a row group: x pairs, ceil(nx / 2), or nx for xpl = 1
     int nseg;          // waves per x-line (rows == 1: ceil(nx / (64 xpl))) or per row group
                        // (rows > 1: ceil(rows * pairs / 64))
     int ty;            // y rows per tile of the traversal order
@@ -69,8 +70,12 @@ __host__ __device__ constexpr bool pair_lanes_ok(int fp64, int deg, int ncomp)
     return !fp64 && deg >= 1 && ncomp >= 1;
 }
 
-// Sweep body of a traversal: 1 one x per lane, 2 x pairs, 3 x pairs over a group of 2-8 y rows.
-__host__ __device__ constexpr int lane_form(int xpl, int rows) { return xpl == 1 ? 1 : (rows > 1 ? 3 : 2); }
+// Sweep body of a traversal: 1 one x per lane, 2 x pairs, 3 x pairs over a group of y rows, 4 one
+// x per lane over a group of y rows (FP64).
+__host__ __device__ constexpr int lane_form(int xpl, int rows)
+{
+    return xpl == 1 ? (rows > 1 ? 4 : 1) : (rows > 1 ? 3 : 2);
+}
 
 // Default: pairs in FP32.  Measured on spin-1 / spin-2 BCC, FCC and Cube boxes of 96-192 blocks,
 // pairs run 30-40% faster than single values, also at degree 8 with 5 components where they cut

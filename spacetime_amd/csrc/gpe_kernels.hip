@@ -77,23 +77,25 @@ __device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const 
 }
 
 // One x value per lane (FP64, and FP32 where the neighbour pairs would not fit).
-template <typename R, int C, int DEG, int MODE>
+// ROWS: the wave's lanes lie in a group of g.rows consecutive y rows of one (z, v), as in
+// sweep_body_pair: y0 is the group's first row and a lane's offsets are from its line.
+template <typename R, int C, int DEG, int MODE, bool ROWS>
 __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, int sweep, int b, int nb)
 {
     using V2 = vec2_t<R>;
     const Geometry &g = a.g;
-    const WaveCoord wc = decode(g, b, nb);
+    const LaneCoord lc = lane_coord<ROWS>(g, b, nb);
     double part = 0.0;
 
-    if (wc.valid) {
-        const int x = wc.x, v = wc.v, y = wc.y, z = wc.z;
-        const bool act = x < g.nx;
-        const int xc = act ? x : g.nx - 1;
+    if (lc.valid) {
+        const int x = lc.x, v = lc.v, y = lc.y, z = lc.z;
+        const bool act = lc.act;
+        const int xc = lc.at;  // the lane's offset from the line of row y0 (its own x, clamped into the box)
         const V2 *__restrict__ cur = (const V2 *)a.cur;
         V2 *__restrict__ nxt = (V2 *)a.next;
         const V2 *__restrict__ prv = (const V2 *)(a.prev ? a.prev : a.next);
         const long long cstride = comp_stride(g);  // elements between components of a line
-        const long long own_line = line_index(g, 0, z, y, v);
+        const long long own_line = line_index(g, 0, z, lc.y0, v);
 
         // issue every load of the wave before any use: own values, psi_{k-1}, and the
         // DEG neighbour lines (wave-uniform line bases, per-lane 32-bit offsets)
@@ -123,42 +125,12 @@ __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, int sweep,
             fd[f] = e.y;
         }
         const R *wt = table_w<R>(a.tb) + v * DEG;
-        R wu[DEG];    // wave-uniform weight: 0 when the neighbour's y or z is outside the box
+        R wu[DEG];    // weight: 0 when the neighbour's y or z is outside the box (wave-uniform unless ROWS)
         bool xok[DEG];
         int dxf[DEG];
         const V2 *nbase[DEG];
         int noff[DEG];
-#pragma unroll
-        for (int f = 0; f < DEG; ++f) {
-            const int dx = (face[f] & 3) - 1;
-            const int xn = xc + dx;
-            xok[f] = (unsigned)xn < (unsigned)g.nx;
-            dxf[f] = dx;
-            noff[f] = xn < 0 ? 0 : (xn >= g.nx ? g.nx - 1 : xn);
-        }
-        if (z >= 1 && z <= g.nz - 2 && y >= 1 && y <= g.ny - 2) {
-            // every y / z neighbour inside the box: own line plus the table's per-face offsets
-            const V2 *own = cur + own_line;
-#pragma unroll
-            for (int f = 0; f < DEG; ++f) {
-                wu[f] = wt[f];
-                nbase[f] = own + fd[f];
-            }
-        } else {
-#pragma unroll
-            for (int f = 0; f < DEG; ++f) {
-                const int pk = face[f];
-                const int dy = ((pk >> 2) & 3) - 1, dz = ((pk >> 4) & 3) - 1, t = pk >> 8;
-                int zn = z + dz, yn = y + dy;
-                const bool inside = (unsigned)zn < (unsigned)g.nz && (unsigned)yn < (unsigned)g.ny;
-                if (!inside) {
-                    zn = z;
-                    yn = y;
-                }
-                wu[f] = inside ? wt[f] : (R)0;
-                nbase[f] = cur + line_index(g, 0, zn, yn, t);
-            }
-        }
+        face_lanes<R, DEG, ROWS>(g, lc, cur + own_line, face, fd, wt, wu, xok, dxf, nbase, noff);
         // degree-8 tables pad some unknowns with zero-weight faces: skip their loads
         const int nf = DEG == 8 ? a.tb.nface[v] : DEG;
         V2 nb[DEG][C];
@@ -275,7 +247,7 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
     int x0, v, y0, z, r = 0;
     bool valid;
     if constexpr (ROWS) {
-        const RowCoord rc = decode_rows(g, b, nb);
+        const RowCoord rc = decode_rows<2>(g, b, nb);
         x0 = rc.x, v = rc.v, y0 = rc.y0, z = rc.z, r = rc.r, valid = rc.valid;
     } else {
         const WaveCoord wc = decode(g, b, nb);
@@ -533,7 +505,7 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
     }
 }
 
-// X: the lane form (lane_form): 1 one x per lane, 2 x pairs, 3 x pairs over a group of 2-8 y rows.
+// X: the lane form (lane_form).
 template <typename R, int C, int DEG, int MODE, int X>
 __device__ __forceinline__ void sweep_body(const SweepArgs &a, int sweep, int b, int nb)
 {
@@ -542,7 +514,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &a, int sweep, int b,
     else if constexpr (X == 2)
         sweep_body_pair<C, DEG, MODE, false>(a, sweep, b, nb);
     else
-        sweep_body_single<R, C, DEG, MODE>(a, sweep, b, nb);
+        sweep_body_single<R, C, DEG, MODE, X == 4>(a, sweep, b, nb);
 }
 
 template <typename R, int C, int DEG, int MODE, int X>
@@ -1387,6 +1359,9 @@ static hipError_t sweep_mode(int mode, const SweepArgs &a, hipStream_t s)
 {
     const int form = lane_form(a.g.xpl, a.g.rows);
     if (form == 1) return sweep_mode_x<R, C, DEG, 1>(mode, a, s);
+    if constexpr (std::is_same<R, double>::value) {
+        if (form == 4) return sweep_mode_x<R, C, DEG, 4>(mode, a, s);
+    }
     if constexpr (pair_lanes_ok(std::is_same<R, double>::value, DEG, C)) {
         if (form == 2) return sweep_mode_x<R, C, DEG, 2>(mode, a, s);
         if (form == 3) return sweep_mode_x<R, C, DEG, 3>(mode, a, s);
@@ -1478,6 +1453,12 @@ static hipError_t ens_x(int form, const EnsembleArgs &e, int blocks, hipStream_t
     if (form == 1) {
         hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, 1>), grid, block, 0, s, e);
         return hipGetLastError();
+    }
+    if constexpr (std::is_same<R, double>::value) {
+        if (form == 4) {
+            hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, 4>), grid, block, 0, s, e);
+            return hipGetLastError();
+        }
     }
     if constexpr (pair_lanes_ok(std::is_same<R, double>::value, DEG, C)) {
         if (form == 2) {
