@@ -284,6 +284,23 @@ __device__ __forceinline__ void face_lanes(const Geometry &g, const LaneCoord &l
     }
 }
 
+// Exchange between the waves of a workgroup that hold a ring of four unknowns of the same cells
+// (Geometry::exchange): every wave writes its own values to LDS, and two of its four neighbours
+// are read from there.  A sweep's face loads cost more than their bytes from HBM: without them the
+// sweeps run 3-25% faster, and most of that is same-cell faces, whose lines other waves are
+// fetching at the same time.  us a sweep, without -> with the exchange: spin-1 BCC 128^3 FP32 304 ->
+// 282, FP64 96^3 291 -> 249, its imaginary time 254 -> 215; spin-2 128^3 506 -> 471; spin-1 64^3
+// 38.1 -> 35.3, 16^3 4.4 -> 3.9.  One component loses (98 -> 123: too little work per wave for the
+// barrier) but gains 5% from the numbering alone.  Whole cells in one workgroup (12 waves) lost
+// 10% (fewer workgroups fit a CU); pairs and paths of four in A15, C15 and Z, which have no such
+// rings, gained nothing.
+// The barrier waits for LDS only (a __syncthreads would also wait for the loads in flight).  Every
+// wave of the workgroup has to arrive.
+__device__ __forceinline__ void exchange_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// The wave that holds the neighbour across exchanged face f (0, 1).
+__device__ __forceinline__ unsigned exchange_wave(int f) { return (threadIdx.x >> 6) ^ (f == 0 ? 1u : 3u); }
+
 // ------------------------------------------------------------------ local Hamiltonian --
 
 // (W . f) psi for spin-1 (m = +1, 0, -1): Spin1GpeBCC.cu:890-895 expanded form.

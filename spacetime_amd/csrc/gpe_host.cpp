@@ -78,7 +78,7 @@ struct gpe_ctx {
     int device = 0;
     void *level[2] = {nullptr, nullptr};
     // tables
-    int *d_face = nullptr, *d_nface = nullptr, *d_facex = nullptr;
+    int *d_abi = nullptr, *d_nface = nullptr, *d_facex = nullptr;  // d_abi: V places, then their inverse
     int *d_oface = nullptr, *d_nfwd = nullptr;  // the observables' faces (ObsArgs)
     double *d_ow = nullptr;
     float *d_w32 = nullptr, *d_wsum32 = nullptr, *d_pos32 = nullptr;
@@ -196,7 +196,8 @@ bool quad_active(const gpe_ctx *c)
 Tables tables(const gpe_ctx *c)
 {
     Tables t;
-    t.face = c->d_face;
+    t.abi = c->d_abi;
+    t.place = c->d_abi + c->g.V;
     t.w32 = c->d_w32;
     t.w64 = c->d_w64;
     t.wsum32 = c->d_wsum32;
@@ -304,6 +305,7 @@ bool finish_geometry(Geometry &g, bool pack = false)
     g.nseg = rows > 1 ? (rows * g.pairs + 63) / 64 : (g.nx + 64 * g.xpl - 1) / (64 * g.xpl);
     g.ntile = (g.ny + g.ty - 1) / g.ty;
     g.waves = (long long)g.ntile * g.tyr * g.nz * g.V * g.nseg;
+    g.exchange = g.rings && exchange_ok(g.deg, g.C) && (g.nseg == 1 || g.v_inner);
     const long long blocks = (g.waves + 3) / 4;
     if (blocks >= (1ll << 29)) return false;  // wave indices below 2^31 (the decode's divisions)
     g.blocks = (int)blocks;
@@ -361,6 +363,7 @@ Geometry base_geometry(const gpe_config &cfg)
     g.nz = cfg.nz;
     g.V = kLattices[cfg.lattice].V;
     g.deg = kLattices[cfg.lattice].deg;
+    g.rings = kLattices[cfg.lattice].rings;
     g.C = cfg.ncomp;
     g.xpl = 1;
     g.ty = cfg.ny < 8 ? cfg.ny : 8;
@@ -391,6 +394,7 @@ Geometry base_geometry(const gpe_config &cfg)
         g.zs = g.ys * cfg.ny;
     }
     g.xcd_remap = 1;
+    g.v_inner = g.rings && exchange_ok(g.deg, g.C);  // rings of four in a workgroup
     return g;
 }
 
@@ -481,6 +485,7 @@ int ctx_view(gpe_ctx *c, CtxView *out)
 {
     if (!c || !out) return GPE_EINVAL;
     out->g = c->g;
+    out->tb = tables(c);
     out->fp64 = c->fp64;
     out->ncomp = c->cfg.ncomp;
     out->device = c->device;
@@ -583,23 +588,40 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     std::vector<float> w32(V * deg), wsum32(V), pos32(3 * V);
     std::vector<int> nface(V), facex(2 * V * deg), oface(2 * V * deg), nfwd(V);
     std::vector<double> ow(V * deg);
+    // place p of a cell on the device holds the table's unknown order[p]
+    const int *order = c->lat->order;
+    std::vector<int> place(V);
+    for (int p = 0; p < V; ++p) place[order[p]] = p;
     for (int v = 0; v < V; ++v) {
+        const int src = order[v] * deg;
+        int nf = deg;  // pad faces (zero Hodge weight) trail the real ones
+        while (nf > 0 && c->lat->hodge[src + nf - 1] == 0.0) --nf;
+        nface[v] = nf;
+        // rings: the faces to places v ^ 1 and v ^ 3 of the same cell lead, the others follow in the
+        // table's order
+        std::vector<int> row;
+        for (int k = 0; k < (c->lat->rings ? 2 : 0); ++k)
+            for (int f = 0; f < nf; ++f) {
+                const int pk = c->lat->face[src + f];
+                if ((pk & 63) == 21 && place[pk >> 8] == (v ^ (k ? 3 : 1))) {
+                    row.push_back(f);
+                    break;
+                }
+            }
+        for (int f = 0; f < deg; ++f)
+            if (std::find(row.begin(), row.end(), f) == row.end()) row.push_back(f);
         for (int f = 0; f < deg; ++f) {
-            const int pk = c->lat->face[v * deg + f];
+            const int tab = c->lat->face[src + row[f]];
+            const int pk = (tab & 63) | (place[tab >> 8] << 8);
             const long long dy = ((pk >> 2) & 3) - 1, dz = ((pk >> 4) & 3) - 1, t = pk >> 8;
             facex[2 * (v * deg + f)] = pk;
             // |offset| < 3 zs, checked against the int range at creation
             facex[2 * (v * deg + f) + 1] = (int)(dz * g.zs + dy * g.ys + (t - v) * g.vs);
-        }
-        int nf = deg;  // pad faces (zero Hodge weight) trail the real ones
-        while (nf > 0 && c->lat->hodge[v * deg + nf - 1] == 0.0) --nf;
-        nface[v] = nf;
-        for (int f = 0; f < deg; ++f) {
-            const double w = -0.5 * c->lat->hodge[v * deg + f] / (s * s);
+            const double w = -0.5 * c->lat->hodge[src + row[f]] / (s * s);
             w64[v * deg + f] = w;
             w32[v * deg + f] = (float)w;
-            wsum64[v] += w;
         }
+        for (int f = 0; f < deg; ++f) wsum64[v] += -0.5 * c->lat->hodge[src + f] / (s * s);
         wsum32[v] = (float)wsum64[v];
         // the observables' order: faces to a higher address (offset between the two unknowns, dx
         // included), the others, then the pad faces
@@ -616,10 +638,10 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
             if (pass == 0) nfwd[v] = o - v * deg;
         }
         for (int k = 0; k < 3; ++k) {
-            pos64[3 * v + k] = s * c->lat->pos[3 * v + k];
+            pos64[3 * v + k] = s * c->lat->pos[3 * order[v] + k];
             pos32[3 * v + k] = (float)pos64[3 * v + k];
         }
-        dv[v] = s * s * s * c->lat->vol[v];
+        dv[v] = s * s * s * c->lat->vol[order[v]];
     }
     auto up = [&](void **dst, const void *src, size_t bytes) {
         if (rc) return;
@@ -631,7 +653,9 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
         ee = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
         if (ee != hipSuccess) rc = hip_fail(c, ee, "hipMemcpy tables");
     };
-    up((void **)&c->d_face, c->lat->face, sizeof(int) * V * deg);
+    std::vector<int> abi(order, order + V);
+    abi.insert(abi.end(), place.begin(), place.end());
+    up((void **)&c->d_abi, abi.data(), sizeof(int) * 2 * V);
     up((void **)&c->d_nface, nface.data(), sizeof(int) * V);
     up((void **)&c->d_facex, facex.data(), sizeof(int) * 2 * V * deg);
     up((void **)&c->d_oface, oface.data(), sizeof(int) * 2 * V * deg);
@@ -667,7 +691,7 @@ int gpe_destroy(gpe_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (int l = 0; l < 2; ++l)
         if (c->level[l]) (void)hipFree(c->level[l]);
-    void *ptrs[] = {c->d_face, c->d_nface, c->d_facex, c->d_oface, c->d_ow, c->d_nfwd, c->d_w32, c->d_w64, c->d_wsum32, c->d_wsum64, c->d_pos32,
+    void *ptrs[] = {c->d_abi, c->d_nface, c->d_facex, c->d_oface, c->d_ow, c->d_nfwd, c->d_w32, c->d_w64, c->d_wsum32, c->d_wsum64, c->d_pos32,
                     c->d_pos64, c->d_dv, c->d_fields, c->d_partials, c->d_scalars, c->d_red};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -695,7 +719,7 @@ static int set_state_impl(gpe_ctx *c, int level, const double *psi, double t, hi
         HIPCALL(c, hipMemcpyAsync(staging, psi, nbytes, hipMemcpyHostToDevice, c->stream));
         src = staging;
     }
-    hipError_t e = launch_pack(c->fp64, g, c->cfg.ncomp, src, c->level[level], c->stream);
+    hipError_t e = launch_pack(c->fp64, g, tables(c), c->cfg.ncomp, src, c->level[level], c->stream);
     if (staging) (void)hipFreeAsync(staging, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "pack");
     HIPCALL(c, hipStreamSynchronize(c->stream));
@@ -733,7 +757,7 @@ static int get_state_impl(gpe_ctx *c, int level, double *psi, bool host)
         HIPCALL(c, hipMallocAsync((void **)&staging, nbytes, c->stream));
         dst = staging;
     }
-    hipError_t e = launch_unpack(c->fp64, g, c->cfg.ncomp, c->level[level], dst, c->stream);
+    hipError_t e = launch_unpack(c->fp64, g, tables(c), c->cfg.ncomp, c->level[level], dst, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "unpack");
     if (host) {
         HIPCALL(c, hipMemcpyAsync(psi, staging, nbytes, hipMemcpyDeviceToHost, c->stream));
@@ -1056,7 +1080,7 @@ int gpe_local_fields(gpe_ctx *c, int level, int kind, double *out)
     const size_t bytes = sizeof(double) * (size_t)width * (size_t)c->cfg.nx * c->cfg.ny * c->cfg.nz * c->g.V;
     double *d = nullptr;
     if (hipMalloc((void **)&d, bytes) != hipSuccess) return fail(c, GPE_ENOMEM, "field map does not fit");
-    hipError_t e = launch_local_fields(c->fp64, c->cfg.ncomp, c->g, c->level[level], kind, d, c->stream);
+    hipError_t e = launch_local_fields(c->fp64, c->cfg.ncomp, c->g, tables(c), c->level[level], kind, d, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out, d, bytes, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     (void)hipFree(d);
@@ -1166,7 +1190,7 @@ int gpe_add_noise(gpe_ctx *c, int level, double amplitude, unsigned long long se
     int rc = check_level(c, level);
     if (rc) return rc;
     if (!(amplitude >= 0.0)) return fail(c, GPE_EINVAL, "negative noise amplitude");
-    hipError_t e = launch_noise(c->fp64, c->cfg.ncomp, c->g, c->level[level], amplitude, seed, c->stream);
+    hipError_t e = launch_noise(c->fp64, c->cfg.ncomp, c->g, tables(c), c->level[level], amplitude, seed, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     return e == hipSuccess ? GPE_OK : hip_fail(c, e, "noise");
 }
@@ -1381,7 +1405,7 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
         ADJ_CHECK(hipMalloc((void **)&staging, abi), "staging");
         bufs.push_back(staging);
         ADJ_CHECK(hipMemcpyAsync(staging, spec->target, abi, hipMemcpyHostToDevice, c->stream), "target");
-        ADJ_CHECK(launch_pack(c->fp64, g, c->cfg.ncomp, staging, target, c->stream), "pack target");
+        ADJ_CHECK(launch_pack(c->fp64, g, tables(c), c->cfg.ncomp, staging, target, c->stream), "pack target");
         oa.mode = OBJ_PARTIALS;
         ADJ_CHECK(launch_objective(c->fp64, c->cfg.ncomp, oa, c->stream), "overlap");
         ADJ_CHECK(launch_finalize(d_part, g.blocks, 2, -1, c->d_scalars + 32, c->d_red, c->stream), "overlap sum");
@@ -1540,6 +1564,7 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
 // Members sharing (face degree, x per lane) form a group launched by one specialised kernel.
 struct EnsembleGroup {
     int deg, form;      // face degree and lane_form of every member
+    int exchange;       // their Geometry::exchange
     int first, count;   // members [first, first + count) of the sorted member list
     int blocks;         // workgroups of the group's launch
 };
@@ -1584,8 +1609,10 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
     if (!e) return GPE_ENOMEM;
     e->m.assign(members, members + n);
     std::stable_sort(e->m.begin(), e->m.end(), [](const gpe_ctx *a, const gpe_ctx *b) {
-        return a->gs.deg != b->gs.deg ? a->gs.deg < b->gs.deg
-                                      : lane_form(a->gs.xpl, a->gs.rows) < lane_form(b->gs.xpl, b->gs.rows);
+        const auto key = [](const Geometry &g) {
+            return std::make_tuple(g.deg, lane_form(g.xpl, g.rows), g.exchange);
+        };
+        return key(a->gs) < key(b->gs);
     });
     e->ncomp = c0->cfg.ncomp;
     e->fp64 = c0->fp64;
@@ -1598,8 +1625,9 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
         const int form = lane_form(c->gs.xpl, c->gs.rows);
         const bool solo = c->gs.blocks >= ENS_SOLO_BLOCKS;
         if (i == 0 || solo || prev_solo || c->gs.deg != e->groups.back().deg || form != e->groups.back().form ||
+            c->gs.exchange != e->groups.back().exchange ||
             e->groups.back().count == ENS_GROUP_MAX) {
-            e->groups.push_back(EnsembleGroup{c->gs.deg, form, i, 0, 0});
+            e->groups.push_back(EnsembleGroup{c->gs.deg, form, c->gs.exchange, i, 0, 0});
             begin = 0;
         }
         prev_solo = solo;
@@ -1680,7 +1708,7 @@ int gpe_ensemble_step(gpe_ensemble *e, int nsteps, int graph_sweeps)
         a.sweep = k;
         a.sweep_base = base;
         for (int i = 0; i < gr.count; ++i) a.begin[i] = e->h[gr.first + i].begin;
-        return launch_ensemble_sweep(e->fp64, e->ncomp, gr.deg, gr.form, a, gr.blocks, st);
+        return launch_ensemble_sweep(e->fp64, e->ncomp, gr.deg, gr.form, gr.exchange, a, gr.blocks, st);
     };
     auto launch_all = [&](int k, const int *base) -> hipError_t {
         for (const EnsembleGroup &gr : e->groups) {

@@ -60,6 +60,8 @@ struct Geometry {
     int blocks;        // workgroups of a sweep (4 waves each)
     int xcd_remap;     // give each XCD a contiguous range of the traversal order
     int v_inner;       // 1: the unknown v varies faster than the x segment (lines of several waves)
+    int rings;         // the lattice's device numbering is rings of four (LatticeTable)
+    int exchange;      // 1: the sweep's waves exchange two neighbours of every unknown (exchange_ok)
 };
 
 // x values per lane of the sweep kernel.  Two (one 16-byte load per component and neighbour,
@@ -86,9 +88,14 @@ __host__ __device__ constexpr int default_xpl(int fp64, int deg, int ncomp, int 
     return (pair_lanes_ok(fp64, deg, ncomp) && nx >= 1) ? 2 : 1;
 }
 
+// Sweep bodies that exchange same-cell neighbours between the waves of a workgroup (lattices whose
+// device numbering is rings of four, traversals with the unknown fastest).
+__host__ __device__ constexpr bool exchange_ok(int deg, int ncomp) { return deg == 4 && ncomp > 1; }
+
 // Per-context constant tables on the device (weights already scaled by -1/2 / s^2).
 struct Tables {
-    const int *face;       // V*deg packed faces
+    const int *abi;        // V: the ABI's unknown at each place of the device's numbering of a cell
+    const int *place;      // V: its inverse
     const float *w32;      // V*deg
     const double *w64;     // V*deg
     const float *wsum32;   // V: sum of the weights of unknown v
@@ -152,8 +159,8 @@ enum {
     OBS_SPIN, OBS_RX, OBS_RY, OBS_RZ, OBS_REF_SPIN, OBS_REF_MZ, OBS_COUNT
 };
 enum { FIELD_DENSITY = 0, FIELD_SPIN = 1, FIELD_SPIN_NORM = 2, FIELD_UV_THETA = 3 };
-hipError_t launch_local_fields(int fp64, int ncomp, const Geometry &g, const void *psi, int kind, double *out,
-                               hipStream_t s);
+hipError_t launch_local_fields(int fp64, int ncomp, const Geometry &g, const Tables &tb, const void *psi, int kind,
+                               double *out, hipStream_t s);
 
 // Constants of the observables, combined on the host.
 struct ObsConsts {
@@ -258,10 +265,10 @@ struct EnsembleArgs {
     int begin[ENS_GROUP_MAX]; // members[i].begin
 };
 
-// All members of one launch share the component count, precision, face degree and lanes.
+// All members of one launch share the component count, precision, face degree, lanes and exchange.
 // form: lane_form of the group's traversal
-hipError_t launch_ensemble_sweep(int fp64, int ncomp, int deg, int form, const EnsembleArgs &e, int blocks,
-                                 hipStream_t s);
+hipError_t launch_ensemble_sweep(int fp64, int ncomp, int deg, int form, int exchange, const EnsembleArgs &e,
+                                 int blocks, hipStream_t s);
 hipError_t launch_advance_base(int *base, int by, hipStream_t s);
 hipError_t launch_set_base(int *base, int value, hipStream_t s);
 
@@ -303,14 +310,17 @@ hipError_t launch_norm_to_scale(const double *in, double target, double *out, hi
 hipError_t launch_scale(int fp64, void *psi, long long nelem, double factor, const double *dfactor,
                         hipStream_t s);
 // ABI complex128 [c][z][y][x][v] <-> device layout
-hipError_t launch_pack(int fp64, const Geometry &g, int ncomp, const double *abi, void *dev, hipStream_t s);
-hipError_t launch_unpack(int fp64, const Geometry &g, int ncomp, const void *dev, double *abi, hipStream_t s);
+hipError_t launch_pack(int fp64, const Geometry &g, const Tables &tb, int ncomp, const double *abi, void *dev,
+                       hipStream_t s);
+hipError_t launch_unpack(int fp64, const Geometry &g, const Tables &tb, int ncomp, const void *dev, double *abi,
+                         hipStream_t s);
 // dst = phase * src (complex), for the staggered start
 hipError_t launch_phase_copy(int fp64, const void *src, void *dst, long long nelem, double pre, double pim,
                              hipStream_t s);
 // What other source files of the library see of a context (gpe_host.cpp owns the struct).
 struct CtxView {
     Geometry g;          // one x per lane: the layout of a level
+    Tables tb;
     int fp64, ncomp, device;
     hipStream_t stream;
     void *level[2];
@@ -320,7 +330,7 @@ int ctx_fail(gpe_ctx *c, int code, const char *what);
 
 // spinor phase projection (GPE_PHASE_*) and spinor noise of a level, in place
 hipError_t launch_project(int fp64, int ncomp, const Geometry &g, void *psi, int phase, double param, hipStream_t s);
-hipError_t launch_noise(int fp64, int ncomp, const Geometry &g, void *psi, double amp, unsigned long long seed,
+hipError_t launch_noise(int fp64, int ncomp, const Geometry &g, const Tables &tb, void *psi, double amp, unsigned long long seed,
                         hipStream_t s);
 
 }  // namespace gpe

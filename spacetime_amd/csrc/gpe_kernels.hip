@@ -79,7 +79,7 @@ __device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const 
 // One x value per lane (FP64, and FP32 where the neighbour pairs would not fit).
 // ROWS: the wave's lanes lie in a group of g.rows consecutive y rows of one (z, v), as in
 // sweep_body_pair: y0 is the group's first row and a lane's offsets are from its line.
-template <typename R, int C, int DEG, int MODE, bool ROWS>
+template <typename R, int C, int DEG, int MODE, bool ROWS, int NIN>
 __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, int sweep, int b, int nb)
 {
     using V2 = vec2_t<R>;
@@ -133,27 +133,46 @@ __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, int sweep,
         face_lanes<R, DEG, ROWS>(g, lc, cur + own_line, face, fd, wt, wu, xok, dxf, nbase, noff);
         // degree-8 tables pad some unknowns with zero-weight faces: skip their loads
         const int nf = DEG == 8 ? a.tb.nface[v] : DEG;
-        V2 nb[DEG][C];
+        V2 nb[DEG - NIN][C];
 #pragma unroll
-        for (int f = 0; f < DEG; ++f)
+        for (int f = NIN; f < DEG; ++f)
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 if (f < nf) {
-                    nb[f][c] = nbase[f][c * cstride + noff[f]];
+                    nb[f - NIN][c] = nbase[f][c * cstride + noff[f]];
                 } else {
-                    nb[f][c].x = 0;
-                    nb[f][c].y = 0;
+                    nb[f - NIN][c].x = 0;
+                    nb[f - NIN][c].y = 0;
                 }
             }
         // stencil: sum_f w_f psi_t(f); out-of-box neighbours carry weight 0.  Same-x faces need
         // no per-lane test (a live lane's own x is inside the box): wave-uniform weight.
+        if constexpr (NIN > 0) {
+            __shared__ V2 ex[4][C][64];
 #pragma unroll
-        for (int f = 0; f < DEG; ++f) {
+            for (int c = 0; c < C; ++c) {
+                V2 o;
+                o.x = pr[c];
+                o.y = pi[c];
+                ex[threadIdx.x >> 6][c][threadIdx.x & 63] = o;
+            }
+            exchange_barrier();
+#pragma unroll
+            for (int f = 0; f < NIN; ++f)
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    const V2 o = ex[exchange_wave(f)][c][threadIdx.x & 63];
+                    ar[c] += wt[f] * o.x;
+                    ai[c] += wt[f] * o.y;
+                }
+        }
+#pragma unroll
+        for (int f = NIN; f < DEG; ++f) {
             const R w = (dxf[f] == 0 || xok[f]) ? wu[f] : (R)0;
 #pragma unroll
             for (int c = 0; c < C; ++c) {
-                ar[c] += w * nb[f][c].x;
-                ai[c] += w * nb[f][c].y;
+                ar[c] += w * nb[f - NIN][c].x;
+                ai[c] += w * nb[f - NIN][c].y;
             }
         }
         const R wsum = table_wsum<R>(a.tb)[v];
@@ -215,6 +234,8 @@ __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, int sweep,
             if (act) nt_store<R>(o, &nxt[idx]);
         }
         if constexpr (MODE == MODE_ITP) part *= a.tb.dv[v];
+    } else if constexpr (NIN > 0) {
+        exchange_barrier();
     }
 
     if constexpr (MODE == MODE_ITP) {
@@ -240,7 +261,7 @@ typedef float f4a __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
 typedef float f2n __attribute__((ext_vector_type(2)));
 
-template <int C, int DEG, int MODE, bool ROWS>
+template <int C, int DEG, int MODE, bool ROWS, int NIN>
 __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, int b, int nb)
 {
     const Geometry &g = a.g;
@@ -370,18 +391,43 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
 #pragma unroll
         for (int f0 = 0; f0 < DEG; f0 += FB) {
             if (f0 > 0 && f0 >= nf) break;
-            f4u nbv[FB][C];
+            constexpr int N0 = NIN;  // (exchanging tables have one batch)
+            f4u nbv[FB - N0][C];
 #pragma unroll
-            for (int k = 0; k < FB; ++k)
+            for (int k = N0; k < FB; ++k)
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
                     if (f0 + k < nf)
-                        nbv[k][c] = *(const f4u *)(nbase[f0 + k] + c * cstride);
+                        nbv[k - N0][c] = *(const f4u *)(nbase[f0 + k] + c * cstride);
                     else
-                        nbv[k][c] = (f4u)(0.f);
+                        nbv[k - N0][c] = (f4u)(0.f);
                 }
+            if constexpr (NIN > 0) {
+                static_assert(NIN == 0 || FB == DEG, "one batch");
+                __shared__ f4a ex[4][C][64];
 #pragma unroll
-            for (int k = 0; k < FB; ++k) {
+                for (int c = 0; c < C; ++c) {
+                    f4a o;
+                    o.x = pr[0][c];
+                    o.y = pi[0][c];
+                    o.z = pr[1][c];
+                    o.w = pi[1][c];
+                    ex[threadIdx.x >> 6][c][threadIdx.x & 63] = o;
+                }
+                exchange_barrier();
+#pragma unroll
+                for (int f = 0; f < NIN; ++f)
+#pragma unroll
+                    for (int c = 0; c < C; ++c) {
+                        const f4a e = ex[exchange_wave(f)][c][threadIdx.x & 63];
+                        ar[0][c] += wt[f] * e.x;
+                        ai[0][c] += wt[f] * e.y;
+                        ar[1][c] += wt[f] * e.z;
+                        ai[1][c] += wt[f] * e.w;
+                    }
+            }
+#pragma unroll
+            for (int k = N0; k < FB; ++k) {
                 const int f = f0 + k;
                 const float w = wf[f];
                 if (dxf[f] == 0) {
@@ -389,7 +435,7 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
                     // box (the second value of a lone last x is never stored): no per-lane masks
 #pragma unroll
                     for (int c = 0; c < C; ++c) {
-                        const f4u e = nbv[k][c];
+                        const f4u e = nbv[k - N0][c];
                         ar[0][c] += w * e.x;
                         ai[0][c] += w * e.y;
                         ar[1][c] += w * e.z;
@@ -398,7 +444,7 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
                 } else {
 #pragma unroll
                     for (int c = 0; c < C; ++c) {
-                        const f4u e = nbv[k][c];
+                        const f4u e = nbv[k - N0][c];
                         // values at x0 + dx and x0 + 1 + dx from the clamped pair
                         float n0r = sh[f] == 0 ? e.x : e.z, n0i = sh[f] == 0 ? e.y : e.w;
                         float n1r = sh[f] == 0 ? e.z : e.x, n1i = sh[f] == 0 ? e.w : e.y;
@@ -494,6 +540,8 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
             }
         }
         if constexpr (MODE == MODE_ITP) part *= a.tb.dv[v];
+    } else if constexpr (NIN > 0) {
+        exchange_barrier();
     }
 
     if constexpr (MODE == MODE_ITP) {
@@ -506,21 +554,21 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
 }
 
 // X: the lane form (lane_form).
-template <typename R, int C, int DEG, int MODE, int X>
+template <typename R, int C, int DEG, int MODE, int X, int NIN = 0>
 __device__ __forceinline__ void sweep_body(const SweepArgs &a, int sweep, int b, int nb)
 {
     if constexpr (X == 3)
-        sweep_body_pair<C, DEG, MODE, true>(a, sweep, b, nb);
+        sweep_body_pair<C, DEG, MODE, true, NIN>(a, sweep, b, nb);
     else if constexpr (X == 2)
-        sweep_body_pair<C, DEG, MODE, false>(a, sweep, b, nb);
+        sweep_body_pair<C, DEG, MODE, false, NIN>(a, sweep, b, nb);
     else
-        sweep_body_single<R, C, DEG, MODE, X == 4>(a, sweep, b, nb);
+        sweep_body_single<R, C, DEG, MODE, X == 4, NIN>(a, sweep, b, nb);
 }
 
-template <typename R, int C, int DEG, int MODE, int X>
+template <typename R, int C, int DEG, int MODE, int X, int NIN>
 __global__ __launch_bounds__(256) void k_sweep(SweepArgs a)
 {
-    sweep_body<R, C, DEG, MODE, X>(a, a.sweep, sweep_order(a.g, blockIdx.x, gridDim.x, a.order), gridDim.x);
+    sweep_body<R, C, DEG, MODE, X, NIN>(a, a.sweep, sweep_order(a.g, blockIdx.x, gridDim.x, a.order), gridDim.x);
 }
 
 // One leapfrog sweep of every member of an ensemble group in a single launch (a group: the
@@ -528,7 +576,7 @@ __global__ __launch_bounds__(256) void k_sweep(SweepArgs a)
 // specialised as a single run's).  Member m owns workgroups [begin_m, begin_m + blocks_m)
 // (begin_m a multiple of 8, so the XCD remap of the member's own range stays valid); its
 // arguments for parity p are m.args[p].
-template <typename R, int C, int DEG, int X>
+template <typename R, int C, int DEG, int X, int NIN>
 __global__ __launch_bounds__(256) void k_ensemble_sweep(EnsembleArgs e)
 {
     // parity-1 sweeps take the whole launch in reverse (members included), keeping each
@@ -547,7 +595,7 @@ __global__ __launch_bounds__(256) void k_ensemble_sweep(EnsembleArgs e)
     if (local >= m.blocks) return;  // padding workgroup (uniform)
     const SweepArgs &a = m.args[e.parity];
     const int sweep = e.sweep + (e.sweep_base ? *e.sweep_base : 0);
-    sweep_body<R, C, DEG, MODE_UPDATE, X>(a, sweep, local, m.blocks);
+    sweep_body<R, C, DEG, MODE_UPDATE, X, NIN>(a, sweep, local, m.blocks);
 }
 
 __global__ void k_advance_base(int *base, int by)
@@ -860,7 +908,7 @@ __global__ __launch_bounds__(256) void k_aux(AuxArgs a)
         if (a.ref) {
             const long long line = (long long)g.nx * g.V;
             const long long plane = line * g.ny, comp = plane * g.nz;
-            const long long at = (long long)z * plane + (long long)y * line + (long long)x * g.V + v;
+            const long long at = (long long)z * plane + (long long)y * line + (long long)x * g.V + a.tb.abi[v];
             double an = 0, dn = 0;
 #pragma unroll
             for (int c = 0; c < C; ++c) {
@@ -1025,7 +1073,7 @@ __global__ __launch_bounds__(256) void k_fill_tf(Geometry g, Tables tb, Physics 
     const double rz = ph.p0[2] + ph.cell[2] * z + pos[2];
     const double V = 0.5 * (ph.trap2[0] * rx * rx + ph.trap2[1] * ry * ry + ph.trap2[2] * rz * rz) + ph.trap_offset;
     const double a = sqrt(fmax(f.mu - V, 0.0) / f.g);
-    const unsigned long long node = (((unsigned long long)z * g.ny + y) * g.nx + x) * g.V + v;
+    const unsigned long long node = (((unsigned long long)z * g.ny + y) * g.nx + x) * g.V + tb.abi[v];
     vec2_t<R> *out = (vec2_t<R> *)psi;
     for (int c = 0; c < ncomp; ++c) {
         double er = 0, ei = 0;
@@ -1121,12 +1169,12 @@ __global__ __launch_bounds__(256) void k_project(Geometry g, vec2_t<R> *psi, int
 // psi_m += amp sqrt(n) eps_m, eps_m uniform in the unit disk from the counter hash of (seed,
 // unknown in ABI order, 2m / 2m + 1) -- the variates of k_fill_tf -- n the density before.
 template <typename R, int C>
-__global__ __launch_bounds__(256) void k_noise(Geometry g, vec2_t<R> *psi, double amp, unsigned long long seed)
+__global__ __launch_bounds__(256) void k_noise(Geometry g, const int *abi, vec2_t<R> *psi, double amp, unsigned long long seed)
 {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= (long long)g.nz * g.ny * g.V * g.nx) return;
     const Unknown u = unknown_of(g, i);
-    const unsigned long long node = (((unsigned long long)u.z * g.ny + u.y) * g.nx + u.x) * g.V + u.v;
+    const unsigned long long node = (((unsigned long long)u.z * g.ny + u.y) * g.nx + u.x) * g.V + abi[u.v];
     double pr[C], pi[C], n = 0.0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -1162,11 +1210,11 @@ hipError_t launch_project(int fp64, int ncomp, const Geometry &g, void *psi, int
     return hipGetLastError();
 }
 
-hipError_t launch_noise(int fp64, int ncomp, const Geometry &g, void *psi, double amp, unsigned long long seed,
+hipError_t launch_noise(int fp64, int ncomp, const Geometry &g, const Tables &tb, void *psi, double amp, unsigned long long seed,
                         hipStream_t s)
 {
     const unsigned grid = (unsigned)(((long long)g.nz * g.ny * g.V * g.nx + 255) / 256);
-#define NZ(R, C) hipLaunchKernelGGL((k_noise<R, C>), dim3(grid), dim3(256), 0, s, g, (vec2_t<R> *)psi, amp, seed)
+#define NZ(R, C) hipLaunchKernelGGL((k_noise<R, C>), dim3(grid), dim3(256), 0, s, g, tb.abi, (vec2_t<R> *)psi, amp, seed)
     if (fp64) {
         if (ncomp == 1) NZ(double, 1); else if (ncomp == 3) NZ(double, 3); else NZ(double, 5);
     } else {
@@ -1196,13 +1244,13 @@ hipError_t launch_fill_tf(int fp64, const Geometry &g, const Tables &tb, const P
 //                    = m + i n; theta = atan2(-2 m.n, |m|^2 - |n|^2) / 2 in [0, pi) makes u = Re(a e^{i theta}),
 //                    v = Im(a e^{i theta}) orthogonal; (u, v) ordered so that |u| >= |v|; out = u, v, theta.
 template <typename R, int C>
-__global__ __launch_bounds__(256) void k_local_fields(Geometry g, const vec2_t<R> *psi, int kind, double *out)
+__global__ __launch_bounds__(256) void k_local_fields(Geometry g, const int *place, const vec2_t<R> *psi, int kind, double *out)
 {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     const long long total = (long long)g.nz * g.ny * g.nx * g.V;
     if (i >= total) return;
     long long r = i;
-    const int v = (int)(r % g.V);
+    const int v = place[(int)(r % g.V)];
     r /= g.V;
     const int x = (int)(r % g.nx);
     r /= g.nx;
@@ -1265,12 +1313,12 @@ __global__ __launch_bounds__(256) void k_local_fields(Geometry g, const vec2_t<R
     }
 }
 
-hipError_t launch_local_fields(int fp64, int ncomp, const Geometry &g, const void *psi, int kind, double *out,
+hipError_t launch_local_fields(int fp64, int ncomp, const Geometry &g, const Tables &tb, const void *psi, int kind, double *out,
                                hipStream_t s)
 {
     const long long total = (long long)g.nz * g.ny * g.nx * g.V;
     const unsigned grid = (unsigned)((total + 255) / 256);
-#define LF(R, C) hipLaunchKernelGGL((k_local_fields<R, C>), dim3(grid), dim3(256), 0, s, g, (const vec2_t<R> *)psi, kind, out)
+#define LF(R, C) hipLaunchKernelGGL((k_local_fields<R, C>), dim3(grid), dim3(256), 0, s, g, tb.place, (const vec2_t<R> *)psi, kind, out)
     if (fp64) {
         if (ncomp == 1) LF(double, 1); else if (ncomp == 3) LF(double, 3); else LF(double, 5);
     } else {
@@ -1308,14 +1356,14 @@ hipError_t launch_stream(int kind, const void *a, void *b, long long n16, hipStr
 
 // ABI index (c, z, y, x, v) <-> device index (c, z, y, v, x)
 template <typename R, bool PACK>
-__global__ __launch_bounds__(256) void k_pack(Geometry g, int ncomp, const double2 *abi_in, double2 *abi_out,
+__global__ __launch_bounds__(256) void k_pack(Geometry g, const int *place, int ncomp, const double2 *abi_in, double2 *abi_out,
                                               const vec2_t<R> *dev_in, vec2_t<R> *dev_out)
 {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     const long long total = (long long)ncomp * g.nz * g.ny * g.nx * g.V;
     if (i >= total) return;
     long long r = i;
-    const int v = (int)(r % g.V);
+    const int v = place[(int)(r % g.V)];
     r /= g.V;
     const int x = (int)(r % g.nx);
     r /= g.nx;
@@ -1340,18 +1388,27 @@ __global__ __launch_bounds__(256) void k_pack(Geometry g, int ncomp, const doubl
 
 static inline unsigned grid1(long long n) { return (unsigned)((n + 255) / 256); }
 
-template <typename R, int C, int DEG, int X>
-static hipError_t sweep_mode_x(int mode, const SweepArgs &a, hipStream_t s)
+template <typename R, int C, int DEG, int X, int NIN>
+static hipError_t sweep_mode_n(int mode, const SweepArgs &a, hipStream_t s)
 {
     dim3 grid(a.g.blocks), block(256);
     switch (mode) {
-    case MODE_UPDATE: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_UPDATE, X>), grid, block, 0, s, a); break;
-    case MODE_EULER: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_EULER, X>), grid, block, 0, s, a); break;
-    case MODE_ITP: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_ITP, X>), grid, block, 0, s, a); break;
-    case MODE_HPSI: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_HPSI, X>), grid, block, 0, s, a); break;
+    case MODE_UPDATE: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_UPDATE, X, NIN>), grid, block, 0, s, a); break;
+    case MODE_EULER: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_EULER, X, NIN>), grid, block, 0, s, a); break;
+    case MODE_ITP: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_ITP, X, NIN>), grid, block, 0, s, a); break;
+    case MODE_HPSI: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_HPSI, X, NIN>), grid, block, 0, s, a); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+template <typename R, int C, int DEG, int X>
+static hipError_t sweep_mode_x(int mode, const SweepArgs &a, hipStream_t s)
+{
+    if constexpr (exchange_ok(DEG, C)) {
+        if (a.g.exchange) return sweep_mode_n<R, C, DEG, X, 2>(mode, a, s);
+    }
+    return sweep_mode_n<R, C, DEG, X, 0>(mode, a, s);
 }
 
 template <typename R, int C, int DEG>
@@ -1446,60 +1503,61 @@ hipError_t launch_aux(int fp64, int ncomp, const AuxArgs &a, hipStream_t s)
     return fp64 ? aux_comp<double>(ncomp, a, s) : aux_comp<float>(ncomp, a, s);
 }
 
-template <typename R, int C, int DEG>
-static hipError_t ens_x(int form, const EnsembleArgs &e, int blocks, hipStream_t s)
+template <typename R, int C, int DEG, int X>
+static hipError_t ens_n(int exchange, const EnsembleArgs &e, int blocks, hipStream_t s)
 {
     dim3 grid(blocks), block(256);
-    if (form == 1) {
-        hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, 1>), grid, block, 0, s, e);
-        return hipGetLastError();
-    }
-    if constexpr (std::is_same<R, double>::value) {
-        if (form == 4) {
-            hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, 4>), grid, block, 0, s, e);
+    if constexpr (exchange_ok(DEG, C)) {
+        if (exchange) {
+            hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, X, 2>), grid, block, 0, s, e);
             return hipGetLastError();
         }
+    }
+    hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, X, 0>), grid, block, 0, s, e);
+    return hipGetLastError();
+}
+
+template <typename R, int C, int DEG>
+static hipError_t ens_x(int form, int exchange, const EnsembleArgs &e, int blocks, hipStream_t s)
+{
+    if (form == 1) return ens_n<R, C, DEG, 1>(exchange, e, blocks, s);
+    if constexpr (std::is_same<R, double>::value) {
+        if (form == 4) return ens_n<R, C, DEG, 4>(exchange, e, blocks, s);
     }
     if constexpr (pair_lanes_ok(std::is_same<R, double>::value, DEG, C)) {
-        if (form == 2) {
-            hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, 2>), grid, block, 0, s, e);
-            return hipGetLastError();
-        }
-        if (form == 3) {
-            hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, 3>), grid, block, 0, s, e);
-            return hipGetLastError();
-        }
+        if (form == 2) return ens_n<R, C, DEG, 2>(exchange, e, blocks, s);
+        if (form == 3) return ens_n<R, C, DEG, 3>(exchange, e, blocks, s);
     }
     return hipErrorInvalidValue;
 }
 
 template <typename R, int C>
-static hipError_t ens_deg(int deg, int form, const EnsembleArgs &e, int blocks, hipStream_t s)
+static hipError_t ens_deg(int deg, int form, int exchange, const EnsembleArgs &e, int blocks, hipStream_t s)
 {
     switch (deg) {
-    case 4: return ens_x<R, C, 4>(form, e, blocks, s);
-    case 6: return ens_x<R, C, 6>(form, e, blocks, s);
-    case 8: return ens_x<R, C, 8>(form, e, blocks, s);
+    case 4: return ens_x<R, C, 4>(form, exchange, e, blocks, s);
+    case 6: return ens_x<R, C, 6>(form, exchange, e, blocks, s);
+    case 8: return ens_x<R, C, 8>(form, exchange, e, blocks, s);
     default: return hipErrorInvalidValue;
     }
 }
 
 template <typename R>
-static hipError_t ens_comp(int ncomp, int deg, int form, const EnsembleArgs &e, int blocks, hipStream_t s)
+static hipError_t ens_comp(int ncomp, int deg, int form, int exchange, const EnsembleArgs &e, int blocks, hipStream_t s)
 {
     switch (ncomp) {
-    case 1: return ens_deg<R, 1>(deg, form, e, blocks, s);
-    case 3: return ens_deg<R, 3>(deg, form, e, blocks, s);
-    case 5: return ens_deg<R, 5>(deg, form, e, blocks, s);
+    case 1: return ens_deg<R, 1>(deg, form, exchange, e, blocks, s);
+    case 3: return ens_deg<R, 3>(deg, form, exchange, e, blocks, s);
+    case 5: return ens_deg<R, 5>(deg, form, exchange, e, blocks, s);
     default: return hipErrorInvalidValue;
     }
 }
 
-hipError_t launch_ensemble_sweep(int fp64, int ncomp, int deg, int form, const EnsembleArgs &e, int blocks,
-                                 hipStream_t s)
+hipError_t launch_ensemble_sweep(int fp64, int ncomp, int deg, int form, int exchange, const EnsembleArgs &e,
+                                 int blocks, hipStream_t s)
 {
-    return fp64 ? ens_comp<double>(ncomp, deg, form, e, blocks, s)
-                : ens_comp<float>(ncomp, deg, form, e, blocks, s);
+    return fp64 ? ens_comp<double>(ncomp, deg, form, exchange, e, blocks, s)
+                : ens_comp<float>(ncomp, deg, form, exchange, e, blocks, s);
 }
 
 hipError_t launch_advance_base(int *base, int by, hipStream_t s)
@@ -1577,26 +1635,26 @@ hipError_t launch_phase_copy(int fp64, const void *src, void *dst, long long nel
     return hipGetLastError();
 }
 
-hipError_t launch_pack(int fp64, const Geometry &g, int ncomp, const double *abi, void *dev, hipStream_t s)
+hipError_t launch_pack(int fp64, const Geometry &g, const Tables &tb, int ncomp, const double *abi, void *dev, hipStream_t s)
 {
     const long long total = (long long)ncomp * g.nz * g.ny * g.nx * g.V;
     if (fp64)
-        hipLaunchKernelGGL((k_pack<double, true>), dim3(grid1(total)), dim3(256), 0, s, g, ncomp,
+        hipLaunchKernelGGL((k_pack<double, true>), dim3(grid1(total)), dim3(256), 0, s, g, tb.place, ncomp,
                            (const double2 *)abi, nullptr, nullptr, (double2 *)dev);
     else
-        hipLaunchKernelGGL((k_pack<float, true>), dim3(grid1(total)), dim3(256), 0, s, g, ncomp,
+        hipLaunchKernelGGL((k_pack<float, true>), dim3(grid1(total)), dim3(256), 0, s, g, tb.place, ncomp,
                            (const double2 *)abi, nullptr, nullptr, (float2 *)dev);
     return hipGetLastError();
 }
 
-hipError_t launch_unpack(int fp64, const Geometry &g, int ncomp, const void *dev, double *abi, hipStream_t s)
+hipError_t launch_unpack(int fp64, const Geometry &g, const Tables &tb, int ncomp, const void *dev, double *abi, hipStream_t s)
 {
     const long long total = (long long)ncomp * g.nz * g.ny * g.nx * g.V;
     if (fp64)
-        hipLaunchKernelGGL((k_pack<double, false>), dim3(grid1(total)), dim3(256), 0, s, g, ncomp, nullptr,
+        hipLaunchKernelGGL((k_pack<double, false>), dim3(grid1(total)), dim3(256), 0, s, g, tb.place, ncomp, nullptr,
                            (double2 *)abi, (const double2 *)dev, nullptr);
     else
-        hipLaunchKernelGGL((k_pack<float, false>), dim3(grid1(total)), dim3(256), 0, s, g, ncomp, nullptr,
+        hipLaunchKernelGGL((k_pack<float, false>), dim3(grid1(total)), dim3(256), 0, s, g, tb.place, ncomp, nullptr,
                            (double2 *)abi, (const float2 *)dev, nullptr);
     return hipGetLastError();
 }
