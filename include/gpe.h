@@ -338,7 +338,10 @@ int gpe_fill_thomas_fermi(gpe_ctx *ctx, double g, double mu, const double *weigh
  * 3-level leapfrog with checkpoints every K sweeps and recomputation (FP64 accumulation).
  * Starts from level 0 (call right after gpe_set_state); requires GPE_SCHEME_LEAPFROG3,
  * alpha = 0 and no ramp on the quadratic field (qscale_q = qscale_b = 0).  On return the
- * context holds psi_N (level 0) and psi_{N-1} (level 1). */
+ * context holds psi_N (level 0) and psi_{N-1} (level 1).  The buffers (two levels a checkpoint,
+ * a segment of at most K levels, two adjoint levels) stay with the context for its next call
+ * while half of the device is free; they are given back when an allocation of this library
+ * fails, and by gpe_destroy. */
 #define GPE_OBJ_OVERLAP 0         /* J = |<target|psi_N>|^2, <a|b> = sum dv conj(a) b */
 #define GPE_OBJ_ENERGY 1          /* J = E[psi_N] (GP energy functional)              */
 #define GPE_OBJ_MAGNETIZATION_Z 2 /* J = sum dv psi^dag f_z psi                         */

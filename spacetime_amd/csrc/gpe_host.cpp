@@ -13,6 +13,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <set>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -62,7 +63,21 @@ void ramp_channel(const std::vector<double> &val, const std::vector<double> &dur
 
 }  // namespace
 
+// Device memory a context keeps between calls that need a lot of it (the adjoint's levels): the
+// driver clears what is freed, so freeing and allocating gigabytes on every call costs from
+// nothing to seconds (4.6 GB in one block: 134 ms a call once the first few have gone through; in
+// blocks of 75 MB 17 ms; 18 GB up to 5 s), the kernels of a 200-sweep call on spin-1 BCC 64^3 25 ms.
+// Idle workspaces are given back when an allocation of the library fails, when less than half of
+// the device would stay free, and with their context.
+struct Workspace {
+    void *p = nullptr;
+    size_t bytes = 0;
+    int device = 0;
+    bool busy = false;
+};
+
 struct gpe_ctx {
+    Workspace ws;    // guarded by g_ws_mutex
     gpe_config cfg{};
     const LatticeTable *lat = nullptr;
     Geometry g{};    // one x per lane: observables, packing, adjoint
@@ -75,6 +90,7 @@ struct gpe_ctx {
     size_t elem_bytes = 0;   // bytes of one complex element
     long long level_elems = 0;
     hipStream_t stream = nullptr;
+    hipStream_t copy_stream = nullptr;  // uploads beside the sweeps (adjoint target), made on first use
     int device = 0;
     void *level[2] = {nullptr, nullptr};
     // tables
@@ -126,6 +142,86 @@ int hip_fail(gpe_ctx *c, hipError_t e, const char *where)
         hipError_t e_ = (call);                                \
         if (e_ != hipSuccess) return hip_fail(ctx, e_, #call); \
     } while (0)
+
+std::mutex &g_ws_mutex = *new std::mutex;  // never destroyed: a context may outlive static objects
+std::set<Workspace *> &g_workspaces = *new std::set<Workspace *>;  // those that hold memory
+
+void drop_workspace(Workspace *w)  // with g_ws_mutex held
+{
+    if (!w->p) return;
+    (void)hipFree(w->p);
+    w->p = nullptr;
+    w->bytes = 0;
+    g_workspaces.erase(w);
+}
+
+// hipMalloc; where that fails, again after the device's idle workspaces are given back.
+hipError_t device_malloc(void **out, size_t bytes, int device)
+{
+    hipError_t e = hipMalloc(out, bytes);
+    if (e == hipSuccess) return e;
+    {
+        std::lock_guard<std::mutex> lk(g_ws_mutex);
+        std::vector<Workspace *> idle;
+        for (Workspace *w : g_workspaces)
+            if (!w->busy && w->device == device) idle.push_back(w);
+        if (idle.empty()) return e;
+        for (Workspace *w : idle) drop_workspace(w);
+    }
+    (void)hipGetLastError();
+    return hipMalloc(out, bytes);
+}
+
+// At least `bytes` of the context's workspace, until end_workspace.
+hipError_t begin_workspace(gpe_ctx *c, size_t bytes, char **out)
+{
+    Workspace &w = c->ws;
+    {
+        std::lock_guard<std::mutex> lk(g_ws_mutex);
+        if (w.bytes >= bytes) {
+            w.busy = true;
+            *out = (char *)w.p;
+            return hipSuccess;
+        }
+        drop_workspace(&w);
+    }
+    void *p = nullptr;
+    const hipError_t e = device_malloc(&p, bytes, c->device);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return e;
+    }
+    std::lock_guard<std::mutex> lk(g_ws_mutex);
+    w.p = p;
+    w.bytes = bytes;
+    w.device = c->device;
+    w.busy = true;
+    g_workspaces.insert(&w);
+    *out = (char *)p;
+    return hipSuccess;
+}
+
+// `to` takes over the workspace of `from` (both idle).
+void move_workspace(Workspace *from, Workspace *to)
+{
+    std::lock_guard<std::mutex> lk(g_ws_mutex);
+    if (!from->p) return;
+    drop_workspace(to);
+    *to = *from;
+    g_workspaces.erase(from);
+    g_workspaces.insert(to);
+    *from = Workspace{};
+}
+
+// The work on the workspace has ended (its streams synchronised): keep it or give it back.
+void end_workspace(gpe_ctx *c)
+{
+    size_t avail = 0, total = 0;
+    const bool known = hipMemGetInfo(&avail, &total) == hipSuccess;
+    std::lock_guard<std::mutex> lk(g_ws_mutex);
+    c->ws.busy = false;
+    if (!known || avail < total / 2) drop_workspace(&c->ws);
+}
 
 double sweep_dt(const gpe_ctx *c) { return c->cfg.scheme == GPE_SCHEME_STAGGERED ? 0.5 * c->cfg.dt : c->cfg.dt; }
 
@@ -576,7 +672,7 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     c->gr = reduce_geometry(g, c->red_blocks, &c->gr_segs);
     const size_t lbytes = (size_t)c->level_elems * c->elem_bytes;
     for (int l = 0; l < 2 && !rc; ++l) {
-        if ((e = hipMalloc(&c->level[l], lbytes)) != hipSuccess)
+        if ((e = device_malloc(&c->level[l], lbytes, c->device)) != hipSuccess)
             rc = GPE_ENOMEM;
         else if ((e = hipMemsetAsync(c->level[l], 0, lbytes, c->stream)) != hipSuccess)
             rc = hip_fail(c, e, "hipMemset");
@@ -689,6 +785,10 @@ int gpe_destroy(gpe_ctx *c)
 {
     if (!c) return GPE_EINVAL;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    {
+        std::lock_guard<std::mutex> lk(g_ws_mutex);
+        drop_workspace(&c->ws);
+    }
     for (int l = 0; l < 2; ++l)
         if (c->level[l]) (void)hipFree(c->level[l]);
     void *ptrs[] = {c->d_abi, c->d_nface, c->d_facex, c->d_oface, c->d_ow, c->d_nfwd, c->d_w32, c->d_w64, c->d_wsum32, c->d_wsum64, c->d_pos32,
@@ -700,6 +800,7 @@ int gpe_destroy(gpe_ctx *c)
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
     delete c;
     return GPE_OK;
 }
@@ -1048,7 +1149,8 @@ int gpe_weighted_diff(gpe_ctx *c, int level, const double *ref, double phase_re,
     if (rc) return rc;
     const size_t bytes = 2 * sizeof(double) * (size_t)c->cfg.ncomp * c->cfg.nx * c->cfg.ny * c->cfg.nz * c->g.V;
     double *d = nullptr;
-    if (hipMalloc((void **)&d, bytes) != hipSuccess) return fail(c, GPE_ENOMEM, "reference state does not fit");
+    if (device_malloc((void **)&d, bytes, c->device) != hipSuccess)
+        return fail(c, GPE_ENOMEM, "reference state does not fit");
     hipError_t e = hipMemcpyAsync(d, ref, bytes, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) rc = gpe_weighted_diff_device(c, level, d, phase_re, phase_im, out);
     else rc = hip_fail(c, e, "reference upload");
@@ -1079,7 +1181,8 @@ int gpe_local_fields(gpe_ctx *c, int level, int kind, double *out)
     if (rc) return rc;
     const size_t bytes = sizeof(double) * (size_t)width * (size_t)c->cfg.nx * c->cfg.ny * c->cfg.nz * c->g.V;
     double *d = nullptr;
-    if (hipMalloc((void **)&d, bytes) != hipSuccess) return fail(c, GPE_ENOMEM, "field map does not fit");
+    if (device_malloc((void **)&d, bytes, c->device) != hipSuccess)
+        return fail(c, GPE_ENOMEM, "field map does not fit");
     hipError_t e = launch_local_fields(c->fp64, c->cfg.ncomp, c->g, tables(c), c->level[level], kind, d, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out, d, bytes, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -1252,7 +1355,7 @@ static int adjoint_fp64_copy(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoi
     }
     const size_t abi = (size_t)cfg.ncomp * c->g.nz * c->g.ny * c->g.nx * c->g.V * 2 * sizeof(double);
     double *tmp = nullptr;
-    if (hipMalloc((void **)&tmp, abi) != hipSuccess) {
+    if (device_malloc((void **)&tmp, abi, c->device) != hipSuccess) {
         gpe_destroy(d);
         return fail(c, GPE_ENOMEM, "staging for the FP64 copy does not fit");
     }
@@ -1262,8 +1365,10 @@ static int adjoint_fp64_copy(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoi
     gpe_adjoint_spec s64 = *spec;
     s64.fp64_trajectory = 0;
     if (!rc) {
+        move_workspace(&c->ws, &d->ws);
         rc = gpe_adjoint(d, &s64, res);
         if (rc) c->err = "FP64 copy: " + d->err;
+        move_workspace(&d->ws, &c->ws);
     }
     if (!rc) rc = gpe_get_state_device(d, 0, tmp);
     if (!rc) rc = gpe_set_state_device(c, 0, tmp, t0);
@@ -1298,40 +1403,52 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
 
     const size_t lbytes = (size_t)c->level_elems * c->elem_bytes;
     const int nck = (N + K - 1) / K;
-    std::vector<void *> bufs;
-    auto alloc = [&](void **p, size_t bytes) -> int {
-        if (hipMalloc(p, bytes) != hipSuccess) return GPE_ENOMEM;
-        bufs.push_back(*p);
-        return GPE_OK;
-    };
-    auto release = [&]() {
-        (void)hipStreamSynchronize(c->stream);
-        for (void *p : bufs) (void)hipFree(p);
-        bufs.clear();
-    };
-    std::vector<void *> ck(2 * nck, nullptr), seg(K, nullptr);
-    void *mu[2] = {nullptr, nullptr};
-    void *target = nullptr;
-    double *d_steps = nullptr, *d_part = nullptr;
-    int rc = GPE_OK;
-    for (int i = 0; i < 2 * nck && !rc; ++i) rc = alloc(&ck[i], lbytes);
-    for (int i = 2; i < K && !rc; ++i) rc = alloc(&seg[i], lbytes);  // seg[0], seg[1] alias checkpoints
-    for (int i = 0; i < 2 && !rc; ++i) rc = alloc(&mu[i], lbytes);
-    if (!rc && spec->objective == GPE_OBJ_OVERLAP) rc = alloc(&target, lbytes);
-    if (!rc) rc = alloc((void **)&d_steps, sizeof(double) * ADJ_COUNT * (size_t)N);
-    if (!rc) rc = alloc((void **)&d_part, sizeof(double) * ADJ_COUNT * (size_t)c->g.blocks);
+    const Geometry &g = c->g;
+    const size_t abi = (size_t)c->cfg.ncomp * g.nz * g.ny * g.nx * g.V * 2 * sizeof(double);
+    const bool overlap = spec->objective == GPE_OBJ_OVERLAP;
     // per-sweep sensitivity partials of up to Q consecutive adjoint sweeps, summed in one launch
     // (one two-stage finalize per sweep cost ~15% of the backward pass in launches)
     // the adjoint sweeps run on the forward sweep's traversal (x pairs in FP32)
     const int adj_blocks = c->gs.blocks;
     const size_t sweep_part = (size_t)ADJ_COUNT * adj_blocks;
     const int Q = (int)std::max<size_t>(1, std::min<size_t>((size_t)K, ((size_t)256 << 20) / (sweep_part * 8)));
-    double *d_qpart = nullptr;
-    if (!rc) rc = alloc((void **)&d_qpart, sizeof(double) * sweep_part * Q);
-    if (rc) {
-        release();
-        return fail(c, rc, "adjoint buffers do not fit");
-    }
+    // every buffer of the run in the context's workspace
+    size_t arena_bytes = 0;
+    const auto place = [&](size_t bytes) {
+        const size_t at = arena_bytes;
+        arena_bytes += (bytes + 255) / 256 * 256;
+        return at;
+    };
+    const size_t at_levels = place(0), level_step = (lbytes + 255) / 256 * 256;
+    const int nseg = std::min(K, N);  // levels of the longest segment
+    const int nlevels = 2 * nck + std::max(nseg - 2, 0) + 2 + (overlap ? 1 : 0);
+    arena_bytes += level_step * nlevels;
+    const size_t at_staging = place(overlap ? abi : 0);
+    const size_t at_steps = place(sizeof(double) * ADJ_COUNT * (size_t)N);
+    const size_t at_part = place(sizeof(double) * ADJ_COUNT * (size_t)g.blocks);
+    const size_t at_qpart = place(sizeof(double) * sweep_part * Q);
+    char *arena = nullptr;
+    if (begin_workspace(c, arena_bytes, &arena) != hipSuccess) return fail(c, GPE_ENOMEM, "adjoint buffers do not fit");
+    const auto release = [&]() {
+        (void)hipStreamSynchronize(c->stream);
+        if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);
+        end_workspace(c);
+    };
+    char *level_at = arena + at_levels;
+    const auto next_level = [&]() {
+        void *p = level_at;
+        level_at += level_step;
+        return p;
+    };
+    std::vector<void *> ck(2 * nck), seg(std::max(nseg, 2), nullptr);
+    for (void *&p : ck) p = next_level();
+    for (int i = 2; i < nseg; ++i) seg[i] = next_level();  // seg[0], seg[1] alias checkpoints
+    void *mu[2] = {next_level(), next_level()};
+    void *target = overlap ? next_level() : nullptr;
+    double *staging = (double *)(arena + at_staging);
+    double *d_steps = (double *)(arena + at_steps), *d_part = (double *)(arena + at_part);
+    double *d_qpart = (double *)(arena + at_qpart);
+    int rc = GPE_OK;
     res->checkpoint_bytes = (double)lbytes * 2 * nck;
     res->segment_bytes = (double)lbytes * (K - 2 + 2);
     hipError_t e = hipSuccess;
@@ -1355,28 +1472,37 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
     }
     // ---- forward pass, keeping (psi_jK, psi_jK+1)
     ADJ_CHECK(hipEventRecord(c->ev0, c->stream), "adjoint");
-    ADJ_CHECK(hipMemcpyAsync(ck[0], c->level[0], lbytes, hipMemcpyDeviceToDevice, c->stream), "checkpoint");
-    {
-        SweepArgs a = sweep_args(c, 0, c->level[0], c->level[1], sdt);
-        ADJ_CHECK(launch_sweep(c->fp64, c->cfg.ncomp, MODE_EULER, a, c->stream), "forward Euler");
-        std::swap(c->level[0], c->level[1]);
-    }
-    ADJ_CHECK(hipMemcpyAsync(ck[1], c->level[0], lbytes, hipMemcpyDeviceToDevice, c->stream), "checkpoint");
-    for (int k = 1; k < N; ++k) {  // produces psi_{k+1}
-        SweepArgs a = sweep_args(c, k, c->level[0], c->level[1], 2.0 * sdt);
+    // where psi_m is written: the last segment's levels stay where the reverse pass reads them, so it
+    // recomputes nothing there, the others' first two in their checkpoints, the rest alternate
+    // between the context's levels
+    const int klast = (nck - 1) * K;
+    void *const even = c->level[0], *const odd = c->level[1];
+    const auto at = [&](int m) -> void * {
+        if (m < N && m >= klast && m - klast >= 2) return seg[m - klast];
+        if (m < N && m % K < 2) return ck[2 * (m / K) + m % K];
+        return m & 1 ? odd : even;
+    };
+    ADJ_CHECK(hipMemcpyAsync(ck[0], even, lbytes, hipMemcpyDeviceToDevice, c->stream), "checkpoint");
+    for (int k = 0; k < N; ++k) {  // produces psi_{k+1}
+        SweepArgs a = sweep_args(c, k, at(k), at(k + 1), k == 0 ? sdt : 2.0 * sdt);
         a.order = k & 1;
-        ADJ_CHECK(launch_sweep(c->fp64, c->cfg.ncomp, MODE_UPDATE, a, c->stream), "forward sweep");
-        std::swap(c->level[0], c->level[1]);
-        const int m = k + 1;
-        if (m < N && m % K == 0)
-            ADJ_CHECK(hipMemcpyAsync(ck[2 * (m / K)], c->level[0], lbytes, hipMemcpyDeviceToDevice, c->stream), "ck");
-        if (m <= N && m % K == 1 && m / K < nck)
-            ADJ_CHECK(hipMemcpyAsync(ck[2 * (m / K) + 1], c->level[0], lbytes, hipMemcpyDeviceToDevice, c->stream),
-                      "ck");
+        if (k > 0 && at(k - 1) != at(k + 1)) a.prev = at(k - 1);
+        ADJ_CHECK(launch_sweep(c->fp64, c->cfg.ncomp, k == 0 ? MODE_EULER : MODE_UPDATE, a, c->stream), "forward sweep");
     }
+    // psi_N in level 0, psi_{N-1} in level 1
+    c->level[0] = at(N);
+    c->level[1] = c->level[0] == even ? odd : even;
+    ADJ_CHECK(hipMemcpyAsync(c->level[1], at(N - 1), lbytes, hipMemcpyDeviceToDevice, c->stream), "psi_{N-1}");
     c->sweeps = N;
     c->level1_valid = true;
     ADJ_CHECK(hipEventRecord(c->ev1, c->stream), "adjoint");
+    if (overlap) {  // the host's copy of the target goes up while the forward sweeps run
+        if (!c->copy_stream)
+            ADJ_CHECK(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking), "copy stream");
+        ADJ_CHECK(hipMemcpyAsync(staging, spec->target, abi, hipMemcpyHostToDevice, c->copy_stream), "target");
+        ADJ_CHECK(launch_pack(c->fp64, g, tables(c), c->cfg.ncomp, staging, target, c->copy_stream), "pack target");
+        ADJ_CHECK(hipStreamSynchronize(c->copy_stream), "target");
+    }
     ADJ_CHECK(hipEventSynchronize(c->ev1), "adjoint");
     float fms = 0.f;
     ADJ_CHECK(hipEventElapsedTime(&fms, c->ev0, c->ev1), "adjoint");
@@ -1398,14 +1524,7 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
     double J = 0.0;
     double explicit_mom[4] = {0, 0, 0, 0};  // energy: sum dv r_a^2 n, s sum dv (dx Fx + dy Fy - 2 dz Fz)
     double explicit_mag[3] = {0, 0, 0};
-    if (spec->objective == GPE_OBJ_OVERLAP) {
-        const Geometry &g = c->g;
-        const size_t abi = (size_t)c->cfg.ncomp * g.nz * g.ny * g.nx * g.V * 2 * sizeof(double);
-        double *staging = nullptr;
-        ADJ_CHECK(hipMalloc((void **)&staging, abi), "staging");
-        bufs.push_back(staging);
-        ADJ_CHECK(hipMemcpyAsync(staging, spec->target, abi, hipMemcpyHostToDevice, c->stream), "target");
-        ADJ_CHECK(launch_pack(c->fp64, g, tables(c), c->cfg.ncomp, staging, target, c->stream), "pack target");
+    if (overlap) {
         oa.mode = OBJ_PARTIALS;
         ADJ_CHECK(launch_objective(c->fp64, c->cfg.ncomp, oa, c->stream), "overlap");
         ADJ_CHECK(launch_finalize(d_part, g.blocks, 2, -1, c->d_scalars + 32, c->d_red, c->stream), "overlap sum");
@@ -1460,7 +1579,7 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
         const int klo = j * K, khi = std::min((j + 1) * K - 1, N - 1);
         seg[0] = ck[2 * j];
         seg[1] = ck[2 * j + 1];
-        for (int m = klo + 1; m < khi; ++m) {  // psi_{m+1} = psi_{m-1} - 2i dt H psi_m
+        for (int m = klo + 1; m < khi && j < nck - 1; ++m) {  // psi_{m+1} = psi_{m-1} - 2i dt H psi_m
             SweepArgs a = sweep_args(c, m, seg[m - klo], seg[m + 1 - klo], 2.0 * sdt);
             a.prev = seg[m - 1 - klo];
             a.order = m & 1;
@@ -1908,7 +2027,8 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
                 c->gs = gs;
             }
         } trial{c, c->g, c->gs};
-        if (hipMalloc(&trial.s0, lbytes) != hipSuccess || hipMalloc(&trial.s1, lbytes) != hipSuccess)
+        if (device_malloc(&trial.s0, lbytes, c->device) != hipSuccess ||
+            device_malloc(&trial.s1, lbytes, c->device) != hipSuccess)
             return fail(c, GPE_ENOMEM, "autotune scratch does not fit");
         HIPCALL(c, hipMemcpyAsync(trial.s0, c->level[0], lbytes, hipMemcpyDeviceToDevice, c->stream));
         HIPCALL(c, hipMemcpyAsync(trial.s1, c->level[1], lbytes, hipMemcpyDeviceToDevice, c->stream));
