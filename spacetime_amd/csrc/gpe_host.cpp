@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <algorithm>
@@ -223,6 +224,24 @@ void end_workspace(gpe_ctx *c)
     if (!known || avail < total / 2) drop_workspace(&c->ws);
 }
 
+// Wait for an event: poll for up to SPIN_US, then block.  A blocking wait of more than about 20 us
+// sleeps and wakes 20 us late (10 sweeps of a small box, 42 us of work: 84 us a call, 65 polled).
+// Shorter waits spin inside hipStreamSynchronize, which is cheaper than an event of their own.
+constexpr double SPIN_US = 1000.0;
+
+hipError_t wait_event(hipEvent_t ev)
+{
+    const auto t0 = std::chrono::steady_clock::now();
+    hipError_t e = hipEventQuery(ev);
+    if (e != hipErrorNotReady) return e;
+    while ((e = hipEventQuery(ev)) == hipErrorNotReady) {
+        const std::chrono::duration<double, std::micro> us = std::chrono::steady_clock::now() - t0;
+        if (us.count() > SPIN_US) break;
+    }
+    (void)hipGetLastError();  // "not ready" is no error of ours
+    return e == hipErrorNotReady ? hipEventSynchronize(ev) : e;
+}
+
 double sweep_dt(const gpe_ctx *c) { return c->cfg.scheme == GPE_SCHEME_STAGGERED ? 0.5 * c->cfg.dt : c->cfg.dt; }
 
 FieldRec field_at(const gpe_ctx *c, double t)
@@ -357,12 +376,21 @@ static double lane_use(int rows, int pairs)
 }
 
 //
-// pack (FP64 sweeps, one x per lane): the rows of a tile are one group wherever one row per wave
-// leaves at least PACK_GAIN of the lanes idle that the packed rows would fill.  Full lines lose
-// nothing by staying (FCC 64^3 runs the one-row body); spin-1 / spin-2 / one component, us a
-// sweep, one row against packed: C15 20^3 54.3 -> 40.7, Cube 75x61x90 8.7 -> 6.4, BCC 70^3 47.3 ->
-// 42.2, A15 30^3 71.3 -> 66.2, BCC 16^3 4.8 -> 4.2, BCC 96^3 (75% of the lanes) 295.7 -> 293.6.
-constexpr double PACK_GAIN = 0.05;
+// pack (FP64 sweeps, one x per lane): the rows of a tile are one group where one row per wave leaves
+// lanes idle that packed rows would fill.  Where lines are whole 128-byte lines, from 5% of the
+// lanes; otherwise a wave then starts inside cache lines that its neighbour also touches, which
+// costs more than the lanes unless more than half of them idle or the box is small.  us a sweep, one
+// row -> packed: whole lines BCC 40^3 one component 9.9 -> 7.8, FCC 40^3 spin-1 29.0 -> 24.4, C15 24^3
+// spin-2 115 -> 86, A15 48^3 147 -> 137; others C15 20^3 (31% of the lanes) 54.3 -> 40.7, A15 30^3
+// (47%) 71 -> 66, Cube 75x61x90 8.7 -> 6.4, but Z 34^3 spin-2 (53%) 184 -> 196, Z 50^3 105 -> 114, A15 39^3
+// 81 -> 84.  Full lines keep one row.
+bool pack_rows(const Geometry &g)
+{
+    const double one = lane_use(1, g.nx);
+    if (g.ty < 2 || lane_use(g.ty, g.nx) < one + 0.05) return false;
+    const long long waves = (long long)g.ny * g.nz * g.V * ((g.nx + 63) / 64);
+    return g.lx % 8 == 0 || one < 0.5 || waves <= 16384;
+}
 
 bool finish_geometry(Geometry &g, bool pack = false)
 {
@@ -393,7 +421,7 @@ bool finish_geometry(Geometry &g, bool pack = false)
                 best = lane_use(r, g.pairs);
                 rows = r;
             }
-    } else if (pack && g.ty > 1 && lane_use(g.ty, g.nx) > lane_use(1, g.nx) + PACK_GAIN) {
+    } else if (pack && pack_rows(g)) {
         rows = g.ty;
     }
     g.rows = rows;
@@ -494,7 +522,8 @@ Geometry base_geometry(const gpe_config &cfg)
     return g;
 }
 
-SweepArgs sweep_args(gpe_ctx *c, int mode_coef_sweep, const void *cur, void *next, double coef)
+// Arguments of one sweep at time t of the run.
+SweepArgs sweep_args(gpe_ctx *c, double t, const void *cur, void *next, double coef)
 {
     SweepArgs a;
     a.g = c->gs;
@@ -503,8 +532,8 @@ SweepArgs sweep_args(gpe_ctx *c, int mode_coef_sweep, const void *cur, void *nex
     a.cur = cur;
     a.next = next;
     a.prev = nullptr;
-    a.fields = c->d_fields;
-    a.sweep = mode_coef_sweep;
+    a.field = field_at(c, t);
+    a.fields = nullptr;
     a.order = 0;
     a.quad = quad_active(c) ? 1 : 0;
     a.loss = c->cfg.alpha != 0.0 ? 1 : 0;
@@ -566,6 +595,9 @@ hipError_t reduce_observables(gpe_ctx *c, int level, double t)
                                 c->stream);
     return e;
 }
+
+// Time of a level.
+double time_of(const gpe_ctx *c, int level) { return c->t0 + (double)(c->sweeps - level) * sweep_dt(c); }
 
 int check_level(gpe_ctx *c, int level)
 {
@@ -920,9 +952,7 @@ int gpe_start(gpe_ctx *c, int mode, double mu)
     if (!c) return GPE_EINVAL;
     const double sdt = sweep_dt(c);
     if (mode == GPE_START_EULER) {
-        int rc = upload_fields(c, c->sweeps, 1);
-        if (rc) return rc;
-        SweepArgs a = sweep_args(c, 0, c->level[0], c->level[1], sdt);
+        SweepArgs a = sweep_args(c, time_of(c, 0), c->level[0], c->level[1], sdt);
         hipError_t e = launch_sweep(c->fp64, c->cfg.ncomp, MODE_EULER, a, c->stream);
         if (e != hipSuccess) return hip_fail(c, e, "forward Euler");
         std::swap(c->level[0], c->level[1]);
@@ -952,29 +982,23 @@ int gpe_step(gpe_ctx *c, int nsteps)
     const int per = c->cfg.scheme == GPE_SCHEME_STAGGERED ? 2 : 1;
     const long long total = (long long)nsteps * per;
     const double coef = 2.0 * sweep_dt(c);
-    const int chunk = 1 << 16;
-    double ms_total = 0.0;
-    for (long long done = 0; done < total;) {
-        const int n = (int)std::min<long long>(chunk, total - done);
-        int rc = upload_fields(c, c->sweeps, n);
-        if (rc) return rc;
-        HIPCALL(c, hipEventRecord(c->ev0, c->stream));
-        for (int k = 0; k < n; ++k) {
-            SweepArgs a = sweep_args(c, k, c->level[0], c->level[1], coef);
-            a.order = (int)(c->sweeps & 1);
-            hipError_t e = launch_sweep(c->fp64, c->cfg.ncomp, MODE_UPDATE, a, c->stream);
-            if (e != hipSuccess) return hip_fail(c, e, "sweep launch");
-            std::swap(c->level[0], c->level[1]);
-            c->sweeps += 1;
-        }
-        HIPCALL(c, hipEventRecord(c->ev1, c->stream));
-        HIPCALL(c, hipEventSynchronize(c->ev1));
-        float ms = 0.f;
-        HIPCALL(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
-        ms_total += ms;
-        done += n;
+    HIPCALL(c, hipEventRecord(c->ev0, c->stream));
+    for (long long k = 0; k < total; ++k) {
+        // the field travels in the kernel's arguments: nothing to upload, and one load less in the
+        // sweep's chain of scalar loads
+        SweepArgs a = sweep_args(c, time_of(c, 0), c->level[0], c->level[1], coef);
+        a.order = (int)(c->sweeps & 1);
+        hipError_t e = launch_sweep(c->fp64, c->cfg.ncomp, MODE_UPDATE, a, c->stream);
+        if (e != hipSuccess) return hip_fail(c, e, "sweep launch");
+        std::swap(c->level[0], c->level[1]);
+        c->sweeps += 1;
+        if ((k & 0xffff) == 0xffff) HIPCALL(c, hipStreamSynchronize(c->stream));  // bounds the queue
     }
-    c->last_ms_per_sweep = ms_total / (double)total;
+    HIPCALL(c, hipEventRecord(c->ev1, c->stream));
+    HIPCALL(c, wait_event(c->ev1));
+    float ms = 0.f;
+    HIPCALL(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
+    c->last_ms_per_sweep = ms / (double)total;
     return GPE_OK;
 }
 
@@ -982,16 +1006,14 @@ int gpe_itp(gpe_ctx *c, int nsteps, double dt_itp)
 {
     if (!c) return GPE_EINVAL;
     if (nsteps < 0 || !(dt_itp > 0.0)) return fail(c, GPE_EINVAL, "bad ITP arguments");
-    int rc = upload_fields(c, c->sweeps, 1);  // field and time of level 0
-    if (rc) return rc;
     double *norm = c->d_scalars + 0;
     double *scale[2] = {c->d_scalars + 1, c->d_scalars + 2};
     // initial scale from the norm of level 0
-    hipError_t e = reduce_observables(c, 0, c->t0 + c->sweeps * sweep_dt(c));
+    hipError_t e = reduce_observables(c, 0, time_of(c, 0));
     if (e == hipSuccess) e = launch_norm_to_scale(c->d_scalars + 8 + OBS_NORM, 1.0, scale[0], c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "ITP initial norm");
     for (int i = 0; i < nsteps; ++i) {
-        SweepArgs a = sweep_args(c, 0, c->level[0], c->level[1], dt_itp);
+        SweepArgs a = sweep_args(c, time_of(c, 0), c->level[0], c->level[1], dt_itp);
         a.scale_in = scale[i & 1];
         a.order = i & 1;
         e = launch_sweep(c->fp64, c->cfg.ncomp, MODE_ITP, a, c->stream);
@@ -1013,7 +1035,7 @@ int gpe_observables(gpe_ctx *c, int level, gpe_observables_t *out)
     if (!out) return fail(c, GPE_EINVAL, "null output");
     int rc = check_level(c, level);
     if (rc) return rc;
-    const double t = c->t0 + (double)(c->sweeps - level) * sweep_dt(c);
+    const double t = time_of(c, level);
     const hipError_t e = reduce_observables(c, level, t);
     if (e != hipSuccess) return hip_fail(c, e, "observables");
     HIPCALL(c, hipStreamSynchronize(c->stream));
@@ -1097,7 +1119,7 @@ int gpe_series_save(gpe_series *s, const char *path)
 // k_aux over a level with an optional device reference state; h[0] = maximum, h[1] = sum.
 static int aux_reduce(gpe_ctx *c, int level, const double *dref, double pre, double pim, double h[AUX_COUNT])
 {
-    const double t = c->t0 + (double)(c->sweeps - level) * sweep_dt(c);
+    const double t = time_of(c, level);
     AuxArgs aa;
     aa.g = c->g;
     aa.tb = tables(c);
@@ -1484,7 +1506,7 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
     };
     ADJ_CHECK(hipMemcpyAsync(ck[0], even, lbytes, hipMemcpyDeviceToDevice, c->stream), "checkpoint");
     for (int k = 0; k < N; ++k) {  // produces psi_{k+1}
-        SweepArgs a = sweep_args(c, k, at(k), at(k + 1), k == 0 ? sdt : 2.0 * sdt);
+        SweepArgs a = sweep_args(c, c->t0 + k * sdt, at(k), at(k + 1), k == 0 ? sdt : 2.0 * sdt);
         a.order = k & 1;
         if (k > 0 && at(k - 1) != at(k + 1)) a.prev = at(k - 1);
         ADJ_CHECK(launch_sweep(c->fp64, c->cfg.ncomp, k == 0 ? MODE_EULER : MODE_UPDATE, a, c->stream), "forward sweep");
@@ -1551,12 +1573,7 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
                                       c->stream), "adjoint");
             ADJ_CHECK(hipStreamSynchronize(c->stream), "adjoint");
             // H psi_N at the time of psi_N into mu[1], then scaled by 2 dv
-            int frc = upload_fields(c, N, 1);
-            if (frc) {
-                release();
-                return frc;
-            }
-            SweepArgs a = sweep_args(c, 0, c->level[0], mu[1], 0.0);
+            SweepArgs a = sweep_args(c, c->t0 + N * sdt, c->level[0], mu[1], 0.0);
             ADJ_CHECK(launch_sweep(c->fp64, c->cfg.ncomp, MODE_HPSI, a, c->stream), "H psi");
             oa.mode = OBJ_ENERGY;
         } else {
@@ -1564,11 +1581,6 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
             oa.mode = OBJ_MAGZ;
         }
         ADJ_CHECK(launch_objective(c->fp64, c->cfg.ncomp, oa, c->stream), "objective grad");
-        int frc = upload_fields(c, 0, N);
-        if (frc) {
-            release();
-            return frc;
-        }
     }
     res->objective = J;
 
@@ -1580,7 +1592,7 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
         seg[0] = ck[2 * j];
         seg[1] = ck[2 * j + 1];
         for (int m = klo + 1; m < khi && j < nck - 1; ++m) {  // psi_{m+1} = psi_{m-1} - 2i dt H psi_m
-            SweepArgs a = sweep_args(c, m, seg[m - klo], seg[m + 1 - klo], 2.0 * sdt);
+            SweepArgs a = sweep_args(c, c->t0 + m * sdt, seg[m - klo], seg[m + 1 - klo], 2.0 * sdt);
             a.prev = seg[m - 1 - klo];
             a.order = m & 1;
             ADJ_CHECK(launch_sweep(c->fp64, c->cfg.ncomp, MODE_UPDATE, a, c->stream), "recompute");
@@ -1691,9 +1703,11 @@ struct EnsembleGroup {
 struct gpe_ensemble {
     std::vector<gpe_ctx *> m;          // sorted by group
     std::vector<Geometry> trav;        // each member's sweep traversal when the ensemble was made
-    std::vector<EnsembleMember> h;
+    std::vector<std::pair<int, int>> span;  // each member's first workgroup and workgroups in its launch
     std::vector<EnsembleGroup> groups;
-    EnsembleMember *d = nullptr;
+    EnsembleMember *d = nullptr;  // records and fields of the current call (up_bytes)
+    char *up = nullptr;           // their pinned staging
+    size_t up_bytes = 0;
     int *d_base = nullptr;
     int ncomp = 0, fp64 = 0, per = 1;
     hipStream_t stream = nullptr;
@@ -1736,7 +1750,6 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
     e->ncomp = c0->cfg.ncomp;
     e->fp64 = c0->fp64;
     e->per = c0->cfg.scheme == GPE_SCHEME_STAGGERED ? 2 : 1;
-    e->h.resize(n);
     int begin = 0;
     bool prev_solo = false;
     for (int i = 0; i < n; ++i) {
@@ -1751,8 +1764,7 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
         }
         prev_solo = solo;
         e->groups.back().count += 1;
-        e->h[i].begin = begin;
-        e->h[i].blocks = c->gs.blocks;
+        e->span.emplace_back(begin, c->gs.blocks);
         begin += (c->gs.blocks + 7) / 8 * 8;
         e->groups.back().blocks = begin;
         e->trav.push_back(c->gs);
@@ -1760,7 +1772,6 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
     }
     int rc = GPE_OK;
     if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess) rc = GPE_EDEVICE;
-    if (!rc && hipMalloc((void **)&e->d, sizeof(EnsembleMember) * n) != hipSuccess) rc = GPE_ENOMEM;
     if (!rc && hipMalloc((void **)&e->d_base, sizeof(int) * 4) != hipSuccess) rc = GPE_ENOMEM;
     if (!rc && (hipEventCreate(&e->ev0) != hipSuccess || hipEventCreate(&e->ev1) != hipSuccess)) rc = GPE_EDEVICE;
     if (rc) {
@@ -1778,6 +1789,7 @@ int gpe_ensemble_destroy(gpe_ensemble *e)
     if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
     if (e->graph) (void)hipGraphDestroy(e->graph);
     if (e->d) (void)hipFree(e->d);
+    if (e->up) (void)hipHostFree(e->up);
     if (e->d_base) (void)hipFree(e->d_base);
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
@@ -1809,15 +1821,39 @@ int gpe_ensemble_step(gpe_ensemble *e, int nsteps, int graph_sweeps)
         if (c->gs.blocks != t.blocks || c->gs.xpl != t.xpl || c->gs.rows != t.rows || c->gs.ty != t.ty ||
             c->gs.xcd_remap != t.xcd_remap || c->gs.v_inner != t.v_inner)
             return ens_fail(e, GPE_ESTATE, "member traversal changed after the ensemble was created");
-        int rc = upload_fields(c, c->sweeps, nsw);
-        if (rc) return ens_fail(e, rc, c->err);
         ENSCALL(e, hipStreamSynchronize(c->stream));
-        const double coef = 2.0 * sweep_dt(c);
-        e->h[i].args[0] = sweep_args(c, 0, c->level[0], c->level[1], coef);
-        e->h[i].args[1] = sweep_args(c, 0, c->level[1], c->level[0], coef);
     }
-    ENSCALL(e, hipMemcpyAsync(e->d, e->h.data(), sizeof(EnsembleMember) * e->h.size(), hipMemcpyHostToDevice,
-                              e->stream));
+    // the members' records and the fields of all their sweeps go up in one copy: members first, then
+    // member i's fields at i nsw
+    const size_t rec = (sizeof(EnsembleMember) * e->m.size() + 255) / 256 * 256;
+    const size_t bytes = rec + sizeof(FieldRec) * e->m.size() * (size_t)nsw;
+    if (bytes > e->up_bytes) {
+        if (e->d) (void)hipFree(e->d);
+        if (e->up) (void)hipHostFree(e->up);
+        e->d = nullptr;
+        e->up = nullptr;
+        e->up_bytes = 0;
+        if (e->gexec) (void)hipGraphExecDestroy(e->gexec);  // captured with the old records' address
+        e->gexec = nullptr;
+        ENSCALL(e, hipMalloc((void **)&e->d, bytes));
+        ENSCALL(e, hipHostMalloc((void **)&e->up, bytes, hipHostMallocDefault));
+        e->up_bytes = bytes;
+    }
+    EnsembleMember *h = (EnsembleMember *)e->up;
+    FieldRec *hf = (FieldRec *)(e->up + rec);
+    const FieldRec *df = (const FieldRec *)((const char *)e->d + rec);
+    for (size_t i = 0; i < e->m.size(); ++i) {
+        gpe_ctx *c = e->m[i];
+        const double coef = 2.0 * sweep_dt(c), sdt = sweep_dt(c);
+        h[i].begin = e->span[i].first;
+        h[i].blocks = e->span[i].second;
+        for (int p = 0; p < 2; ++p) {
+            h[i].args[p] = sweep_args(c, time_of(c, 0), c->level[p], c->level[1 - p], coef);
+            h[i].args[p].fields = df + i * nsw;
+        }
+        for (int k = 0; k < nsw; ++k) hf[i * nsw + k] = field_at(c, c->t0 + (double)(c->sweeps + k) * sdt);
+    }
+    ENSCALL(e, hipMemcpyAsync(e->d, e->up, bytes, hipMemcpyHostToDevice, e->stream));
     // one launch per group per sweep; groups are independent of each other
     auto launch_group = [&](const EnsembleGroup &gr, int k, const int *base, hipStream_t st) -> hipError_t {
         EnsembleArgs a;
@@ -1826,7 +1862,7 @@ int gpe_ensemble_step(gpe_ensemble *e, int nsteps, int graph_sweeps)
         a.parity = k & 1;
         a.sweep = k;
         a.sweep_base = base;
-        for (int i = 0; i < gr.count; ++i) a.begin[i] = e->h[gr.first + i].begin;
+        for (int i = 0; i < gr.count; ++i) a.begin[i] = e->span[gr.first + i].first;
         return launch_ensemble_sweep(e->fp64, e->ncomp, gr.deg, gr.form, gr.exchange, a, gr.blocks, st);
     };
     auto launch_all = [&](int k, const int *base) -> hipError_t {
@@ -1871,7 +1907,7 @@ int gpe_ensemble_step(gpe_ensemble *e, int nsteps, int graph_sweeps)
         for (int k = 0; k < nsw; ++k) ENSCALL(e, launch_all(k, nullptr));
     }
     ENSCALL(e, hipEventRecord(e->ev1, e->stream));
-    ENSCALL(e, hipEventSynchronize(e->ev1));
+    ENSCALL(e, wait_event(e->ev1));
     float ms = 0.f;
     ENSCALL(e, hipEventElapsedTime(&ms, e->ev0, e->ev1));
     e->last_ms = ms / nsw;
@@ -2032,8 +2068,6 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
             return fail(c, GPE_ENOMEM, "autotune scratch does not fit");
         HIPCALL(c, hipMemcpyAsync(trial.s0, c->level[0], lbytes, hipMemcpyDeviceToDevice, c->stream));
         HIPCALL(c, hipMemcpyAsync(trial.s1, c->level[1], lbytes, hipMemcpyDeviceToDevice, c->stream));
-        int rc = upload_fields(c, c->sweeps, 1);
-        if (rc) return rc;
         // tile heights: powers of two, and multiples of 3, 5, 6 and 7 rows, which are
         // candidates only where their row groups are not powers of two; and the whole plane
         // (one tile: each XCD a range of planes that share their y neighbours in its L2;
@@ -2053,7 +2087,7 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
                 void *cur = trial.s0, *nxt = trial.s1;
                 for (int k = 0; k < trial_sweeps + 2; ++k) {
                     if (k == 2) HIPCALL(c, hipEventRecord(c->ev0, c->stream));
-                    SweepArgs a = sweep_args(c, 0, cur, nxt, 2.0 * sweep_dt(c));
+                    SweepArgs a = sweep_args(c, time_of(c, 0), cur, nxt, 2.0 * sweep_dt(c));
                     a.order = k & 1;
                     hipError_t e = launch_sweep(c->fp64, c->cfg.ncomp, MODE_UPDATE, a, c->stream);
                     if (e != hipSuccess) return hip_fail(c, e, "autotune sweep");

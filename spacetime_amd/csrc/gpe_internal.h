@@ -144,8 +144,8 @@ struct SweepArgs {
     const void *cur;          // level read by the stencil (psi_k)
     void *next;               // level written (psi_{k-1} -> psi_{k+1})
     const void *prev;         // update: psi_{k-1} read from here instead of next (may be null)
-    const FieldRec *fields;   // field of sweep k at fields[k]
-    int sweep;                // index into fields
+    FieldRec field;           // field and time of the sweep (a single launch)
+    const FieldRec *fields;   // batched launches: field of sweep k at fields[k]
     int order;                // 1: the workgroups take their tiles in reverse order (sweep_order)
     int quad, loss;           // quadratic Zeeman / three-body loss active
     double coef;              // update: next += coef * (-i) H cur ; ITP: dt

@@ -80,7 +80,7 @@ __device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const 
 // ROWS: the wave's lanes lie in a group of g.rows consecutive y rows of one (z, v), as in
 // sweep_body_pair: y0 is the group's first row and a lane's offsets are from its line.
 template <typename R, int C, int DEG, int MODE, bool ROWS, int NIN>
-__device__ __forceinline__ void sweep_body_single(const SweepArgs &a, int sweep, int b, int nb)
+__device__ __forceinline__ void sweep_body_single(const SweepArgs &a, const FieldRec &fr, int b, int nb)
 {
     using V2 = vec2_t<R>;
     const Geometry &g = a.g;
@@ -177,7 +177,6 @@ __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, int sweep,
         }
         const R wsum = table_wsum<R>(a.tb)[v];
         const Physics &ph = a.ph;
-        const FieldRec &fr = a.fields[sweep];
         const LocalConsts<R> k = local_consts<R>(ph, fr);
         R hr[C], hi[C];
         R sc = (R)1;
@@ -262,7 +261,7 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
 typedef float f2n __attribute__((ext_vector_type(2)));
 
 template <int C, int DEG, int MODE, bool ROWS, int NIN>
-__device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, int b, int nb)
+__device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, const FieldRec &fr, int b, int nb)
 {
     const Geometry &g = a.g;
     int x0, v, y0, z, r = 0;
@@ -465,7 +464,6 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
         if constexpr (MODE == MODE_ITP) sc = (float)(*a.scale_in);
         const Physics &ph = a.ph;
         const PhysicsF &pf = ph.f;
-        const FieldRec &fr = a.fields[sweep];
         const float sig = fr.fsigma;        // expanding grid: lengths x sigma
         const float ksc = sc * fr.fksc;     // Laplacian / sigma^2
         const float *pos = a.tb.pos32 + 3 * v;
@@ -555,20 +553,20 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, int sweep, i
 
 // X: the lane form (lane_form).
 template <typename R, int C, int DEG, int MODE, int X, int NIN = 0>
-__device__ __forceinline__ void sweep_body(const SweepArgs &a, int sweep, int b, int nb)
+__device__ __forceinline__ void sweep_body(const SweepArgs &a, const FieldRec &fr, int b, int nb)
 {
     if constexpr (X == 3)
-        sweep_body_pair<C, DEG, MODE, true, NIN>(a, sweep, b, nb);
+        sweep_body_pair<C, DEG, MODE, true, NIN>(a, fr, b, nb);
     else if constexpr (X == 2)
-        sweep_body_pair<C, DEG, MODE, false, NIN>(a, sweep, b, nb);
+        sweep_body_pair<C, DEG, MODE, false, NIN>(a, fr, b, nb);
     else
-        sweep_body_single<R, C, DEG, MODE, X == 4, NIN>(a, sweep, b, nb);
+        sweep_body_single<R, C, DEG, MODE, X == 4, NIN>(a, fr, b, nb);
 }
 
 template <typename R, int C, int DEG, int MODE, int X, int NIN>
 __global__ __launch_bounds__(256) void k_sweep(SweepArgs a)
 {
-    sweep_body<R, C, DEG, MODE, X, NIN>(a, a.sweep, sweep_order(a.g, blockIdx.x, gridDim.x, a.order), gridDim.x);
+    sweep_body<R, C, DEG, MODE, X, NIN>(a, a.field, sweep_order(a.g, blockIdx.x, gridDim.x, a.order), gridDim.x);
 }
 
 // One leapfrog sweep of every member of an ensemble group in a single launch (a group: the
@@ -595,7 +593,7 @@ __global__ __launch_bounds__(256) void k_ensemble_sweep(EnsembleArgs e)
     if (local >= m.blocks) return;  // padding workgroup (uniform)
     const SweepArgs &a = m.args[e.parity];
     const int sweep = e.sweep + (e.sweep_base ? *e.sweep_base : 0);
-    sweep_body<R, C, DEG, MODE_UPDATE, X, NIN>(a, sweep, local, m.blocks);
+    sweep_body<R, C, DEG, MODE_UPDATE, X, NIN>(a, a.fields[sweep], local, m.blocks);
 }
 
 __global__ void k_advance_base(int *base, int by)
@@ -1392,13 +1390,15 @@ template <typename R, int C, int DEG, int X, int NIN>
 static hipError_t sweep_mode_n(int mode, const SweepArgs &a, hipStream_t s)
 {
     dim3 grid(a.g.blocks), block(256);
+    void (*k)(SweepArgs) = nullptr;
     switch (mode) {
-    case MODE_UPDATE: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_UPDATE, X, NIN>), grid, block, 0, s, a); break;
-    case MODE_EULER: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_EULER, X, NIN>), grid, block, 0, s, a); break;
-    case MODE_ITP: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_ITP, X, NIN>), grid, block, 0, s, a); break;
-    case MODE_HPSI: hipLaunchKernelGGL((k_sweep<R, C, DEG, MODE_HPSI, X, NIN>), grid, block, 0, s, a); break;
+    case MODE_UPDATE: k = k_sweep<R, C, DEG, MODE_UPDATE, X, NIN>; break;
+    case MODE_EULER: k = k_sweep<R, C, DEG, MODE_EULER, X, NIN>; break;
+    case MODE_ITP: k = k_sweep<R, C, DEG, MODE_ITP, X, NIN>; break;
+    case MODE_HPSI: k = k_sweep<R, C, DEG, MODE_HPSI, X, NIN>; break;
     default: return hipErrorInvalidValue;
     }
+    hipLaunchKernelGGL(k, grid, block, 0, s, a);
     return hipGetLastError();
 }
 
