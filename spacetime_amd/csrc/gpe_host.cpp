@@ -366,8 +366,6 @@ FastDiv make_fast_div(unsigned d)
     return f;
 }
 
-// Segments, tiles, waves and workgroups of a traversal from nx, ny, nz, V, ty and xpl.
-// Wave indices must stay below 2^31 (the decode's divisions).
 // Lanes of a traversal's waves that carry values: rows * pairs pair slots in whole waves.
 static double lane_use(int rows, int pairs)
 {
@@ -375,7 +373,6 @@ static double lane_use(int rows, int pairs)
     return (double)slots / (64.0 * ((slots + 63) / 64));
 }
 
-//
 // pack (FP64 sweeps, one x per lane): the rows of a tile are one group where one row per wave leaves
 // lanes idle that packed rows would fill.  Where lines are whole 128-byte lines, from 5% of the
 // lanes; otherwise a wave then starts inside cache lines that its neighbour also touches, which
@@ -392,6 +389,8 @@ bool pack_rows(const Geometry &g)
     return g.lx % 8 == 0 || one < 0.5 || waves <= 16384;
 }
 
+// Segments, tiles, waves and workgroups of a traversal from nx, ny, nz, V, ty and xpl.
+// Wave indices must stay below 2^31 (the decode's divisions).
 bool finish_geometry(Geometry &g, bool pack = false)
 {
     g.ty = g.ty < g.ny ? g.ty : g.ny;
@@ -1006,19 +1005,28 @@ int gpe_itp(gpe_ctx *c, int nsteps, double dt_itp)
 {
     if (!c) return GPE_EINVAL;
     if (nsteps < 0 || !(dt_itp > 0.0)) return fail(c, GPE_EINVAL, "bad ITP arguments");
-    double *norm = c->d_scalars + 0;
     double *scale[2] = {c->d_scalars + 1, c->d_scalars + 2};
     // initial scale from the norm of level 0
-    hipError_t e = reduce_observables(c, 0, time_of(c, 0));
-    if (e == hipSuccess) e = launch_norm_to_scale(c->d_scalars + 8 + OBS_NORM, 1.0, scale[0], c->stream);
+    NormArgs na;
+    na.g = c->gr;
+    na.psi = c->level[0];
+    na.dv = c->d_dv;
+    na.segs = c->gr_segs;
+    na.per = (c->gr.blocks + c->red_blocks - 1) / c->red_blocks;
+    na.blocks = ((c->gr.blocks + na.per - 1) / na.per + 7) / 8 * 8;
+    na.partials = c->d_partials;
+    hipError_t e = launch_norm(c->fp64, c->cfg.ncomp, na, c->stream);
+    if (e == hipSuccess) e = launch_norm_scale(c->d_partials, na.blocks, 1.0, scale[0], c->d_red, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "ITP initial norm");
+    SweepArgs a = sweep_args(c, time_of(c, 0), nullptr, nullptr, dt_itp);
     for (int i = 0; i < nsteps; ++i) {
-        SweepArgs a = sweep_args(c, time_of(c, 0), c->level[0], c->level[1], dt_itp);
+        a.cur = c->level[0];
+        a.next = c->level[1];
         a.scale_in = scale[i & 1];
         a.order = i & 1;
         e = launch_sweep(c->fp64, c->cfg.ncomp, MODE_ITP, a, c->stream);
-        if (e == hipSuccess) e = launch_finalize(c->d_partials, c->gs.blocks, 1, -1, norm, c->d_red, c->stream);
-        if (e == hipSuccess) e = launch_norm_to_scale(norm, 1.0, scale[(i + 1) & 1], c->stream);
+        if (e == hipSuccess)
+            e = launch_norm_scale(c->d_partials, c->gs.blocks, 1.0, scale[(i + 1) & 1], c->d_red, c->stream);
         if (e != hipSuccess) return hip_fail(c, e, "ITP step");
         std::swap(c->level[0], c->level[1]);
     }

@@ -187,6 +187,15 @@ struct ObsArgs {
     double *partials;         // OBS_COUNT per workgroup
 };
 
+// The norm of a level over the same traversal.
+struct NormArgs {
+    Geometry g;
+    const void *psi;
+    const double *dv;         // Tables::dv
+    int segs, blocks, per;    // as in ObsArgs
+    double *partials;         // one per workgroup
+};
+
 // Most workgroups of a reduction whose waves keep their sums over many unknowns: 8 a CU.
 constexpr int RED_BLOCKS_MAX = 2048;
 
@@ -304,8 +313,13 @@ hipError_t launch_finalize(const double *partials, int n, int width, int maxcol,
 // unless it is null
 hipError_t launch_finalize_few(const double *partials, int n, int width, int maxcol, double *out, double *host,
                                hipStream_t s);
-// out = sqrt(target / in[0])
-hipError_t launch_norm_to_scale(const double *in, double target, double *out, hipStream_t s);
+hipError_t launch_norm(int fp64, int ncomp, const NormArgs &a, hipStream_t s);
+// out = sqrt(target / sum of n partials); scratch as in launch_finalize
+hipError_t launch_norm_scale(const double *partials, int n, double target, double *out, double *scratch,
+                             hipStream_t s);
+// Partials that one workgroup sums itself (64 a thread, about 7 us; a first stage over 256
+// workgroups costs a launch more).
+constexpr int NORM_ONE_MAX = 65536;
 // level *= factor (device scalar if dfactor != nullptr)
 hipError_t launch_scale(int fp64, void *psi, long long nelem, double factor, const double *dfactor,
                         hipStream_t s);

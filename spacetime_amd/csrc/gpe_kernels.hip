@@ -855,6 +855,44 @@ __global__ __launch_bounds__(256) void k_observables(ObsArgs a)
     }
 }
 
+// FP64 norm of a level (OBS_NORM alone) over the same traversal: one read of the level.
+template <typename R, int C>
+__global__ __launch_bounds__(256) void k_norm(NormArgs a)
+{
+    using V2 = vec2_t<R>;
+    const Geometry &g = a.g;
+    const unsigned wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned each = gridDim.x >> 3;
+    const unsigned first = ((blockIdx.x & 7u) * each * (unsigned)a.per + (blockIdx.x >> 3)) * 4u + wid;
+    const long long cstride = comp_stride(g);
+    double sum = 0.0;
+    for (int j = 0; j < a.per; ++j) {
+        RedCoord rc;
+        if (!decode_reduce(g, a.segs, first + 4u * each * (unsigned)j, rc)) break;
+        const V2 *base = (const V2 *)a.psi + line_index(g, 0, rc.z, rc.y0, rc.v);
+        const unsigned slots = (unsigned)rc.nrow * (unsigned)g.nx;
+        const unsigned end = rc.slot0 + 64u * (unsigned)a.segs < slots ? rc.slot0 + 64u * (unsigned)a.segs : slots;
+        double n = 0.0;
+#pragma unroll 4
+        for (unsigned p = rc.slot0 + (threadIdx.x & 63); p < end; p += 64u) {
+            const unsigned r = fast_div(p, g.f_pairs);
+            const int at = (int)r * (int)g.ys + (int)(p - r * (unsigned)g.nx);
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const V2 o = base[c * cstride + at];
+                n += (double)o.x * (double)o.x;
+                n += (double)o.y * (double)o.y;
+            }
+        }
+        sum += n * a.dv[rc.v];
+    }
+    __shared__ double red[4];
+    sum = wave_sum(sum);
+    if ((threadIdx.x & 63) == 0) red[wid] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) a.partials[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
 // Two local reductions over a level, one x per lane:
 //   max over unknowns of the local Hamiltonian bound (Spin1GpeBCC.cu:144-189): with
 //   p = V(r) + c0 n and B = B(r, t) + c1 <F> (<F> = psi^dag f psi, not divided by n),
@@ -1008,9 +1046,24 @@ __global__ __launch_bounds__(256) void k_sum_tables(const double *partials, int 
     }
 }
 
-__global__ void k_norm_to_scale(const double *in, double target, double *out)
+// out = sqrt(target / sum of the n partial norms), one workgroup: fixed strides and trees.  41472
+// partials (FP64 BCC 96^3) in one launch instead of a two-stage sum and a scale kernel.
+__global__ __launch_bounds__(1024) void k_norm_scale(const double *partials, int n, double target, double *out)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) out[0] = sqrt(target / in[0]);
+    __shared__ double red[16];
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    int i = threadIdx.x;
+    for (; i + 3 * 1024 < n; i += 4 * 1024)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[k] += partials[i + k * 1024];
+    for (int k = 0; i < n; i += 1024, ++k) acc[k] += partials[i];
+    const double w = wave_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const double sum = wave_sum(threadIdx.x < 16 ? red[threadIdx.x] : 0.0);
+        if (threadIdx.x == 0) out[0] = sqrt(target / sum);
+    }
 }
 
 template <typename R>
@@ -1606,9 +1659,29 @@ hipError_t launch_sum_tables(const double *partials, int nslot, int n, int width
     return hipGetLastError();
 }
 
-hipError_t launch_norm_to_scale(const double *in, double target, double *out, hipStream_t s)
+hipError_t launch_norm_scale(const double *partials, int n, double target, double *out, double *scratch, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_norm_to_scale, dim3(1), dim3(64), 0, s, in, target, out);
+    if (n <= 0) return hipErrorInvalidValue;
+    if (n > NORM_ONE_MAX) {
+        const int chunk = (n + FIN_BLOCKS - 1) / FIN_BLOCKS, nb = (n + chunk - 1) / chunk;
+        hipLaunchKernelGGL(k_finalize_stage, dim3(nb), dim3(256), 0, s, partials, n, 1, -1, chunk, scratch);
+        partials = scratch;
+        n = nb;
+    }
+    hipLaunchKernelGGL(k_norm_scale, dim3(1), dim3(1024), 0, s, partials, n, target, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_norm(int fp64, int ncomp, const NormArgs &a, hipStream_t s)
+{
+    void (*k)(NormArgs) = nullptr;
+    switch (ncomp) {
+    case 1: k = fp64 ? k_norm<double, 1> : k_norm<float, 1>; break;
+    case 3: k = fp64 ? k_norm<double, 3> : k_norm<float, 3>; break;
+    case 5: k = fp64 ? k_norm<double, 5> : k_norm<float, 5>; break;
+    default: return hipErrorInvalidValue;
+    }
+    hipLaunchKernelGGL(k, dim3(a.blocks), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
