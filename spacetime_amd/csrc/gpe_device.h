@@ -81,13 +81,19 @@ __device__ __forceinline__ const_ptr<T> fresh(const T *p)
     return q;
 }
 
-// A member of the kernel's argument (its only one, a struct) at `offset`.
+// A member of the kernel's argument (its only one, a struct) at `offset`; fresh_args as fresh().
+template <typename T>
+__device__ __forceinline__ const_ptr<T> args_at(unsigned offset)
+{
+    return (const_ptr<T>)((const_ptr<char>)__builtin_amdgcn_kernarg_segment_ptr() + offset);
+}
+
 template <typename T>
 __device__ __forceinline__ const_ptr<T> fresh_args(unsigned offset)
 {
-    const_ptr<char> q = (const_ptr<char>)__builtin_amdgcn_kernarg_segment_ptr() + offset;
+    const_ptr<T> q = args_at<T>(offset);
     asm volatile("" : "+s"(q));
-    return (const_ptr<T>)q;
+    return q;
 }
 
 struct WaveCoord {
@@ -169,7 +175,9 @@ __device__ __forceinline__ RowCoord decode_rows(const Geometry &g, int b, int nb
     const unsigned q3 = fast_div(q2, g.f_nz);
     rc.z = (int)(q2 - q3 * (unsigned)g.nz);
     rc.y0 = (int)q3 * g.ty + yg * g.rows;
-    rc.valid = ((long long)w < g.waves) && (rc.y0 < g.ny);
+    // a wave whose first slot is past the group's rows in the box has nothing to do
+    const int left = g.ny - rc.y0;
+    rc.valid = ((long long)w < g.waves) && xseg * 64 < left * g.pairs;
     const unsigned p = (unsigned)(xseg * 64) + (threadIdx.x & 63);
     const unsigned r = fast_div(p, g.f_pairs);
     rc.r = (int)r;
@@ -208,11 +216,10 @@ __device__ __forceinline__ LaneCoord lane_coord(const Geometry &g, int b, int nb
         lc.act = rc.r < nrow;
         lc.y = rc.y0 + rr;
         lc.at = rr * (int)g.ys + rc.x;
-        // a lane's row grows with its lane number: lanes 0 and 63 bound the wave's rows; a wave
-        // whose first lane is past the group has nothing to do
+        // a lane's row grows with its lane number: lanes 0 and 63 bound the wave's rows
         lc.ylo = rc.y0 + __builtin_amdgcn_readfirstlane(rr);
         lc.yhi = rc.y0 + __builtin_amdgcn_readlane(rr, 63);
-        lc.valid = rc.valid && __builtin_amdgcn_readfirstlane(rc.r) < nrow;
+        lc.valid = rc.valid;
     } else {
         const WaveCoord wc = decode(g, b, nb);
         lc.x = wc.x, lc.v = wc.v, lc.y = lc.y0 = lc.ylo = lc.yhi = wc.y, lc.z = wc.z, lc.valid = wc.valid;

@@ -440,6 +440,37 @@ bool finish_geometry(Geometry &g, bool pack = false)
     return true;
 }
 
+// Tile height of an untuned sweep: 8 rows, or the lowest height up to 32 that fills the most lanes
+// where that is a tenth more.  Lines of a few dozen values fill waves only in some heights, and a
+// low last tile leaves whole waves empty on the XCDs that have it (20 rows of A15's 10 pairs: 52%
+// of the lanes in tiles of 8, 78% in one tile; FCC 19^3 49% and 99%).  Taller tiles have to keep
+// a plane's rows in an XCD's L2 with room for its neighbours (TILE_BYTES: C15 57^3 spin-2 588 us
+// at 8 rows, 700 at 24), and large cells' tiles to start on 128-byte boundaries (A15 41^3 49 -> 51).
+constexpr double TILE_BYTES = 2.6e6;
+
+int default_tile(const Geometry &g0, int elem_bytes, bool pack)
+{
+    const auto use = [&](int ty) {
+        Geometry g = g0;
+        g.ty = ty;
+        if (!finish_geometry(g, pack)) return 0.0;
+        const int slots = g.xpl == 2 ? g.pairs : g.nx;
+        return (double)g.ny * slots / (64.0 * g.ntile * g.tyr * g.nseg);
+    };
+    const int lo = std::min(8, g0.ny), hi = std::min(32, g0.ny);
+    int ty = lo;
+    double best = use(lo) * 1.1;
+    for (int t = lo + 1; t <= hi; ++t) {
+        if ((double)t * g0.lx * g0.V * g0.C * elem_bytes > TILE_BYTES) break;
+        if (g0.V > 12 && t < g0.ny && (t * g0.lx) % 16 != 0) continue;
+        if (use(t) > best + 1e-9) {
+            best = use(t);
+            ty = t;
+        }
+    }
+    return ty;
+}
+
 // Traversal of a reduction over a level: one x per lane, the rows of a tile as one group whose
 // slots (row, x) fill whole waves.  The tile is the lowest of 8-32 rows whose waves carry within
 // 3% of the most values (57-value lines, 57 rows: 19 rows 99% against 8 rows 87%, and one row
@@ -662,6 +693,7 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     g = base_geometry(*cfg);
     c->gs = g;
     c->gs.xpl = default_xpl(c->fp64, g.deg, cfg->ncomp, cfg->nx);
+    c->gs.ty = default_tile(c->gs, c->elem_bytes, c->fp64);
     if (!finish_geometry(g) || !finish_geometry(c->gs, c->fp64)) {
         delete c;
         return GPE_EINVAL;
@@ -1751,7 +1783,7 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
     e->m.assign(members, members + n);
     std::stable_sort(e->m.begin(), e->m.end(), [](const gpe_ctx *a, const gpe_ctx *b) {
         const auto key = [](const Geometry &g) {
-            return std::make_tuple(g.deg, lane_form(g.xpl, g.rows), g.exchange);
+            return std::make_tuple(g.deg, lane_form(g.xpl, g.rows), g.blocks >= ENS_SOLO_BLOCKS);
         };
         return key(a->gs) < key(b->gs);
     });
@@ -1764,10 +1796,11 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
         const gpe_ctx *c = e->m[i];
         const int form = lane_form(c->gs.xpl, c->gs.rows);
         const bool solo = c->gs.blocks >= ENS_SOLO_BLOCKS;
+        const int exchange = solo ? c->gs.exchange : 0;  // a launch shared with other lattices does without
         if (i == 0 || solo || prev_solo || c->gs.deg != e->groups.back().deg || form != e->groups.back().form ||
-            c->gs.exchange != e->groups.back().exchange ||
+            exchange != e->groups.back().exchange ||
             e->groups.back().count == ENS_GROUP_MAX) {
-            e->groups.push_back(EnsembleGroup{c->gs.deg, form, c->gs.exchange, i, 0, 0});
+            e->groups.push_back(EnsembleGroup{c->gs.deg, form, exchange, i, 0, 0});
             begin = 0;
         }
         prev_solo = solo;

@@ -119,20 +119,22 @@ struct Physics {
     double p0[3];
     double trap[3];        // trap frequencies
     double trap2[3];       // squared trap frequencies
-    double trap_offset, trap_off_time;
+    double trap_offset;
     double c0, c1, c2, alpha, quad_sign, q;
     double center[3];
+    double trap_off_time;
     PhysicsF f;            // the same in FP32
 };
 
-// Field and time of one sweep (computed on the host from the ramp).
+// Field and time of one sweep (computed on the host from the ramp); what one component reads
+// comes first.
 struct FieldRec {
-    double bq, bb[3];
-    double bqq, bbq[3];
     double t;
     double sigma;         // block-scale factor of the expanding grid (1: static)
-    // FP32 copies for the FP32 sweep: bq, bb[3], bqq, bbq[3], sigma, 1 / sigma^2
-    float fbq, fbb[3], fbqq, fbbq[3], fsigma, fksc, pad[2];
+    // FP32 copies for the FP32 sweep: sigma, 1 / sigma^2, bq, bb[3], bqq, bbq[3]
+    float fsigma, fksc, fbq, fbb[3], fbqq, fbbq[3];
+    double bq, bb[3];
+    double bqq, bbq[3];
 };
 
 enum Mode { MODE_UPDATE = 0, MODE_EULER = 1, MODE_ITP = 2, MODE_HPSI = 3 };
@@ -144,13 +146,13 @@ struct SweepArgs {
     const void *cur;          // level read by the stencil (psi_k)
     void *next;               // level written (psi_{k-1} -> psi_{k+1})
     const void *prev;         // update: psi_{k-1} read from here instead of next (may be null)
-    FieldRec field;           // field and time of the sweep (a single launch)
     const FieldRec *fields;   // batched launches: field of sweep k at fields[k]
     int order;                // 1: the workgroups take their tiles in reverse order (sweep_order)
     int quad, loss;           // quadratic Zeeman / three-body loss active
     double coef;              // update: next += coef * (-i) H cur ; ITP: dt
     const double *scale_in;   // ITP: scale applied to cur before H (device scalar)
     double *partials;         // ITP: one FP64 partial norm per workgroup
+    FieldRec field;           // field and time of the sweep (a single launch), beside coef for its head
 };
 
 // Observables partial sums per workgroup.

@@ -28,7 +28,7 @@ struct LocalConsts {
 };
 
 template <typename R>
-__device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const FieldRec &fr)
+__device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const const_ptr<FieldRec> fr)
 {
     LocalConsts<R> k;
     if constexpr (std::is_same<R, float>::value) {
@@ -38,8 +38,8 @@ __device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const 
             k.p0[i] = f.p0[i];
             k.trap2[i] = f.trap2[i];
             k.center[i] = f.center[i];
-            k.bb[i] = fr.fbb[i];
-            k.bbq[i] = fr.fbbq[i];
+            k.bb[i] = fr->fbb[i];
+            k.bbq[i] = fr->fbbq[i];
         }
         k.trap_offset = f.trap_offset;
         k.c0 = f.c0;
@@ -48,18 +48,18 @@ __device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const 
         k.alpha = f.alpha;
         k.quad_sign = f.quad_sign;
         k.q = f.q;
-        k.bq = fr.fbq;
-        k.bqq = fr.fbqq;
-        k.sigma = fr.fsigma;
-        k.ksc = fr.fksc;
+        k.bq = fr->fbq;
+        k.bqq = fr->fbqq;
+        k.sigma = fr->fsigma;
+        k.ksc = fr->fksc;
     } else {
         for (int i = 0; i < 3; ++i) {
             k.cell[i] = ph.cell[i];
             k.p0[i] = ph.p0[i];
             k.trap2[i] = ph.trap2[i];
             k.center[i] = ph.center[i];
-            k.bb[i] = fr.bb[i];
-            k.bbq[i] = fr.bbq[i];
+            k.bb[i] = fr->bb[i];
+            k.bbq[i] = fr->bbq[i];
         }
         k.trap_offset = ph.trap_offset;
         k.c0 = ph.c0;
@@ -68,10 +68,10 @@ __device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const 
         k.alpha = ph.alpha;
         k.quad_sign = ph.quad_sign;
         k.q = ph.q;
-        k.bq = fr.bq;
-        k.bqq = fr.bqq;
-        k.sigma = fr.sigma;
-        k.ksc = 1.0 / (fr.sigma * fr.sigma);
+        k.bq = fr->bq;
+        k.bqq = fr->bqq;
+        k.sigma = fr->sigma;
+        k.ksc = 1.0 / (fr->sigma * fr->sigma);
     }
     return k;
 }
@@ -79,8 +79,8 @@ __device__ __forceinline__ LocalConsts<R> local_consts(const Physics &ph, const 
 // One x value per lane (FP64, and FP32 where the neighbour pairs would not fit).
 // ROWS: the wave's lanes lie in a group of g.rows consecutive y rows of one (z, v), as in
 // sweep_body_pair: y0 is the group's first row and a lane's offsets are from its line.
-template <typename R, int C, int DEG, int MODE, bool ROWS, int NIN>
-__device__ __forceinline__ void sweep_body_single(const SweepArgs &a, const FieldRec &fr, int b, int nb)
+template <typename R, int C, int DEG, int MODE, bool ROWS, int NIN, typename Field>
+__device__ __forceinline__ void sweep_body_single(const SweepArgs &a, const Field &field, int b, int nb)
 {
     using V2 = vec2_t<R>;
     const Geometry &g = a.g;
@@ -177,6 +177,7 @@ __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, const Fiel
         }
         const R wsum = table_wsum<R>(a.tb)[v];
         const Physics &ph = a.ph;
+        const const_ptr<FieldRec> fr = field();
         const LocalConsts<R> k = local_consts<R>(ph, fr);
         R hr[C], hi[C];
         R sc = (R)1;
@@ -196,7 +197,7 @@ __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, const Fiel
         const R ry = k.p0[1] + sig * (k.cell[1] * (R)y + pos[1]);
         const R rz = k.p0[2] + sig * (k.cell[2] * (R)z + pos[2]);
         R vtrap = 0;
-        if (fr.t < ph.trap_off_time)
+        if (fr->t < ph.trap_off_time)
             vtrap = (R)0.5 * (k.trap2[0] * rx * rx + k.trap2[1] * ry * ry + k.trap2[2] * rz * rz) + k.trap_offset;
         R Bx = 0, By = 0, Bz = 0, Qx = 0, Qy = 0, Qz = 0;
         if constexpr (C > 1) {
@@ -260,8 +261,8 @@ typedef float f4a __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
 typedef float f2n __attribute__((ext_vector_type(2)));
 
-template <int C, int DEG, int MODE, bool ROWS, int NIN>
-__device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, const FieldRec &fr, int b, int nb)
+template <int C, int DEG, int MODE, bool ROWS, int NIN, typename Field>
+__device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, const Field &field, int b, int nb)
 {
     const Geometry &g = a.g;
     int x0, v, y0, z, r = 0;
@@ -464,12 +465,13 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, const FieldR
         if constexpr (MODE == MODE_ITP) sc = (float)(*a.scale_in);
         const Physics &ph = a.ph;
         const PhysicsF &pf = ph.f;
-        const float sig = fr.fsigma;        // expanding grid: lengths x sigma
-        const float ksc = sc * fr.fksc;     // Laplacian / sigma^2
+        const const_ptr<FieldRec> fr = field();
+        const float sig = fr->fsigma;        // expanding grid: lengths x sigma
+        const float ksc = sc * fr->fksc;     // Laplacian / sigma^2
         const float *pos = a.tb.pos32 + 3 * v;
         const float ry = pf.p0[1] + sig * (pf.cell[1] * (float)y + pos[1]);
         const float rz = pf.p0[2] + sig * (pf.cell[2] * (float)z + pos[2]);
-        const bool trap_on = fr.t < ph.trap_off_time;
+        const bool trap_on = fr->t < ph.trap_off_time;
         const float coef = (float)a.coef;
         float2 out[2][C];
 #pragma unroll
@@ -490,12 +492,12 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, const FieldR
             float Bx = 0, By = 0, Bz = 0, Qx = 0, Qy = 0, Qz = 0;
             if constexpr (C > 1) {
                 const float dxr = rx - pf.center[0], dyr = ry - pf.center[1], dzr = rz - pf.center[2];
-                Bx = fr.fbq * dxr + fr.fbb[0];
-                By = fr.fbq * dyr + fr.fbb[1];
-                Bz = -2.f * fr.fbq * dzr + fr.fbb[2];
-                Qx = fr.fbqq * dxr + fr.fbbq[0];
-                Qy = fr.fbqq * dyr + fr.fbbq[1];
-                Qz = -2.f * fr.fbqq * dzr + fr.fbbq[2];
+                Bx = fr->fbq * dxr + fr->fbb[0];
+                By = fr->fbq * dyr + fr->fbb[1];
+                Bz = -2.f * fr->fbq * dzr + fr->fbb[2];
+                Qx = fr->fbqq * dxr + fr->fbbq[0];
+                Qy = fr->fbqq * dyr + fr->fbbq[1];
+                Qz = -2.f * fr->fbqq * dzr + fr->fbbq[2];
             }
             add_local_h<float, C>(pr[e], pi[e], vtrap, Bx, By, Bz, Qx, Qy, Qz, pf.c0, pf.c1, pf.c2, pf.alpha,
                                   pf.quad_sign, pf.q, a.quad, a.loss, hr, hi);
@@ -552,21 +554,29 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, const FieldR
 }
 
 // X: the lane form (lane_form).
-template <typename R, int C, int DEG, int MODE, int X, int NIN = 0>
-__device__ __forceinline__ void sweep_body(const SweepArgs &a, const FieldRec &fr, int b, int nb)
+// field: gives the sweep's FieldRec, loaded where it is used (fresh).
+template <typename R, int C, int DEG, int MODE, int X, int NIN, typename Field>
+__device__ __forceinline__ void sweep_body(const SweepArgs &a, const Field &field, int b, int nb)
 {
     if constexpr (X == 3)
-        sweep_body_pair<C, DEG, MODE, true, NIN>(a, fr, b, nb);
+        sweep_body_pair<C, DEG, MODE, true, NIN>(a, field, b, nb);
     else if constexpr (X == 2)
-        sweep_body_pair<C, DEG, MODE, false, NIN>(a, fr, b, nb);
+        sweep_body_pair<C, DEG, MODE, false, NIN>(a, field, b, nb);
     else
-        sweep_body_single<R, C, DEG, MODE, X == 4, NIN>(a, fr, b, nb);
+        sweep_body_single<R, C, DEG, MODE, X == 4, NIN>(a, field, b, nb);
 }
 
 template <typename R, int C, int DEG, int MODE, int X, int NIN>
 __global__ __launch_bounds__(256) void k_sweep(SweepArgs a)
 {
-    sweep_body<R, C, DEG, MODE, X, NIN>(a, a.field, sweep_order(a.g, blockIdx.x, gridDim.x, a.order), gridDim.x);
+    // spinors load it after the neighbours (fewer scalar registers held: FCC 30^3 spin-1 8.3 -> 7.9 us a
+    // sweep); one component needs its first 24 bytes only, at once, from a line of the arguments that
+    // it reads anyway (BCC 30^3 4.4 -> 4.2, FCC 24x18x23 5.2 -> 5.0 against a line of its own)
+    const auto field = []() {
+        constexpr unsigned at = offsetof(SweepArgs, field);
+        return C > 1 ? fresh_args<FieldRec>(at) : args_at<FieldRec>(at);
+    };
+    sweep_body<R, C, DEG, MODE, X, NIN>(a, field, sweep_order(a.g, blockIdx.x, gridDim.x, a.order), gridDim.x);
 }
 
 // One leapfrog sweep of every member of an ensemble group in a single launch (a group: the
@@ -593,7 +603,8 @@ __global__ __launch_bounds__(256) void k_ensemble_sweep(EnsembleArgs e)
     if (local >= m.blocks) return;  // padding workgroup (uniform)
     const SweepArgs &a = m.args[e.parity];
     const int sweep = e.sweep + (e.sweep_base ? *e.sweep_base : 0);
-    sweep_body<R, C, DEG, MODE_UPDATE, X, NIN>(a, a.fields[sweep], local, m.blocks);
+    const auto field = [&]() { return (const_ptr<FieldRec>)(unsigned long long)(a.fields + sweep); };
+    sweep_body<R, C, DEG, MODE_UPDATE, X, NIN>(a, field, local, m.blocks);
 }
 
 __global__ void k_advance_base(int *base, int by)
