@@ -1416,33 +1416,83 @@ hipError_t launch_stream(int kind, const void *a, void *b, long long n16, hipStr
     return hipGetLastError();
 }
 
-// ABI index (c, z, y, x, v) <-> device index (c, z, y, v, x)
+// ABI order (c, z, y, x, v) in FP64 <-> device layout.  A workgroup turns a run of 2^lg consecutive
+// cells of one component round in LDS: the ABI side is one contiguous run, a device line is read or
+// written 2^lg values at a time.  With one ABI value a thread, whose device address is a line away
+// from its neighbour's, the cache bound it; now bytes do (spin-1 128^3 FP32 out 425 -> 312 us, 5.8
+// TB/s, in 450 -> 325; C15 57^3 spin-2 1290 -> 527, 5.7 TB/s, and 1240 -> 840, where 32 cells are short
+// pieces of unaligned lines; BCC 96^3 FP64 195 -> 181 and 240 -> 169).  A cell takes an odd number of
+// places in LDS, so lanes that hold one unknown of consecutive cells meet no bank twice.
+constexpr int PACK_BATCH = 4;  // values a thread has in flight
+
 template <typename R, bool PACK>
-__global__ __launch_bounds__(256) void k_pack(Geometry g, const int *place, int ncomp, const double2 *abi_in, double2 *abi_out,
-                                              const vec2_t<R> *dev_in, vec2_t<R> *dev_out)
+__global__ __launch_bounds__(256) void k_pack(Geometry g, const int *__restrict__ abi_of, int lg,
+                                              const double2 *__restrict__ abi_in, double2 *__restrict__ abi_out,
+                                              const vec2_t<R> *__restrict__ dev_in, vec2_t<R> *__restrict__ dev_out)
 {
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    const long long total = (long long)ncomp * g.nz * g.ny * g.nx * g.V;
-    if (i >= total) return;
-    long long r = i;
-    const int v = place[(int)(r % g.V)];
-    r /= g.V;
-    const int x = (int)(r % g.nx);
-    r /= g.nx;
-    const int y = (int)(r % g.ny);
-    r /= g.ny;
-    const int z = (int)(r % g.nz);
-    const int c = (int)(r / g.nz);
-    const long long d = line_index(g, c, z, y, v) + x;
+    using V2 = vec2_t<R>;
+    extern __shared__ double2 pack_lds[];
+    const int nb = 1 << lg, odd = g.V | 1;
+    V2 *tile = (V2 *)pack_lds;                 // [cell][unknown]
+    int *off = (int *)(tile + nb * odd);       // a cell's device offset in its component and plane z0
+    int *order = off + nb;                     // the ABI's unknown at each device place
+    const long long cells = (long long)g.nz * g.ny * g.nx;
+    const long long q0 = (long long)blockIdx.x << lg;
+    const int n = (int)(cells - q0 < nb ? cells - q0 : nb);
+    const unsigned plane = (unsigned)(g.ny * g.nx);  // < 2^31 (Geometry::zs)
+    const long long z0 = q0 / plane;
+    const unsigned at = (unsigned)(q0 - z0 * plane);
+    const unsigned y0 = at / (unsigned)g.nx, x0 = at - y0 * (unsigned)g.nx;
+    for (int k = threadIdx.x; k < n; k += 256) {
+        const unsigned row = (x0 + k) / (unsigned)g.nx, x = x0 + k - row * (unsigned)g.nx;
+        const unsigned dz = (y0 + row) / (unsigned)g.ny, y = y0 + row - dz * (unsigned)g.ny;
+        off[k] = (int)(dz * (unsigned)g.zs + y * (unsigned)g.ys + x);
+    }
+    for (int p = threadIdx.x; p < g.V; p += 256) order[p] = abi_of[p];
+    __syncthreads();
+    const long long dev0 = z0 * g.zs + (long long)blockIdx.y * g.cs;
+    const long long abi0 = ((long long)blockIdx.y * cells + q0) * g.V;
+    const int vs = (int)g.vs, pad = odd - g.V;
+    const int nabi = n * g.V, ndev = g.V << lg;
     if constexpr (PACK) {
-        const double2 s = abi_in[i];
-        vec2_t<R> o;
-        o.x = (R)s.x;
-        o.y = (R)s.y;
-        dev_out[d] = o;
+        for (int i0 = threadIdx.x; i0 < nabi; i0 += 256 * PACK_BATCH) {
+            double2 s[PACK_BATCH];
+#pragma unroll
+            for (int j = 0; j < PACK_BATCH; ++j)
+                s[j] = nt_load<double>(&abi_in[abi0 + (i0 + 256 * j < nabi ? i0 + 256 * j : 0)]);
+#pragma unroll
+            for (int j = 0; j < PACK_BATCH; ++j) {
+                const int i = i0 + 256 * j;
+                V2 o;
+                o.x = (R)s[j].x;
+                o.y = (R)s[j].y;
+                if (i < nabi) tile[i + pad * (int)fast_div((unsigned)i, g.f_V)] = o;
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < ndev; i += 256) {
+            const int k = i & (nb - 1), p = i >> lg;
+            if (k < n) dev_out[dev0 + off[k] + p * vs] = tile[k * odd + order[p]];
+        }
     } else {
-        const vec2_t<R> s = dev_in[d];
-        abi_out[i] = make_double2((double)s.x, (double)s.y);
+        for (int i0 = threadIdx.x; i0 < ndev; i0 += 256 * PACK_BATCH) {
+            V2 s[PACK_BATCH];
+#pragma unroll
+            for (int j = 0; j < PACK_BATCH; ++j) {
+                const int i = i0 + 256 * j, k = i & (nb - 1), p = i >> lg;
+                s[j] = dev_in[dev0 + (i < ndev && k < n ? off[k] + p * vs : 0)];
+            }
+#pragma unroll
+            for (int j = 0; j < PACK_BATCH; ++j) {
+                const int i = i0 + 256 * j, k = i & (nb - 1), p = i >> lg;
+                if (i < ndev && k < n) tile[k * odd + order[p]] = s[j];
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < nabi; i += 256) {
+            const V2 s = tile[i + pad * (int)fast_div((unsigned)i, g.f_V)];
+            nt_store<double>(make_double2((double)s.x, (double)s.y), &abi_out[abi0 + i]);
+        }
     }
 }
 
@@ -1719,28 +1769,34 @@ hipError_t launch_phase_copy(int fp64, const void *src, void *dst, long long nel
     return hipGetLastError();
 }
 
+// Cells per workgroup: a tile of up to 40 KiB (four workgroups a CU; up to 64 KiB: BCC 96^3 FP64 out
+// 181 -> 256 us; up to 32 KiB: C15 57^3 spin-2 in 840 -> 930), less while that leaves the chip short of
+// workgroups, but 16 cells, 128-byte pieces of a line in FP32, at least.
+template <typename R, bool PACK>
+static hipError_t pack(const Geometry &g, const Tables &tb, int ncomp, const double *abi_in, double *abi_out, const void *dev_in,
+                       void *dev_out, hipStream_t s)
+{
+    const long long cells = (long long)g.nz * g.ny * g.nx;
+    const size_t cell = (size_t)(g.V | 1) * sizeof(vec2_t<R>);
+    int lg = 4;
+    while (lg < 10 && (cell << (lg + 1)) <= 40960 && ncomp * ((cells >> (lg + 1)) + 1) >= 1024) ++lg;
+    const size_t lds = (cell << lg) + (sizeof(int) << lg) + sizeof(int) * (size_t)g.V;
+    const dim3 grid((unsigned)((cells + (1 << lg) - 1) >> lg), (unsigned)ncomp);
+    hipLaunchKernelGGL((k_pack<R, PACK>), grid, dim3(256), lds, s, g, tb.abi, lg, (const double2 *)abi_in, (double2 *)abi_out,
+                       (const vec2_t<R> *)dev_in, (vec2_t<R> *)dev_out);
+    return hipGetLastError();
+}
+
 hipError_t launch_pack(int fp64, const Geometry &g, const Tables &tb, int ncomp, const double *abi, void *dev, hipStream_t s)
 {
-    const long long total = (long long)ncomp * g.nz * g.ny * g.nx * g.V;
-    if (fp64)
-        hipLaunchKernelGGL((k_pack<double, true>), dim3(grid1(total)), dim3(256), 0, s, g, tb.place, ncomp,
-                           (const double2 *)abi, nullptr, nullptr, (double2 *)dev);
-    else
-        hipLaunchKernelGGL((k_pack<float, true>), dim3(grid1(total)), dim3(256), 0, s, g, tb.place, ncomp,
-                           (const double2 *)abi, nullptr, nullptr, (float2 *)dev);
-    return hipGetLastError();
+    return fp64 ? pack<double, true>(g, tb, ncomp, abi, nullptr, nullptr, dev, s)
+                : pack<float, true>(g, tb, ncomp, abi, nullptr, nullptr, dev, s);
 }
 
 hipError_t launch_unpack(int fp64, const Geometry &g, const Tables &tb, int ncomp, const void *dev, double *abi, hipStream_t s)
 {
-    const long long total = (long long)ncomp * g.nz * g.ny * g.nx * g.V;
-    if (fp64)
-        hipLaunchKernelGGL((k_pack<double, false>), dim3(grid1(total)), dim3(256), 0, s, g, tb.place, ncomp, nullptr,
-                           (double2 *)abi, (const double2 *)dev, nullptr);
-    else
-        hipLaunchKernelGGL((k_pack<float, false>), dim3(grid1(total)), dim3(256), 0, s, g, tb.place, ncomp, nullptr,
-                           (double2 *)abi, (const float2 *)dev, nullptr);
-    return hipGetLastError();
+    return fp64 ? pack<double, false>(g, tb, ncomp, nullptr, abi, dev, nullptr, s)
+                : pack<float, false>(g, tb, ncomp, nullptr, abi, dev, nullptr, s);
 }
 
 }  // namespace gpe
