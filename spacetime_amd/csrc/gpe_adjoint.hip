@@ -360,7 +360,7 @@ __device__ __forceinline__ void adjoint_single(const AdjArgs &a, int b, int nb, 
     }
     const FieldRec &fr = a.fields[a.sweep];
     const AdjConsts<R> k = adj_consts<R>(a.ph, fr);
-    const bool trap_on = fr.t < a.ph.trap_off_time;
+    const bool trap_on = fr.trap_on != 0;
     const R *pos = table_pos<R>(a.tb) + 3 * v;
     const R rx = k.p0[0] + (k.cell[0] * (R)x + pos[0]);
     const R ry = k.p0[1] + (k.cell[1] * (R)y + pos[1]);
@@ -571,7 +571,7 @@ __device__ __forceinline__ void adjoint_pair(const AdjArgs &a, int b, int nb, do
     const float wsum = a.tb.wsum32[v];
     const FieldRec &fr = a.fields[a.sweep];
     const AdjConsts<float> k = adj_consts<float>(a.ph, fr);
-    const bool trap_on = fr.t < a.ph.trap_off_time;
+    const bool trap_on = fr.trap_on != 0;
     const float *pos = a.tb.pos32 + 3 * v;
     const float ry = k.p0[1] + (k.cell[1] * (float)y + pos[1]);
     const float rz = k.p0[2] + (k.cell[2] * (float)z + pos[2]);

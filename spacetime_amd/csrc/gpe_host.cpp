@@ -248,6 +248,7 @@ FieldRec field_at(const gpe_ctx *c, double t)
 {
     FieldRec f{};
     f.t = t;
+    f.trap_on = t < c->ph.trap_off_time;
     f.sigma = 1.0;
     if (c->cfg.expansion_rate != 0.0 && t > c->cfg.expansion_start)
         f.sigma = 1.0 + c->cfg.expansion_rate * (t - c->cfg.expansion_start);

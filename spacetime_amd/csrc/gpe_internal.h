@@ -122,17 +122,19 @@ struct Physics {
     double trap_offset;
     double c0, c1, c2, alpha, quad_sign, q;
     double center[3];
-    double trap_off_time;
     PhysicsF f;            // the same in FP32
+    double trap_off_time;  // read on the host (FieldRec::trap_on)
 };
 
 // Field and time of one sweep (computed on the host from the ramp); what one component reads
 // comes first.
 struct FieldRec {
-    double t;
-    double sigma;         // block-scale factor of the expanding grid (1: static)
+    int trap_on;          // t is before the trap's end
     // FP32 copies for the FP32 sweep: sigma, 1 / sigma^2, bq, bb[3], bqq, bbq[3]
-    float fsigma, fksc, fbq, fbb[3], fbqq, fbbq[3];
+    float fsigma, fksc, pad;
+    double sigma;         // block-scale factor of the expanding grid (1: static)
+    float fbq, fbb[3], fbqq, fbbq[3];
+    double t;
     double bq, bb[3];
     double bqq, bbq[3];
 };

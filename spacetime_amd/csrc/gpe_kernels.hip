@@ -197,7 +197,7 @@ __device__ __forceinline__ void sweep_body_single(const SweepArgs &a, const Fiel
         const R ry = k.p0[1] + sig * (k.cell[1] * (R)y + pos[1]);
         const R rz = k.p0[2] + sig * (k.cell[2] * (R)z + pos[2]);
         R vtrap = 0;
-        if (fr->t < ph.trap_off_time)
+        if (fr->trap_on)
             vtrap = (R)0.5 * (k.trap2[0] * rx * rx + k.trap2[1] * ry * ry + k.trap2[2] * rz * rz) + k.trap_offset;
         R Bx = 0, By = 0, Bz = 0, Qx = 0, Qy = 0, Qz = 0;
         if constexpr (C > 1) {
@@ -471,7 +471,7 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, const Field 
         const float *pos = a.tb.pos32 + 3 * v;
         const float ry = pf.p0[1] + sig * (pf.cell[1] * (float)y + pos[1]);
         const float rz = pf.p0[2] + sig * (pf.cell[2] * (float)z + pos[2]);
-        const bool trap_on = fr->t < ph.trap_off_time;
+        const bool trap_on = fr->trap_on != 0;
         const float coef = (float)a.coef;
         float2 out[2][C];
 #pragma unroll
@@ -569,12 +569,13 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &a, const Field &fiel
 template <typename R, int C, int DEG, int MODE, int X, int NIN>
 __global__ __launch_bounds__(256) void k_sweep(SweepArgs a)
 {
-    // spinors load it after the neighbours (fewer scalar registers held: FCC 30^3 spin-1 8.3 -> 7.9 us a
-    // sweep); one component needs its first 24 bytes only, at once, from a line of the arguments that
-    // it reads anyway (BCC 30^3 4.4 -> 4.2, FCC 24x18x23 5.2 -> 5.0 against a line of its own)
+    // FP32 spinors load it after the neighbours (fewer scalar registers held: FCC 30^3 spin-1 8.3 -> 7.9
+    // us a sweep); FP64 ones as early as can be (FCC 64^3 81.6 -> 78.9).  One component needs its first
+    // bytes only, at once, from a line of the arguments that it reads anyway (BCC 30^3 4.4 -> 4.2, FCC
+    // 24x18x23 5.4 -> 5.0 against a line of its own)
     const auto field = []() {
         constexpr unsigned at = offsetof(SweepArgs, field);
-        return C > 1 ? fresh_args<FieldRec>(at) : args_at<FieldRec>(at);
+        return C > 1 && std::is_same<R, float>::value ? fresh_args<FieldRec>(at) : args_at<FieldRec>(at);
     };
     sweep_body<R, C, DEG, MODE, X, NIN>(a, field, sweep_order(a.g, blockIdx.x, gridDim.x, a.order), gridDim.x);
 }
@@ -937,7 +938,7 @@ __global__ __launch_bounds__(256) void k_aux(AuxArgs a)
         const double ry = ph.p0[1] + sig * (ph.cell[1] * y + pos[1]);
         const double rz = ph.p0[2] + sig * (ph.cell[2] * z + pos[2]);
         double vtrap = 0;
-        if (a.field.t < ph.trap_off_time)
+        if (a.field.trap_on)
             vtrap = 0.5 * (ph.trap2[0] * rx * rx + ph.trap2[1] * ry * ry + ph.trap2[2] * rz * rz) + ph.trap_offset;
         const double p = vtrap + ph.c0 * n;
         hmax = p;
