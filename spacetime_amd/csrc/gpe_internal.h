@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstdint>
 
 #include "gpe.h"
@@ -124,6 +125,7 @@ struct Physics {
     double center[3];
     PhysicsF f;            // the same in FP32
     double trap_off_time;  // read on the host (FieldRec::trap_on)
+    double pad[4];         // SweepArgs::cur on a line
 };
 
 // Field and time of one sweep (computed on the host from the ramp); what one component reads
@@ -156,6 +158,10 @@ struct SweepArgs {
     double *partials;         // ITP: one FP64 partial norm per workgroup
     FieldRec field;           // field and time of the sweep (a single launch), beside coef for its head
 };
+
+// The level pointers, which a wave's first loads wait for, and coef lie on one line of the arguments
+// (over two: Cube 75x61x90 5.05 us a sweep, 4.94 so).
+static_assert(offsetof(SweepArgs, cur) % 64 == 0, "level pointers start a line");
 
 // Observables partial sums per workgroup.
 enum {
