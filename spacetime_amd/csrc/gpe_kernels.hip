@@ -1497,6 +1497,33 @@ __global__ __launch_bounds__(256) void k_pack(Geometry g, const int *__restrict_
     }
 }
 
+// One ABI value a thread: cells of one unknown, whose two sides are runs of lines already (Cube 150^3 FP64
+// in 30 us through LDS, 26 so), and FP64 levels of small cells that the caches hold, on the way in (BCC
+// 48^3 spin-1 35 us through LDS, 31 so; 96^3 210 and 247).
+template <typename R, bool PACK>
+__global__ __launch_bounds__(256) void k_pack_values(Geometry g, const int *__restrict__ place, const double2 *__restrict__ abi_in,
+                                                     double2 *__restrict__ abi_out, const vec2_t<R> *__restrict__ dev_in,
+                                                     vec2_t<R> *__restrict__ dev_out)
+{
+    const long long values = (long long)g.nz * g.ny * g.nx * g.V;
+    const long long n = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (n >= values) return;
+    const long long q = n / g.V, row = q / g.nx;
+    const int p = place[(int)(n - q * g.V)], x = (int)(q - row * g.nx);
+    const int z = (int)(row / g.ny), y = (int)(row - (long long)z * g.ny);
+    const long long d = line_index(g, blockIdx.y, z, y, p) + x, i = blockIdx.y * values + n;
+    if constexpr (PACK) {
+        const double2 s = abi_in[i];
+        vec2_t<R> o;
+        o.x = (R)s.x;
+        o.y = (R)s.y;
+        dev_out[d] = o;
+    } else {
+        const vec2_t<R> s = dev_in[d];
+        abi_out[i] = make_double2((double)s.x, (double)s.y);
+    }
+}
+
 // ------------------------------------------------------------------------- launchers --
 
 static inline unsigned grid1(long long n) { return (unsigned)((n + 255) / 256); }
@@ -1770,17 +1797,26 @@ hipError_t launch_phase_copy(int fp64, const void *src, void *dst, long long nel
     return hipGetLastError();
 }
 
-// Cells per workgroup: a tile of up to 40 KiB (four workgroups a CU; up to 64 KiB: BCC 96^3 FP64 out
-// 181 -> 256 us; up to 32 KiB: C15 57^3 spin-2 in 840 -> 930), less while that leaves the chip short of
-// workgroups, but 16 cells, 128-byte pieces of a line in FP32, at least.
+// Cells per workgroup: 64 (fewer where those of a large cell fill more than 24 KiB or a
+// small box has under 128 workgroups, but 16 cells), and more, in
+// a tile of up to 40 KiB, while there are workgroups enough to hide a tile's load before its store.
+// Measured: tiles of up to 64 KiB, BCC 96^3 FP64 out 181 -> 256 us; of up to 32 KiB, C15 57^3 spin-2 in
+// 840 -> 930; 16 cells of FCC 30^3 spin-1 in 20 us, 64 16; 256 of FCC 60^3 spin-1 in 45, 64 41.
 template <typename R, bool PACK>
 static hipError_t pack(const Geometry &g, const Tables &tb, int ncomp, const double *abi_in, double *abi_out, const void *dev_in,
                        void *dev_out, hipStream_t s)
 {
     const long long cells = (long long)g.nz * g.ny * g.nx;
+    const long long values = cells * g.V;
+    if (g.V == 1 || (PACK && sizeof(R) == 8 && g.V <= 12 && ncomp * values < (8 << 20))) {
+        hipLaunchKernelGGL((k_pack_values<R, PACK>), dim3(grid1(values), (unsigned)ncomp), dim3(256), 0, s, g, tb.place,
+                           (const double2 *)abi_in, (double2 *)abi_out, (const vec2_t<R> *)dev_in, (vec2_t<R> *)dev_out);
+        return hipGetLastError();
+    }
     const size_t cell = (size_t)(g.V | 1) * sizeof(vec2_t<R>);
-    int lg = 4;
-    while (lg < 10 && (cell << (lg + 1)) <= 40960 && ncomp * ((cells >> (lg + 1)) + 1) >= 1024) ++lg;
+    int lg = 6;
+    while (lg > 4 && ((cell << lg) > 24576 || ncomp * (cells >> lg) < 128)) --lg;
+    while (lg < 10 && (cell << (lg + 1)) <= 40960 && ncomp * ((cells >> (lg + 1)) + 1) >= 8192) ++lg;
     const size_t lds = (cell << lg) + (sizeof(int) << lg) + sizeof(int) * (size_t)g.V;
     const dim3 grid((unsigned)((cells + (1 << lg) - 1) >> lg), (unsigned)ncomp);
     hipLaunchKernelGGL((k_pack<R, PACK>), grid, dim3(256), lds, s, g, tb.abi, lg, (const double2 *)abi_in, (double2 *)abi_out,

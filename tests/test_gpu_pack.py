@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 BOXES = [("cube", 1, (1, 1, 1)), ("cube", 1, (1, 37, 5)), ("cube", 1, (128, 100, 90)), ("cube", 5, (75, 31, 9)),
          ("bcc", 3, (8, 6, 5)), ("bcc", 1, (129, 33, 40)), ("fcc", 3, (41, 40, 21)), ("a15", 5, (17, 3, 11)),
-         ("c15", 3, (57, 9, 2)), ("c15", 1, (30, 29, 23)), ("z", 5, (34, 5, 3))]
+         ("c15", 3, (57, 9, 2)), ("c15", 1, (30, 29, 23)), ("fcc", 3, (61, 61, 61)), ("z", 5, (34, 5, 3))]
 
 
 @pytest.mark.parametrize("precision", [gpe.FP32, gpe.FP64])
