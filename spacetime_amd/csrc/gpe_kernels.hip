@@ -554,7 +554,7 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs &a, const Field 
 }
 
 // X: the lane form (lane_form).
-// field: gives the sweep's FieldRec, loaded where it is used (fresh).
+// field: gives the sweep's FieldRec.
 template <typename R, int C, int DEG, int MODE, int X, int NIN, typename Field>
 __device__ __forceinline__ void sweep_body(const SweepArgs &a, const Field &field, int b, int nb)
 {
@@ -569,14 +569,10 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &a, const Field &fiel
 template <typename R, int C, int DEG, int MODE, int X, int NIN>
 __global__ __launch_bounds__(256) void k_sweep(SweepArgs a)
 {
-    // FP32 spinors load it after the neighbours (fewer scalar registers held: FCC 30^3 spin-1 8.3 -> 7.9
-    // us a sweep); FP64 ones as early as can be (FCC 64^3 81.6 -> 78.9).  One component needs its first
-    // bytes only, at once, from a line of the arguments that it reads anyway (BCC 30^3 4.4 -> 4.2, FCC
-    // 24x18x23 5.4 -> 5.0 against a line of its own)
-    const auto field = []() {
-        constexpr unsigned at = offsetof(SweepArgs, field);
-        return C > 1 && std::is_same<R, float>::value ? fresh_args<FieldRec>(at) : args_at<FieldRec>(at);
-    };
+    // loaded as early as can be: kept for after the neighbours it costs large boxes 2-3% (FCC 128^3 spin-1
+    // 342 -> 351 us a sweep).  Its head lies on a line of the arguments that every wave reads (BCC 30^3
+    // 4.4 -> 4.2, FCC 30^3 spin-1 7.8 -> 7.1)
+    const auto field = []() { return args_at<FieldRec>(offsetof(SweepArgs, field)); };
     sweep_body<R, C, DEG, MODE, X, NIN>(a, field, sweep_order(a.g, blockIdx.x, gridDim.x, a.order), gridDim.x);
 }
 
