@@ -2078,14 +2078,16 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
     if (trial_sweeps < 0) return fail(c, GPE_EINVAL, "negative trial sweeps");
     const TuneKey key(c->cfg.lattice, c->cfg.ncomp, c->fp64, c->cfg.nx, c->cfg.ny, c->cfg.nz);
     const size_t partials_before = partials_bytes(c);
-    int best_ty = c->g.ty, best_remap = c->gs.xcd_remap | (c->gs.v_inner << 1), best_xpl = c->gs.xpl;
+    int best_ty = c->gs.ty, best_remap = c->gs.xcd_remap | (c->gs.v_inner << 1), best_xpl = c->gs.xpl;
     double best_ms = -1.0;
+    bool chosen = trial_sweeps > 0;  // otherwise the context keeps what it has
     {
         std::lock_guard<std::mutex> lk(g_tune_mutex);
         auto it = g_tune_cache.find(key);
         if (it != g_tune_cache.end()) {
             std::tie(best_ty, best_remap, best_xpl) = it->second;
             trial_sweeps = 0;
+            chosen = true;
         }
     }
     if (trial_sweeps > 0) {
@@ -2151,7 +2153,7 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
         std::lock_guard<std::mutex> lk(g_tune_mutex);
         g_tune_cache[key] = std::make_tuple(best_ty, best_remap, best_xpl);
     }
-    if (!set_traversal(c, best_ty, best_remap, best_xpl))
+    if (chosen && !set_traversal(c, best_ty, best_remap, best_xpl))
         return fail(c, GPE_EINVAL, "traversal needs more workgroups than the decode supports");
     int rc = grow_partials(c, partials_before);
     if (rc) return rc;
