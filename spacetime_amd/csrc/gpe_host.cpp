@@ -2116,17 +2116,25 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
         // candidates only where their row groups are not powers of two; and the whole plane
         // (one tile: each XCD a range of planes that share their y neighbours in its L2;
         // FP32 A15 82^3 one component +17%, spin-2 +8%, Cube 293^3 one component +11%)
+        // the height of an untuned sweep comes first, whatever it is: without it the fastest candidate
+        // can be slower than not tuning (lanes used, untuned against the best other candidate: FCC 19^3
+        // spin-1 99% and 74%, A15 9x11x9 86% and 43%, FP64 FCC 17^3 90% and 50%)
         std::vector<int> tys = {1, 2, 4, 8, 16, 32, 3, 6, 12, 24, 5, 10, 20, 7, 14, 28};
         if (c->g.ny > 32 && c->g.ny <= 1024) tys.push_back(c->g.ny);
+        Geometry untuned = base_geometry(c->cfg);
+        untuned.xpl = default_xpl(c->fp64, untuned.deg, c->cfg.ncomp, c->cfg.nx);
+        const int untuned_ty = default_tile(untuned, c->elem_bytes, c->fp64);
+        tys.erase(std::remove(tys.begin(), tys.end(), untuned_ty), tys.end());
+        tys.insert(tys.begin(), untuned_ty);
         const int nxpl = pair_lanes_ok(c->fp64, c->g.deg, c->cfg.ncomp) ? 2 : 1;
         for (int xpl = 1; xpl <= nxpl; ++xpl)
         for (int ty : tys) {
             if (ty > c->g.ny && ty != 1) continue;
-            const bool pow2 = (ty & (ty - 1)) == 0;
+            const bool any_rows = (ty & (ty - 1)) == 0 || (ty == untuned_ty && xpl == untuned.xpl);
             // flags: XCD remap, and the unknown inside the x segment (only where lines span several waves)
             for (int remap = 0; remap < 4; ++remap) {
                 if (!set_traversal(c, ty, remap, xpl)) continue;  // too many workgroups: not a candidate
-                if (!pow2 && (xpl == 1 || (c->gs.rows & (c->gs.rows - 1)) == 0)) continue;
+                if (!any_rows && (xpl == 1 || (c->gs.rows & (c->gs.rows - 1)) == 0)) continue;
                 if ((remap & 2) && c->gs.nseg == 1) continue;
                 void *cur = trial.s0, *nxt = trial.s1;
                 for (int k = 0; k < trial_sweeps + 2; ++k) {
