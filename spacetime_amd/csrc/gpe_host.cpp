@@ -156,21 +156,36 @@ void drop_workspace(Workspace *w)  // with g_ws_mutex held
     g_workspaces.erase(w);
 }
 
-// hipMalloc; where that fails, again after the device's idle workspaces are given back.
+// Give back the device's idle workspaces; whether there were any.
+bool drop_idle_workspaces(int device)
+{
+    std::lock_guard<std::mutex> lk(g_ws_mutex);
+    bool any = false;
+    for (auto it = g_workspaces.begin(); it != g_workspaces.end();) {
+        Workspace *w = *it++;
+        if (w->busy || w->device != device) continue;
+        drop_workspace(w);
+        any = true;
+    }
+    return any;
+}
+
+// The library's device memory: hipMalloc (hipMallocAsync with a stream); where that fails, again
+// after the device's idle workspaces are given back.
 hipError_t device_malloc(void **out, size_t bytes, int device)
 {
-    hipError_t e = hipMalloc(out, bytes);
-    if (e == hipSuccess) return e;
-    {
-        std::lock_guard<std::mutex> lk(g_ws_mutex);
-        std::vector<Workspace *> idle;
-        for (Workspace *w : g_workspaces)
-            if (!w->busy && w->device == device) idle.push_back(w);
-        if (idle.empty()) return e;
-        for (Workspace *w : idle) drop_workspace(w);
-    }
+    const hipError_t e = hipMalloc(out, bytes);
+    if (e == hipSuccess || !drop_idle_workspaces(device)) return e;
     (void)hipGetLastError();
     return hipMalloc(out, bytes);
+}
+
+hipError_t device_malloc(void **out, size_t bytes, int device, hipStream_t stream)
+{
+    const hipError_t e = hipMallocAsync(out, bytes, stream);
+    if (e == hipSuccess || !drop_idle_workspaces(device)) return e;
+    (void)hipGetLastError();
+    return hipMallocAsync(out, bytes, stream);
 }
 
 // At least `bytes` of the context's workspace, until end_workspace.
@@ -338,7 +353,7 @@ int ensure_fields(gpe_ctx *c, int n)
         c->d_fields = nullptr;
         c->h_fields = nullptr;
     }
-    HIPCALL(c, hipMalloc((void **)&c->d_fields, sizeof(FieldRec) * cap));
+    HIPCALL(c, device_malloc((void **)&c->d_fields, sizeof(FieldRec) * cap, c->device));
     HIPCALL(c, hipHostMalloc((void **)&c->h_fields, sizeof(FieldRec) * cap, hipHostMallocDefault));
     c->fields_cap = cap;
     return GPE_OK;
@@ -805,7 +820,7 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     }
     auto up = [&](void **dst, const void *src, size_t bytes) {
         if (rc) return;
-        hipError_t ee = hipMalloc(dst, bytes);
+        hipError_t ee = device_malloc(dst, bytes, c->device);
         if (ee != hipSuccess) {
             rc = GPE_ENOMEM;
             return;
@@ -828,11 +843,11 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
     up((void **)&c->d_pos32, pos32.data(), sizeof(float) * 3 * V);
     up((void **)&c->d_pos64, pos64.data(), sizeof(double) * 3 * V);
     up((void **)&c->d_dv, dv.data(), sizeof(double) * V);
-    if (!rc && hipMalloc((void **)&c->d_partials, partials_bytes(c)) != hipSuccess) rc = GPE_ENOMEM;
+    if (!rc && device_malloc((void **)&c->d_partials, partials_bytes(c), c->device) != hipSuccess) rc = GPE_ENOMEM;
     if (!rc && hipHostMalloc((void **)&c->h_red, sizeof(double) * FIN_WIDTH_MAX, hipHostMallocDefault) != hipSuccess)
         rc = GPE_ENOMEM;
-    if (!rc && hipMalloc((void **)&c->d_scalars, sizeof(double) * 64) != hipSuccess) rc = GPE_ENOMEM;
-    if (!rc && hipMalloc((void **)&c->d_red, sizeof(double) * FIN_SCRATCH) != hipSuccess) rc = GPE_ENOMEM;
+    if (!rc && device_malloc((void **)&c->d_scalars, sizeof(double) * 64, c->device) != hipSuccess) rc = GPE_ENOMEM;
+    if (!rc && device_malloc((void **)&c->d_red, sizeof(double) * FIN_SCRATCH, c->device) != hipSuccess) rc = GPE_ENOMEM;
     if (!rc) rc = ensure_fields(c, 1024);
     if (!rc && (e = hipEventCreate(&c->ev0)) != hipSuccess) rc = hip_fail(c, e, "hipEventCreate");
     if (!rc && (e = hipEventCreate(&c->ev1)) != hipSuccess) rc = hip_fail(c, e, "hipEventCreate");
@@ -880,7 +895,7 @@ static int set_state_impl(gpe_ctx *c, int level, const double *psi, double t, hi
     const double *src = psi;
     double *staging = nullptr;
     if (kind == hipMemcpyHostToDevice) {
-        HIPCALL(c, hipMallocAsync((void **)&staging, nbytes, c->stream));
+        HIPCALL(c, device_malloc((void **)&staging, nbytes, c->device, c->stream));
         HIPCALL(c, hipMemcpyAsync(staging, psi, nbytes, hipMemcpyHostToDevice, c->stream));
         src = staging;
     }
@@ -919,7 +934,7 @@ static int get_state_impl(gpe_ctx *c, int level, double *psi, bool host)
     double *dst = psi;
     double *staging = nullptr;
     if (host) {
-        HIPCALL(c, hipMallocAsync((void **)&staging, nbytes, c->stream));
+        HIPCALL(c, device_malloc((void **)&staging, nbytes, c->device, c->stream));
         dst = staging;
     }
     hipError_t e = launch_unpack(c->fp64, g, tables(c), c->cfg.ncomp, c->level[level], dst, c->stream);
@@ -1814,7 +1829,7 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
     }
     int rc = GPE_OK;
     if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess) rc = GPE_EDEVICE;
-    if (!rc && hipMalloc((void **)&e->d_base, sizeof(int) * 4) != hipSuccess) rc = GPE_ENOMEM;
+    if (!rc && device_malloc((void **)&e->d_base, sizeof(int) * 4, c0->device) != hipSuccess) rc = GPE_ENOMEM;
     if (!rc && (hipEventCreate(&e->ev0) != hipSuccess || hipEventCreate(&e->ev1) != hipSuccess)) rc = GPE_EDEVICE;
     if (rc) {
         gpe_ensemble_destroy(e);
@@ -1877,7 +1892,7 @@ int gpe_ensemble_step(gpe_ensemble *e, int nsteps, int graph_sweeps)
         e->up_bytes = 0;
         if (e->gexec) (void)hipGraphExecDestroy(e->gexec);  // captured with the old records' address
         e->gexec = nullptr;
-        ENSCALL(e, hipMalloc((void **)&e->d, bytes));
+        ENSCALL(e, device_malloc((void **)&e->d, bytes, e->m[0]->device));
         ENSCALL(e, hipHostMalloc((void **)&e->up, bytes, hipHostMallocDefault));
         e->up_bytes = bytes;
     }
@@ -1995,7 +2010,7 @@ static int grow_partials(gpe_ctx *c, size_t before)
     HIPCALL(c, hipStreamSynchronize(c->stream));
     (void)hipFree(c->d_partials);
     c->d_partials = nullptr;
-    if (hipMalloc((void **)&c->d_partials, partials_bytes(c)) != hipSuccess)
+    if (device_malloc((void **)&c->d_partials, partials_bytes(c), c->device) != hipSuccess)
         return fail(c, GPE_ENOMEM, "partials");
     return GPE_OK;
 }
@@ -2180,7 +2195,10 @@ int gpe_stream_bandwidth(long long bytes, int reps, double *copy_gbs, double *up
     hipStream_t s = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = GPE_OK;
-    if (hipMalloc(&a, bytes) != hipSuccess || hipMalloc(&b, bytes) != hipSuccess) rc = GPE_ENOMEM;
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) rc = GPE_EDEVICE;
+    if (!rc && (device_malloc(&a, bytes, device) != hipSuccess || device_malloc(&b, bytes, device) != hipSuccess))
+        rc = GPE_ENOMEM;
     if (!rc && (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&e0) != hipSuccess ||
                 hipEventCreate(&e1) != hipSuccess))
         rc = GPE_EDEVICE;

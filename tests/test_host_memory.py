@@ -1,0 +1,67 @@
+"""Device memory that contexts keep between calls, on the host stand-in: whatever the library
+allocates finds room where only an idle workspace is in the way."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from spacetime_amd import gpe
+from stand_in import stand_in, started  # noqa: F401
+
+BOX = ("bcc", 3, gpe.FP32, (8, 6, 5))
+
+
+def keep_workspace():
+    """A context that holds the workspace of an adjoint run."""
+    st = started(*BOX)
+    st.set_state(np.zeros(st.config.shape, dtype=np.complex128))
+    st.adjoint(60, 30, gpe.OBJ_ENERGY)
+    return st
+
+
+def calls():
+    """Name -> (what a program has made before, the call that allocates)."""
+    def state():
+        return started(*BOX)
+
+    def ensemble():
+        return gpe.Ensemble([started(*BOX), started(*BOX)])
+
+    def tall():  # its reduction partials grow with tiles of 10 rows (20 rows of waves a plane, 16 before)
+        return started("bcc", 1, gpe.FP64, (2, 11, 400))
+
+    zeros = np.zeros(gpe.Config.centred_box(*BOX[:1], BOX[3], 0.7, ncomp=3).shape, dtype=np.complex128)
+    return dict(
+        create=(lambda: None, lambda _: started(*BOX)),
+        set_state=(state, lambda st: st.set_state(zeros)),
+        get_state=(state, lambda st: st.get_state(0)),
+        weighted_diff=(state, lambda st: st.weighted_diff(zeros)),
+        local_fields=(state, lambda st: st.local_fields(0)),
+        autotune=(state, lambda st: st.autotune(1)),
+        partials=(tall, lambda st: st.set_traversal(10, 1, 1)),
+        ensemble_create=(lambda: [started(*BOX)], lambda m: gpe.Ensemble(m)),
+        ensemble_step=(ensemble, lambda e: e.step(50)),
+        bandwidth=(lambda: None, lambda _: gpe.stream_bandwidth(1 << 20, 1)),
+    )
+
+
+@pytest.mark.parametrize("name", sorted(calls()))
+def test_every_allocation_gets_an_idle_workspace_back(stand_in, name):  # noqa: F811
+    before, call = calls()[name]
+    with keep_workspace():
+        held = before()
+        stand_in.limits(capacity=stand_in.counts()["used"] + 1)  # full but for the workspace
+        call(held)
+
+
+def test_fields_of_a_long_adjoint_get_another_runs_workspace(stand_in):  # noqa: F811
+    """The field records of more sweeps than before, allocated while the call's own workspace is in use."""
+    with keep_workspace(), started("cube", 1, gpe.FP32, (2, 2, 2)) as st:
+        st.set_state(np.zeros(st.config.shape, dtype=np.complex128))
+        used = stand_in.counts()["used"]
+        st.adjoint(3000, 2000, gpe.OBJ_ENERGY)
+        need = stand_in.counts()["used"] - used
+    with keep_workspace(), started("cube", 1, gpe.FP32, (2, 2, 2)) as st:
+        st.set_state(np.zeros(st.config.shape, dtype=np.complex128))
+        stand_in.limits(capacity=stand_in.counts()["used"] + need - 1)
+        st.adjoint(3000, 2000, gpe.OBJ_ENERGY)
