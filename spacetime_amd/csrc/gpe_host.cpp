@@ -2003,15 +2003,27 @@ static bool set_traversal(gpe_ctx *c, int ty, int flags, int xpl)
     return true;
 }
 
-// Reduction partials after a change of traversal; `before` their size then.
-static int grow_partials(gpe_ctx *c, size_t before)
+// Apply a traversal with room for its reduction partials; where that fails the context keeps the
+// traversal and the partials it had.
+static int change_traversal(gpe_ctx *c, int ty, int flags, int xpl)
 {
+    const Geometry g = c->g, gs = c->gs;
+    const size_t before = partials_bytes(c);
+    if (!set_traversal(c, ty, flags, xpl))
+        return fail(c, GPE_EINVAL, "traversal needs more workgroups than the decode supports");
     if (partials_bytes(c) <= before) return GPE_OK;
-    HIPCALL(c, hipStreamSynchronize(c->stream));
+    double *grown = nullptr;
+    hipError_t e = device_malloc((void **)&grown, partials_bytes(c), c->device);
+    const int code = e == hipSuccess ? GPE_EDEVICE : GPE_ENOMEM;
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) {
+        if (grown) (void)hipFree(grown);
+        c->g = g;
+        c->gs = gs;
+        return fail(c, code, "partials");
+    }
     (void)hipFree(c->d_partials);
-    c->d_partials = nullptr;
-    if (device_malloc((void **)&c->d_partials, partials_bytes(c), c->device) != hipSuccess)
-        return fail(c, GPE_ENOMEM, "partials");
+    c->d_partials = grown;
     return GPE_OK;
 }
 
@@ -2022,10 +2034,7 @@ int gpe_set_traversal(gpe_ctx *c, int tile_rows, int xcd_remap, int x_per_lane)
         return fail(c, GPE_EINVAL, "bad traversal");
     if (x_per_lane == 2 && !pair_lanes_ok(c->fp64, c->g.deg, c->cfg.ncomp))
         return fail(c, GPE_EINVAL, "two x per lane needs FP32");
-    const size_t before = partials_bytes(c);
-    if (!set_traversal(c, tile_rows, xcd_remap, x_per_lane))
-        return fail(c, GPE_EINVAL, "traversal needs more workgroups than the decode supports");
-    return grow_partials(c, before);
+    return change_traversal(c, tile_rows, xcd_remap, x_per_lane);
 }
 
 int gpe_traversal(const gpe_ctx *c, int *tile_rows, int *xcd_remap, int *x_per_lane)
@@ -2092,7 +2101,6 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
     if (!c) return GPE_EINVAL;
     if (trial_sweeps < 0) return fail(c, GPE_EINVAL, "negative trial sweeps");
     const TuneKey key(c->cfg.lattice, c->cfg.ncomp, c->fp64, c->cfg.nx, c->cfg.ny, c->cfg.nz);
-    const size_t partials_before = partials_bytes(c);
     int best_ty = c->gs.ty, best_remap = c->gs.xcd_remap | (c->gs.v_inner << 1), best_xpl = c->gs.xpl;
     double best_ms = -1.0;
     bool chosen = trial_sweeps > 0;  // otherwise the context keeps what it has
@@ -2176,9 +2184,7 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
         std::lock_guard<std::mutex> lk(g_tune_mutex);
         g_tune_cache[key] = std::make_tuple(best_ty, best_remap, best_xpl);
     }
-    if (chosen && !set_traversal(c, best_ty, best_remap, best_xpl))
-        return fail(c, GPE_EINVAL, "traversal needs more workgroups than the decode supports");
-    int rc = grow_partials(c, partials_before);
+    const int rc = chosen ? change_traversal(c, best_ty, best_remap, best_xpl) : GPE_OK;
     if (rc) return rc;
     if (tile_rows) *tile_rows = best_ty;
     if (xcd_remap) *xcd_remap = best_remap;

@@ -65,3 +65,15 @@ def test_fields_of_a_long_adjoint_get_another_runs_workspace(stand_in):  # noqa:
         st.set_state(np.zeros(st.config.shape, dtype=np.complex128))
         stand_in.limits(capacity=stand_in.counts()["used"] + need - 1)
         st.adjoint(3000, 2000, gpe.OBJ_ENERGY)
+
+
+def test_a_traversal_without_room_for_its_partials_is_refused_and_changes_nothing(stand_in):  # noqa: F811
+    with started("bcc", 1, gpe.FP64, (2, 11, 400)) as st:
+        before = st.traversal()
+        stand_in.limits(capacity=stand_in.counts()["used"] + 1)
+        with pytest.raises(gpe.GpeError, match="ENOMEM"):
+            st.set_traversal(10, 1, 1)
+        assert st.traversal() == before
+        used = stand_in.counts()["used"]
+        st.itp(1, 1e-3)  # its partials are still there
+        assert stand_in.counts()["used"] == used
