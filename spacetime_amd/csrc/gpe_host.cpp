@@ -352,6 +352,7 @@ int ensure_fields(gpe_ctx *c, int n)
         (void)hipHostFree(c->h_fields);
         c->d_fields = nullptr;
         c->h_fields = nullptr;
+        c->fields_cap = 0;
     }
     HIPCALL(c, device_malloc((void **)&c->d_fields, sizeof(FieldRec) * cap, c->device));
     HIPCALL(c, hipHostMalloc((void **)&c->h_fields, sizeof(FieldRec) * cap, hipHostMallocDefault));

@@ -77,3 +77,18 @@ def test_a_traversal_without_room_for_its_partials_is_refused_and_changes_nothin
         used = stand_in.counts()["used"]
         st.itp(1, 1e-3)  # its partials are still there
         assert stand_in.counts()["used"] == used
+
+
+def test_a_failed_growth_of_the_field_records_is_not_taken_for_room(stand_in):  # noqa: F811
+    with started("cube", 1, gpe.FP32, (2, 2, 2)) as st:
+        zeros = np.zeros(st.config.shape, dtype=np.complex128)
+        st.set_state(zeros)
+        st.adjoint(600, 200, gpe.OBJ_ENERGY)  # workspace made, records for 1024 sweeps
+        st.set_state(zeros)
+        # room for the larger workspace, none for 4096 records (the old ones are freed first)
+        stand_in.limits(max_block=400000)
+        with pytest.raises(gpe.GpeError, match="EDEVICE"):
+            st.adjoint(3000, 60, gpe.OBJ_ENERGY)
+        stand_in.limits()
+        st.set_state(zeros)
+        st.adjoint(600, 200, gpe.OBJ_ENERGY)
