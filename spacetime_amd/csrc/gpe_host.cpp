@@ -75,6 +75,7 @@ struct Workspace {
     size_t bytes = 0;
     int device = 0;
     bool busy = false;
+    std::vector<void *> loose;  // buffers of the current call where one block for all does not fit
 };
 
 struct gpe_ctx {
@@ -156,6 +157,12 @@ void drop_workspace(Workspace *w)  // with g_ws_mutex held
     g_workspaces.erase(w);
 }
 
+void drop_loose(Workspace *w)  // the context's own call
+{
+    for (void *p : w->loose) (void)hipFree(p);
+    w->loose.clear();
+}
+
 // Give back the device's idle workspaces; whether there were any.
 bool drop_idle_workspaces(int device)
 {
@@ -188,32 +195,52 @@ hipError_t device_malloc(void **out, size_t bytes, int device, hipStream_t strea
     return hipMallocAsync(out, bytes, stream);
 }
 
-// At least `bytes` of the context's workspace, until end_workspace.
-hipError_t begin_workspace(gpe_ctx *c, size_t bytes, char **out)
+// Buffers of these sizes from the context's workspace, until end_workspace: one block, or where that
+// does not fit (one allocation has to be contiguous and below the driver's limit) each on its own.
+hipError_t begin_workspace(gpe_ctx *c, const std::vector<size_t> &sizes, std::vector<void *> &out)
 {
     Workspace &w = c->ws;
+    size_t bytes = 0;
+    for (size_t n : sizes) bytes += (n + 255) / 256 * 256;
+    out.assign(sizes.size(), nullptr);
+    const auto cut = [&](char *p) {
+        for (size_t i = 0; i < sizes.size(); ++i) {
+            out[i] = p;
+            p += (sizes[i] + 255) / 256 * 256;
+        }
+    };
     {
         std::lock_guard<std::mutex> lk(g_ws_mutex);
         if (w.bytes >= bytes) {
             w.busy = true;
-            *out = (char *)w.p;
+            cut((char *)w.p);
             return hipSuccess;
         }
         drop_workspace(&w);
     }
     void *p = nullptr;
-    const hipError_t e = device_malloc(&p, bytes, c->device);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return e;
+    hipError_t e = device_malloc(&p, bytes, c->device);
+    if (e == hipSuccess) {
+        std::lock_guard<std::mutex> lk(g_ws_mutex);
+        w.p = p;
+        w.bytes = bytes;
+        w.device = c->device;
+        w.busy = true;
+        g_workspaces.insert(&w);
+        cut((char *)p);
+        return hipSuccess;
     }
-    std::lock_guard<std::mutex> lk(g_ws_mutex);
-    w.p = p;
-    w.bytes = bytes;
-    w.device = c->device;
-    w.busy = true;
-    g_workspaces.insert(&w);
-    *out = (char *)p;
+    (void)hipGetLastError();
+    w.loose.reserve(sizes.size());
+    for (size_t i = 0; i < sizes.size(); ++i) {
+        e = device_malloc(&out[i], sizes[i] > 0 ? sizes[i] : 1, c->device);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            drop_loose(&w);
+            return e;
+        }
+        w.loose.push_back(out[i]);
+    }
     return hipSuccess;
 }
 
@@ -232,6 +259,7 @@ void move_workspace(Workspace *from, Workspace *to)
 // The work on the workspace has ended (its streams synchronised): keep it or give it back.
 void end_workspace(gpe_ctx *c)
 {
+    drop_loose(&c->ws);
     size_t avail = 0, total = 0;
     const bool known = hipMemGetInfo(&avail, &total) == hipSuccess;
     std::lock_guard<std::mutex> lk(g_ws_mutex);
@@ -1492,41 +1520,30 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
     const size_t sweep_part = (size_t)ADJ_COUNT * adj_blocks;
     const int Q = (int)std::max<size_t>(1, std::min<size_t>((size_t)K, ((size_t)256 << 20) / (sweep_part * 8)));
     // every buffer of the run in the context's workspace
-    size_t arena_bytes = 0;
-    const auto place = [&](size_t bytes) {
-        const size_t at = arena_bytes;
-        arena_bytes += (bytes + 255) / 256 * 256;
-        return at;
-    };
-    const size_t at_levels = place(0), level_step = (lbytes + 255) / 256 * 256;
     const int nseg = std::min(K, N);  // levels of the longest segment
     const int nlevels = 2 * nck + std::max(nseg - 2, 0) + 2 + (overlap ? 1 : 0);
-    arena_bytes += level_step * nlevels;
-    const size_t at_staging = place(overlap ? abi : 0);
-    const size_t at_steps = place(sizeof(double) * ADJ_COUNT * (size_t)N);
-    const size_t at_part = place(sizeof(double) * ADJ_COUNT * (size_t)g.blocks);
-    const size_t at_qpart = place(sizeof(double) * sweep_part * Q);
-    char *arena = nullptr;
-    if (begin_workspace(c, arena_bytes, &arena) != hipSuccess) return fail(c, GPE_ENOMEM, "adjoint buffers do not fit");
+    std::vector<size_t> sizes(nlevels, lbytes);
+    sizes.push_back(overlap ? abi : 0);
+    sizes.push_back(sizeof(double) * ADJ_COUNT * (size_t)N);
+    sizes.push_back(sizeof(double) * ADJ_COUNT * (size_t)g.blocks);
+    sizes.push_back(sizeof(double) * sweep_part * Q);
+    std::vector<void *> bufs;
+    if (begin_workspace(c, sizes, bufs) != hipSuccess) return fail(c, GPE_ENOMEM, "adjoint buffers do not fit");
     const auto release = [&]() {
         (void)hipStreamSynchronize(c->stream);
         if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);
         end_workspace(c);
     };
-    char *level_at = arena + at_levels;
-    const auto next_level = [&]() {
-        void *p = level_at;
-        level_at += level_step;
-        return p;
-    };
+    size_t taken = 0;
+    const auto next = [&]() { return bufs[taken++]; };
     std::vector<void *> ck(2 * nck), seg(std::max(nseg, 2), nullptr);
-    for (void *&p : ck) p = next_level();
-    for (int i = 2; i < nseg; ++i) seg[i] = next_level();  // seg[0], seg[1] alias checkpoints
-    void *mu[2] = {next_level(), next_level()};
-    void *target = overlap ? next_level() : nullptr;
-    double *staging = (double *)(arena + at_staging);
-    double *d_steps = (double *)(arena + at_steps), *d_part = (double *)(arena + at_part);
-    double *d_qpart = (double *)(arena + at_qpart);
+    for (void *&p : ck) p = next();
+    for (int i = 2; i < nseg; ++i) seg[i] = next();  // seg[0], seg[1] alias checkpoints
+    void *mu[2];
+    for (void *&p : mu) p = next();
+    void *target = overlap ? next() : nullptr;
+    double *staging = (double *)next(), *d_steps = (double *)next(), *d_part = (double *)next();
+    double *d_qpart = (double *)next();
     int rc = GPE_OK;
     res->checkpoint_bytes = (double)lbytes * 2 * nck;
     res->segment_bytes = (double)lbytes * (K - 2 + 2);

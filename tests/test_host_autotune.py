@@ -6,7 +6,7 @@ from stand_in import stand_in, started  # noqa: F401
 
 
 @pytest.mark.parametrize("lat,ncomp,precision,dims,rows", [
-    ("fcc", 3, gpe.FP32, (19, 19, 19), 19), ("fcc", 3, gpe.FP64, (17, 17, 5), 17), ("bcc", 3, gpe.FP32, (64, 40, 4), 8)])
+    ("fcc", 3, gpe.FP32, (19, 19, 3), 19), ("fcc", 3, gpe.FP64, (17, 17, 4), 17), ("bcc", 3, gpe.FP32, (64, 40, 5), 8)])
 def test_no_trials_and_nothing_cached_leaves_the_traversal_alone(stand_in, lat, ncomp, precision, dims, rows):  # noqa: F811
     with started(lat, ncomp, precision, dims) as st:
         before = st.traversal()

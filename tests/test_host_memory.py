@@ -92,3 +92,34 @@ def test_a_failed_growth_of_the_field_records_is_not_taken_for_room(stand_in):  
         stand_in.limits()
         st.set_state(zeros)
         st.adjoint(600, 200, gpe.OBJ_ENERGY)
+
+
+@pytest.mark.parametrize("precision,fp64", [(gpe.FP32, False), (gpe.FP64, False), (gpe.FP32, True)])
+def test_buffers_that_fit_only_one_by_one(stand_in, precision, fp64):  # noqa: F811
+    """One block of every buffer does not fit (or is larger than an allocation may be), the buffers do:
+    the run takes them one by one and gives them back; one byte less and it is refused, with nothing
+    left behind."""
+    with started("bcc", 3, precision, (8, 6, 5)) as st:
+        zeros = np.zeros(st.config.shape, dtype=np.complex128)
+
+        def run():
+            st.set_state(zeros)
+            return st.adjoint(30, 10, gpe.OBJ_OVERLAP, zeros, fp64)
+
+        whole = run()  # the field records and the copy stream are made
+        used = stand_in.counts()["used"]
+        stand_in.limits(max_block=400000)  # a level has 69120 or 138240 bytes, staging 138240
+        before = stand_in.counts()["allocs"]
+        # a larger run than the kept block holds
+        st.set_state(zeros)
+        r = st.adjoint(40, 10, gpe.OBJ_OVERLAP, zeros, fp64)
+        assert stand_in.counts()["allocs"] - before > 20 and r["checkpoint_bytes"] > whole["checkpoint_bytes"]
+        assert stand_in.counts()["used"] < used  # not even the old block is kept
+        base = stand_in.counts()["used"]
+        st.set_state(zeros)
+        with pytest.raises(gpe.GpeError, match="ENOMEM"):
+            stand_in.limits(capacity=base + 1000000, max_block=400000)
+            st.adjoint(40, 10, gpe.OBJ_OVERLAP, zeros, fp64)
+        assert stand_in.counts()["used"] == base
+        stand_in.limits()
+        run()
