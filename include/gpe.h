@@ -342,7 +342,8 @@ int gpe_fill_thomas_fermi(gpe_ctx *ctx, double g, double mu, const double *weigh
  * context holds psi_N (level 0) and psi_{N-1} (level 1).  The buffers (two levels a checkpoint,
  * a segment of at most K levels, two adjoint levels) stay with the context for its next call
  * while half of the device is free; they are given back when an allocation of this library
- * fails, and by gpe_destroy. */
+ * fails, by gpe_release_workspace and by gpe_destroy.  Other allocators of the process do not
+ * see them: a program that needs the room for something else releases them first. */
 #define GPE_OBJ_OVERLAP 0         /* J = |<target|psi_N>|^2, <a|b> = sum dv conj(a) b */
 #define GPE_OBJ_ENERGY 1          /* J = E[psi_N] (GP energy functional)              */
 #define GPE_OBJ_MAGNETIZATION_Z 2 /* J = sum dv psi^dag f_z psi                         */
@@ -376,6 +377,8 @@ typedef struct {
 } gpe_adjoint_result;
 
 int gpe_adjoint(gpe_ctx *ctx, const gpe_adjoint_spec *spec, gpe_adjoint_result *res);
+/* Give back the device memory that the context keeps for its next gpe_adjoint. */
+int gpe_release_workspace(gpe_ctx *ctx);
 
 /* Replace the trap frequencies of a context (V = 0.5 sum (trap_a r_a)^2 + offset): the
  * lambda_x,y,z of the reference's trap() (Spin1GpeBCC.cu:112-122), a parameter here so the

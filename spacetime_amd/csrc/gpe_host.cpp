@@ -1764,6 +1764,14 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
     return GPE_OK;
 }
 
+int gpe_release_workspace(gpe_ctx *c)
+{
+    if (!c) return GPE_EINVAL;
+    std::lock_guard<std::mutex> lk(g_ws_mutex);
+    drop_workspace(&c->ws);
+    return GPE_OK;
+}
+
 // ------------------------------------------------------------------------- ensembles ---
 
 // Members sharing (face degree, x per lane) form a group launched by one specialised kernel.

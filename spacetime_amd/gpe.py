@@ -123,6 +123,7 @@ def load_library(path=LIB_PATH):
     lib.gpe_time.argtypes = [vp, _dp, ctypes.POINTER(ctypes.c_longlong)]
     lib.gpe_last_step_timing.argtypes = [vp, _dp, _dp]
     lib.gpe_adjoint.argtypes = [vp, ctypes.POINTER(_AdjSpec), ctypes.POINTER(_AdjRes)]
+    lib.gpe_release_workspace.argtypes = [vp]
     lib.gpe_ensemble_create.argtypes = [ctypes.POINTER(vp), ctypes.c_int, ctypes.POINTER(vp)]
     lib.gpe_ensemble_destroy.argtypes = [vp]
     lib.gpe_ensemble_last_error.argtypes = [vp]
@@ -374,6 +375,10 @@ class Stepper:
                     grad_static_bb=np.array(res.grad_static_bb[:]), grad_ramp_q=gq[:nq], grad_ramp_b=gb[:nb],
                     forward_ms=res.forward_ms, backward_ms=res.backward_ms,
                     checkpoint_bytes=res.checkpoint_bytes, segment_bytes=res.segment_bytes)
+
+    def release_workspace(self):
+        """Give back the device memory kept for the next adjoint() (gpe_release_workspace)."""
+        self._check(self.lib.gpe_release_workspace(self._h), "gpe_release_workspace")
 
     # -- time stepping -------------------------------------------------------------------------
     def clock(self):

@@ -123,3 +123,21 @@ def test_buffers_that_fit_only_one_by_one(stand_in, precision, fp64):  # noqa: F
         assert stand_in.counts()["used"] == base
         stand_in.limits()
         run()
+
+
+def test_a_program_can_have_the_workspace_back(stand_in):  # noqa: F811
+    with started(*BOX) as st:
+        zeros = np.zeros(st.config.shape, dtype=np.complex128)
+        st.set_state(zeros)
+        st.adjoint(2, 2, gpe.OBJ_ENERGY)  # the field records are made
+        st.release_workspace()
+        used = stand_in.counts()["used"]
+        st.set_state(zeros)
+        st.adjoint(30, 10, gpe.OBJ_ENERGY)
+        assert stand_in.counts()["used"] > used
+        st.release_workspace()
+        assert stand_in.counts()["used"] == used
+        st.release_workspace()  # nothing to give
+        st.set_state(zeros)
+        st.adjoint(30, 10, gpe.OBJ_ENERGY)
+    assert stand_in.lib.gpe_release_workspace(None) == -22
