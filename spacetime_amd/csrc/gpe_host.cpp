@@ -1546,7 +1546,7 @@ int gpe_adjoint(gpe_ctx *c, const gpe_adjoint_spec *spec, gpe_adjoint_result *re
     double *d_qpart = (double *)next();
     int rc = GPE_OK;
     res->checkpoint_bytes = (double)lbytes * 2 * nck;
-    res->segment_bytes = (double)lbytes * (K - 2 + 2);
+    res->segment_bytes = (double)lbytes * nseg;
     hipError_t e = hipSuccess;
     // on a failure the buffers are freed and the levels hold an intermediate state: the
     // context needs gpe_set_state (and gpe_start) before it steps again

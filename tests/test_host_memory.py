@@ -141,3 +141,13 @@ def test_a_program_can_have_the_workspace_back(stand_in):  # noqa: F811
         st.set_state(zeros)
         st.adjoint(30, 10, gpe.OBJ_ENERGY)
     assert stand_in.lib.gpe_release_workspace(None) == -22
+
+
+@pytest.mark.parametrize("nsweeps,every,levels", [(30, 10, 10), (30, 50, 30), (1, 2, 1), (2, 2, 2), (7, 8, 7)])
+def test_adjoint_reports_the_levels_of_its_longest_segment(stand_in, nsweeps, every, levels):  # noqa: F811
+    with started(*BOX) as st:
+        st.set_state(np.zeros(st.config.shape, dtype=np.complex128))
+        r = st.adjoint(nsweeps, every, gpe.OBJ_ENERGY)
+        level = 8 * 3 * 8 * 6 * 5 * 12  # bytes: FP32 spinors of 8x6x5 cells of 12 (whole lines, no padding)
+        assert r["segment_bytes"] == levels * level
+        assert r["checkpoint_bytes"] == 2 * -(-nsweeps // every) * level
