@@ -95,13 +95,14 @@ struct gpe_ctx {
     hipStream_t copy_stream = nullptr;  // uploads beside the sweeps (adjoint target), made on first use
     int device = 0;
     void *level[2] = {nullptr, nullptr};
-    // tables
+    // tables: one block, which d_scalars and d_red share
+    char *d_tables = nullptr;
     int *d_abi = nullptr, *d_nface = nullptr, *d_facex = nullptr;  // d_abi: V places, then their inverse
     int *d_oface = nullptr, *d_nfwd = nullptr;  // the observables' faces (ObsArgs)
     double *d_ow = nullptr;
     float *d_w32 = nullptr, *d_wsum32 = nullptr, *d_pos32 = nullptr;
     double *d_w64 = nullptr, *d_wsum64 = nullptr, *d_pos64 = nullptr, *d_dv = nullptr;
-    // fields per sweep
+    // fields per sweep (the adjoint's; made on first use)
     FieldRec *d_fields = nullptr;
     int fields_cap = 0;
     FieldRec *h_fields = nullptr;  // pinned staging
@@ -847,37 +848,47 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
         }
         dv[v] = s * s * s * c->lat->vol[order[v]];
     }
-    auto up = [&](void **dst, const void *src, size_t bytes) {
-        if (rc) return;
-        hipError_t ee = device_malloc(dst, bytes, c->device);
-        if (ee != hipSuccess) {
-            rc = GPE_ENOMEM;
-            return;
-        }
-        ee = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
-        if (ee != hipSuccess) rc = hip_fail(c, ee, "hipMemcpy tables");
-    };
     std::vector<int> abi(order, order + V);
     abi.insert(abi.end(), place.begin(), place.end());
-    up((void **)&c->d_abi, abi.data(), sizeof(int) * 2 * V);
-    up((void **)&c->d_nface, nface.data(), sizeof(int) * V);
-    up((void **)&c->d_facex, facex.data(), sizeof(int) * 2 * V * deg);
-    up((void **)&c->d_oface, oface.data(), sizeof(int) * 2 * V * deg);
-    up((void **)&c->d_ow, ow.data(), sizeof(double) * V * deg);
-    up((void **)&c->d_nfwd, nfwd.data(), sizeof(int) * V);
-    up((void **)&c->d_w32, w32.data(), sizeof(float) * V * deg);
-    up((void **)&c->d_w64, w64.data(), sizeof(double) * V * deg);
-    up((void **)&c->d_wsum32, wsum32.data(), sizeof(float) * V);
-    up((void **)&c->d_wsum64, wsum64.data(), sizeof(double) * V);
-    up((void **)&c->d_pos32, pos32.data(), sizeof(float) * 3 * V);
-    up((void **)&c->d_pos64, pos64.data(), sizeof(double) * 3 * V);
-    up((void **)&c->d_dv, dv.data(), sizeof(double) * V);
+    // the tables in one allocation and one copy, with the small results behind them: copies of their own
+    // (11 us each) and the pinned records of the adjoint's fields, now made by the call that uses them (27 us
+    // and 250 to free), made it 410 us to set up and tear down a run of 8x6x5 cells, 127 so
+    std::vector<char> image;
+    std::vector<std::pair<void *, size_t>> at;  // a table's pointer and its place
+    const auto put = [&](void *dst, const void *src, size_t bytes) {
+        at.emplace_back(dst, image.size());
+        image.insert(image.end(), (const char *)src, (const char *)src + bytes);
+        image.resize((image.size() + 255) / 256 * 256);
+    };
+    put(&c->d_abi, abi.data(), sizeof(int) * 2 * V);
+    put(&c->d_nface, nface.data(), sizeof(int) * V);
+    put(&c->d_facex, facex.data(), sizeof(int) * 2 * V * deg);
+    put(&c->d_oface, oface.data(), sizeof(int) * 2 * V * deg);
+    put(&c->d_ow, ow.data(), sizeof(double) * V * deg);
+    put(&c->d_nfwd, nfwd.data(), sizeof(int) * V);
+    put(&c->d_w32, w32.data(), sizeof(float) * V * deg);
+    put(&c->d_w64, w64.data(), sizeof(double) * V * deg);
+    put(&c->d_wsum32, wsum32.data(), sizeof(float) * V);
+    put(&c->d_wsum64, wsum64.data(), sizeof(double) * V);
+    put(&c->d_pos32, pos32.data(), sizeof(float) * 3 * V);
+    put(&c->d_pos64, pos64.data(), sizeof(double) * 3 * V);
+    put(&c->d_dv, dv.data(), sizeof(double) * V);
+    const size_t scalar_bytes = sizeof(double) * 64, red_bytes = sizeof(double) * FIN_SCRATCH;
+    if (!rc && device_malloc((void **)&c->d_tables, image.size() + scalar_bytes + red_bytes, c->device) != hipSuccess)
+        rc = GPE_ENOMEM;
+    if (!rc) {
+        for (const auto &t : at) {
+            const void *p = c->d_tables + t.second;
+            std::memcpy(t.first, &p, sizeof p);
+        }
+        c->d_scalars = (double *)(c->d_tables + image.size());
+        c->d_red = c->d_scalars + 64;
+        e = hipMemcpy(c->d_tables, image.data(), image.size(), hipMemcpyHostToDevice);
+        if (e != hipSuccess) rc = hip_fail(c, e, "hipMemcpy tables");
+    }
     if (!rc && device_malloc((void **)&c->d_partials, partials_bytes(c), c->device) != hipSuccess) rc = GPE_ENOMEM;
     if (!rc && hipHostMalloc((void **)&c->h_red, sizeof(double) * FIN_WIDTH_MAX, hipHostMallocDefault) != hipSuccess)
         rc = GPE_ENOMEM;
-    if (!rc && device_malloc((void **)&c->d_scalars, sizeof(double) * 64, c->device) != hipSuccess) rc = GPE_ENOMEM;
-    if (!rc && device_malloc((void **)&c->d_red, sizeof(double) * FIN_SCRATCH, c->device) != hipSuccess) rc = GPE_ENOMEM;
-    if (!rc) rc = ensure_fields(c, 1024);
     if (!rc && (e = hipEventCreate(&c->ev0)) != hipSuccess) rc = hip_fail(c, e, "hipEventCreate");
     if (!rc && (e = hipEventCreate(&c->ev1)) != hipSuccess) rc = hip_fail(c, e, "hipEventCreate");
     if (!rc && (e = hipStreamSynchronize(c->stream)) != hipSuccess) rc = hip_fail(c, e, "create sync");
@@ -899,8 +910,7 @@ int gpe_destroy(gpe_ctx *c)
     }
     for (int l = 0; l < 2; ++l)
         if (c->level[l]) (void)hipFree(c->level[l]);
-    void *ptrs[] = {c->d_abi, c->d_nface, c->d_facex, c->d_oface, c->d_ow, c->d_nfwd, c->d_w32, c->d_w64, c->d_wsum32, c->d_wsum64, c->d_pos32,
-                    c->d_pos64, c->d_dv, c->d_fields, c->d_partials, c->d_scalars, c->d_red};
+    void *ptrs[] = {c->d_tables, c->d_fields, c->d_partials};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_fields) (void)hipHostFree(c->h_fields);

@@ -151,3 +151,13 @@ def test_adjoint_reports_the_levels_of_its_longest_segment(stand_in, nsweeps, ev
         level = 8 * 3 * 8 * 6 * 5 * 12  # bytes: FP32 spinors of 8x6x5 cells of 12 (whole lines, no padding)
         assert r["segment_bytes"] == levels * level
         assert r["checkpoint_bytes"] == 2 * -(-nsweeps // every) * level
+
+
+def test_a_context_is_made_with_few_runtime_calls(stand_in):  # noqa: F811
+    """Two levels, one block of tables and results, the partials; one pinned buffer; one copy: an
+    ensemble or a parameter study pays for each of them per member."""
+    before = stand_in.counts()
+    with gpe.Stepper(gpe.Config.centred_box("bcc", (8, 6, 5), 0.7, ncomp=3, precision=gpe.FP64, dt=1e-4)):
+        after = stand_in.counts()
+    assert {k: after[k] - before[k] for k in ("allocs", "host_allocs", "copies")} == dict(allocs=4, host_allocs=1, copies=1)
+    assert stand_in.counts()["used"] == before["used"]
