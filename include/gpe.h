@@ -280,7 +280,7 @@ int gpe_traversal(const gpe_ctx *ctx, int *tile_rows, int *xcd_remap, int *x_per
  * 32 bits of n m).  No counterpart in the reference, whose
  * launch shape is fixed (Spin1GpeBCC.cu:1376-1380).  With x_per_lane 1 the plan is the launch
  * of one row per wave; the FP64 sweeps of lines that leave lanes idle that way walk the same
- * tiles with the rows of a tile packed into whole waves. */
+ * tiles with the rows of a tile packed into whole waves (gpe_plan_sweep). */
 typedef struct {
     int nx, ny, nz, V, C;
     int x_per_lane, rows, pairs, nseg, tile_rows, row_groups, ntile, xcd_remap;
@@ -295,6 +295,10 @@ typedef struct {
     long long ys, vs, cs, zs;
 } gpe_traversal_plan;
 int gpe_plan_traversal(const gpe_config *cfg, int tile_rows, int xcd_remap, int x_per_lane, gpe_traversal_plan *out);
+/* The launch that a sweep really makes, packed FP64 rows included (rows > 1 with x_per_lane 1: a slot
+ * of the group is one x value, and `pairs` = nx of them make a row).  tile_rows 0: the launch of a
+ * context that was not tuned; the other two arguments do not count then. */
+int gpe_plan_sweep(const gpe_config *cfg, int tile_rows, int xcd_remap, int x_per_lane, gpe_traversal_plan *out);
 
 /* Achievable HBM rate on the current device, from streaming kernels over two buffers of
  * `bytes` each (16-byte non-temporal accesses), averaged over `reps` launches: a copy

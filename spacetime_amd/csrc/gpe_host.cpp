@@ -598,6 +598,16 @@ Geometry base_geometry(const gpe_config &cfg)
     return g;
 }
 
+// The same of an untuned sweep: its x values per lane and tile height.
+Geometry untuned_geometry(const gpe_config &cfg)
+{
+    Geometry g = base_geometry(cfg);
+    const int fp64 = cfg.precision == GPE_FP64;
+    g.xpl = default_xpl(fp64, g.deg, cfg.ncomp, cfg.nx);
+    g.ty = default_tile(g, fp64 ? 16 : 8, fp64);
+    return g;
+}
+
 // Arguments of one sweep at time t of the run.
 SweepArgs sweep_args(gpe_ctx *c, double t, const void *cur, void *next, double coef)
 {
@@ -737,9 +747,7 @@ int gpe_create(const gpe_config *cfg, gpe_ctx **out)
 
     Geometry &g = c->g;
     g = base_geometry(*cfg);
-    c->gs = g;
-    c->gs.xpl = default_xpl(c->fp64, g.deg, cfg->ncomp, cfg->nx);
-    c->gs.ty = default_tile(c->gs, c->elem_bytes, c->fp64);
+    c->gs = untuned_geometry(*cfg);
     if (!finish_geometry(g) || !finish_geometry(c->gs, c->fp64)) {
         delete c;
         return GPE_EINVAL;
@@ -2082,21 +2090,18 @@ int gpe_traversal(const gpe_ctx *c, int *tile_rows, int *xcd_remap, int *x_per_l
     return GPE_OK;
 }
 
-int gpe_plan_traversal(const gpe_config *cfg, int tile_rows, int xcd_remap, int x_per_lane, gpe_traversal_plan *out)
+static bool plan_arguments_ok(const gpe_config *cfg, int tile_rows, int xcd_remap, int x_per_lane, gpe_traversal_plan *out)
 {
-    if (!cfg || !out) return GPE_EINVAL;
-    if (cfg->lattice < 0 || cfg->lattice > 5 || (cfg->ncomp != 1 && cfg->ncomp != 3 && cfg->ncomp != 5)) return GPE_EINVAL;
-    if (cfg->precision != GPE_FP32 && cfg->precision != GPE_FP64) return GPE_EINVAL;
-    if (cfg->nx < 1 || cfg->ny < 1 || cfg->nz < 1) return GPE_EINVAL;
-    if (tile_rows < 1 || tile_rows > 1024 || xcd_remap < 0 || xcd_remap > 3 || (x_per_lane != 1 && x_per_lane != 2))
-        return GPE_EINVAL;
-    Geometry g = base_geometry(*cfg);
-    if (x_per_lane == 2 && !pair_lanes_ok(cfg->precision == GPE_FP64, g.deg, cfg->ncomp)) return GPE_EINVAL;
-    g.ty = tile_rows;
-    g.xcd_remap = xcd_remap & 1;
-    g.v_inner = (xcd_remap >> 1) & 1;
-    g.xpl = x_per_lane;
-    if (!finish_geometry(g)) return GPE_EINVAL;
+    if (!cfg || !out) return false;
+    if (cfg->lattice < 0 || cfg->lattice > 5 || (cfg->ncomp != 1 && cfg->ncomp != 3 && cfg->ncomp != 5)) return false;
+    if (cfg->precision != GPE_FP32 && cfg->precision != GPE_FP64) return false;
+    if (cfg->nx < 1 || cfg->ny < 1 || cfg->nz < 1) return false;
+    if (tile_rows < 1 || tile_rows > 1024 || xcd_remap < 0 || xcd_remap > 3) return false;
+    return x_per_lane == 1 || (x_per_lane == 2 && pair_lanes_ok(cfg->precision == GPE_FP64, kLattices[cfg->lattice].deg, cfg->ncomp));
+}
+
+static void write_plan(const Geometry &g, gpe_traversal_plan *out)
+{
     out->nx = g.nx;
     out->ny = g.ny;
     out->nz = g.nz;
@@ -2125,6 +2130,36 @@ int gpe_plan_traversal(const gpe_config *cfg, int tile_rows, int xcd_remap, int 
         o[k][1] = d[k]->m;
         o[k][2] = d[k]->l;
     }
+}
+
+static int plan(const gpe_config *cfg, int tile_rows, int xcd_remap, int x_per_lane, bool pack, gpe_traversal_plan *out)
+{
+    Geometry g = base_geometry(*cfg);
+    g.ty = tile_rows;
+    g.xcd_remap = xcd_remap & 1;
+    g.v_inner = (xcd_remap >> 1) & 1;
+    g.xpl = x_per_lane;
+    if (!finish_geometry(g, pack)) return GPE_EINVAL;
+    write_plan(g, out);
+    return GPE_OK;
+}
+
+int gpe_plan_traversal(const gpe_config *cfg, int tile_rows, int xcd_remap, int x_per_lane, gpe_traversal_plan *out)
+{
+    if (!plan_arguments_ok(cfg, tile_rows, xcd_remap, x_per_lane, out)) return GPE_EINVAL;
+    return plan(cfg, tile_rows, xcd_remap, x_per_lane, false, out);
+}
+
+int gpe_plan_sweep(const gpe_config *cfg, int tile_rows, int xcd_remap, int x_per_lane, gpe_traversal_plan *out)
+{
+    const bool untuned = tile_rows == 0;
+    if (!plan_arguments_ok(cfg, untuned ? 1 : tile_rows, untuned ? 0 : xcd_remap, untuned ? 1 : x_per_lane, out))
+        return GPE_EINVAL;
+    const int fp64 = cfg->precision == GPE_FP64;
+    if (!untuned) return plan(cfg, tile_rows, xcd_remap, x_per_lane, fp64, out);
+    Geometry g = untuned_geometry(*cfg);
+    if (!finish_geometry(g, fp64)) return GPE_EINVAL;
+    write_plan(g, out);
     return GPE_OK;
 }
 
@@ -2180,9 +2215,8 @@ int gpe_autotune(gpe_ctx *c, int trial_sweeps, int *tile_rows, int *xcd_remap, i
         // spin-1 99% and 74%, A15 9x11x9 86% and 43%, FP64 FCC 17^3 90% and 50%)
         std::vector<int> tys = {1, 2, 4, 8, 16, 32, 3, 6, 12, 24, 5, 10, 20, 7, 14, 28};
         if (c->g.ny > 32 && c->g.ny <= 1024) tys.push_back(c->g.ny);
-        Geometry untuned = base_geometry(c->cfg);
-        untuned.xpl = default_xpl(c->fp64, untuned.deg, c->cfg.ncomp, c->cfg.nx);
-        const int untuned_ty = default_tile(untuned, c->elem_bytes, c->fp64);
+        const Geometry untuned = untuned_geometry(c->cfg);
+        const int untuned_ty = untuned.ty;
         tys.erase(std::remove(tys.begin(), tys.end(), untuned_ty), tys.end());
         tys.insert(tys.begin(), untuned_ty);
         const int nxpl = pair_lanes_ok(c->fp64, c->g.deg, c->cfg.ncomp) ? 2 : 1;

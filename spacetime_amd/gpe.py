@@ -134,7 +134,8 @@ def load_library(path=LIB_PATH):
                                  ctypes.POINTER(ctypes.c_int), _dp]
     lib.gpe_set_trap.argtypes = [vp, _dp]
     lib.gpe_stream_bandwidth.argtypes = [ctypes.c_longlong, ctypes.c_int, _dp, _dp]
-    lib.gpe_plan_traversal.argtypes = [ctypes.POINTER(_Config), ctypes.c_int, ctypes.c_int, ctypes.c_int,
+    for name in ("gpe_plan_traversal", "gpe_plan_sweep"):
+        getattr(lib, name).argtypes = [ctypes.POINTER(_Config), ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                        ctypes.POINTER(_Plan)]
     lib.gpe_set_traversal.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     lib.gpe_traversal.argtypes = [vp, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int),
