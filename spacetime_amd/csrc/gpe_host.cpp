@@ -522,7 +522,9 @@ int default_tile(const Geometry &g0, int elem_bytes, bool pack)
 // 3% of the most values (57-value lines, 57 rows: 19 rows 99% against 8 rows 87%, and one row
 // a wave 89%; 16-value lines one row a wave 25%).  A wave takes a chunk of the group's segments:
 // all of them where the groups alone give every wave of the launch one, fewer in smaller boxes.
-// Needs a finished g; its waves are never more than g's.
+// Needs a finished g.  Its groups are never more than g's waves, and where they are split into chunks there
+// are at most 4 blocks of these (more than g's waves in some small boxes: 57x11 rows of a plane 18 for
+// 16), so wave indices stay below 2^31 where g's do.
 Geometry reduce_geometry(const Geometry &g, int blocks, int *segs)
 {
     Geometry r = g;
