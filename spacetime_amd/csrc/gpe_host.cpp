@@ -291,7 +291,6 @@ double sweep_dt(const gpe_ctx *c) { return c->cfg.scheme == GPE_SCHEME_STAGGERED
 FieldRec field_at(const gpe_ctx *c, double t)
 {
     FieldRec f{};
-    f.t = t;
     f.trap_on = t < c->ph.trap_off_time;
     f.sigma = 1.0;
     if (c->cfg.expansion_rate != 0.0 && t > c->cfg.expansion_start)

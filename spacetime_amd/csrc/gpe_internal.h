@@ -133,11 +133,10 @@ struct Physics {
 struct FieldRec {
     int trap_on;          // t is before the trap's end
     // FP32 copies for the FP32 sweep: sigma, 1 / sigma^2, bq, bb[3], bqq, bbq[3]
-    float fsigma, fksc, pad;
+    float fsigma, fksc;
     double sigma;         // block-scale factor of the expanding grid (1: static)
     float fbq, fbb[3], fbqq, fbbq[3];
-    double t;
-    double bq, bb[3];
+    double bq, bb[3];  // in a sweep's arguments these eight start a line
     double bqq, bbq[3];
 };
 
@@ -162,6 +161,8 @@ struct SweepArgs {
 // The level pointers, which a wave's first loads wait for, and coef lie on one line of the arguments
 // (over two: Cube 75x61x90 5.05 us a sweep, 4.94 so).
 static_assert(offsetof(SweepArgs, cur) % 64 == 0, "level pointers start a line");
+
+static_assert((offsetof(SweepArgs, field) + offsetof(FieldRec, bq)) % 64 == 0, "FP64 fields start a line");
 
 // Observables partial sums per workgroup.
 enum {
