@@ -287,7 +287,8 @@ typedef struct {
     long long lx, waves;
     int blocks;
     unsigned div_nseg[3], div_V[3], div_rows[3], div_nz[3], div_pairs[3]; /* d, m, l */
-    /* level layout: element (z, y, v, c, x) at z zs + y ys + v vs + c cs + x; slabs = 1 when
+    /* level layout: element (z, y, v, c, x) at z zs + y ys + v vs + c cs + x, v the unknown's place
+     * on the device (a permutation of the ABI's v on lattices with rings of four); slabs = 1 when
      * the rows of one (z, v, c) are contiguous (FP32 lines whose even length is not a whole
      * number of 128-byte lines; lx = that even length), 0 when the C components of one
      * (z, y, v) are adjacent x-lines */
