@@ -262,16 +262,13 @@ __device__ __forceinline__ void adj_sens32(const float *pr, const float *pi, con
 // One x value per lane (FP64, and FP32 where the pair form is not chosen): the forward sweep's
 // single body on mu_{k+1} -- interior fast path through the per-face line offsets, wave-uniform
 // weights on same-x faces, zero-weight pad faces skipped.
-template <typename R, int C, int DEG, bool ROWS, int NIN>
+template <typename R, int C, int DEG, bool ROWS>
 __device__ __forceinline__ void adjoint_single(const AdjArgs &a, int b, int nb, double *part)
 {
     using V2 = vec2_t<R>;
     const Geometry &g = a.g;
     const LaneCoord lc = lane_coord<ROWS>(g, b, nb);
-    if (!lc.valid) {
-        if constexpr (NIN > 0) exchange_barrier();
-        return;
-    }
+    if (!lc.valid) return;
     const int x = lc.x, v = lc.v, y = lc.y, z = lc.z;
     const bool act = lc.act;
     const int xc = lc.at;  // the lane's offset from the line of row y0
@@ -311,44 +308,25 @@ __device__ __forceinline__ void adjoint_single(const AdjArgs &a, int b, int nb, 
     const V2 *nbase[DEG];
     face_lanes<R, DEG, ROWS>(g, lc, mu1 + own_line, face, fd, wt, wu, xok, dxf, nbase, noff);
     const int nf = DEG == 8 ? a.tb.nface[v] : DEG;
-    V2 nbv[DEG - NIN][C];
+    V2 nbv[DEG][C];
 #pragma unroll
-    for (int f = NIN; f < DEG; ++f)
+    for (int f = 0; f < DEG; ++f)
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             if (f < nf) {
-                nbv[f - NIN][c] = nbase[f][c * cstride + noff[f]];
+                nbv[f][c] = nbase[f][c * cstride + noff[f]];
             } else {
-                nbv[f - NIN][c].x = 0;
-                nbv[f - NIN][c].y = 0;
+                nbv[f][c].x = 0;
+                nbv[f][c].y = 0;
             }
         }
-    if constexpr (NIN > 0) {
-        __shared__ V2 ex[4][C][64];
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            V2 o;
-            o.x = mr[c];
-            o.y = mi[c];
-            ex[threadIdx.x >> 6][c][threadIdx.x & 63] = o;
-        }
-        exchange_barrier();
-#pragma unroll
-        for (int f = 0; f < NIN; ++f)
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                const V2 o = ex[exchange_wave(f)][c][threadIdx.x & 63];
-                ar[c] += wt[f] * o.x;
-                ai[c] += wt[f] * o.y;
-            }
-    }
-#pragma unroll
-    for (int f = NIN; f < DEG; ++f) {
+    for (int f = 0; f < DEG; ++f) {
         const R w = (dxf[f] == 0 || xok[f]) ? wu[f] : (R)0;
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            ar[c] += w * nbv[f - NIN][c].x;
-            ai[c] += w * nbv[f - NIN][c].y;
+            ar[c] += w * nbv[f][c].x;
+            ai[c] += w * nbv[f][c].y;
         }
     }
     const R wsum = table_wsum<R>(a.tb)[v];
@@ -391,7 +369,7 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));
 // into the line and shifted back; every neighbour value outside the box is replaced by zero with
 // a select, so line padding is never used as a value.  The lone last x of an odd-length line
 // writes its partner slot, which is line padding.
-template <int C, int DEG, bool ROWS, int NIN>
+template <int C, int DEG, bool ROWS>
 __device__ __forceinline__ void adjoint_pair(const AdjArgs &a, int b, int nb, double *part)
 {
     const Geometry &g = a.g;
@@ -404,10 +382,7 @@ __device__ __forceinline__ void adjoint_pair(const AdjArgs &a, int b, int nb, do
         const WaveCoord wc = decode(g, b, nb);
         x0 = wc.x, v = wc.v, y0 = wc.y, z = wc.z, valid = wc.valid;
     }
-    if (!valid) {
-        if constexpr (NIN > 0) exchange_barrier();
-        return;
-    }
+    if (!valid) return;
     bool rowok = true;
     int y = y0, roff = 0;
     const int rowstride = (int)g.ys;
@@ -503,48 +478,24 @@ __device__ __forceinline__ void adjoint_pair(const AdjArgs &a, int b, int nb, do
 #pragma unroll
     for (int f0 = 0; f0 < DEG; f0 += FB) {
         if (f0 > 0 && f0 >= nf) break;
-        f4u nbv[FB - NIN][C];
+        f4u nbv[FB][C];
 #pragma unroll
-        for (int kk = NIN; kk < FB; ++kk)
+        for (int kk = 0; kk < FB; ++kk)
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 if (f0 + kk < nf)
-                    nbv[kk - NIN][c] = *(const f4u *)(nbase[f0 + kk] + c * cstride);
+                    nbv[kk][c] = *(const f4u *)(nbase[f0 + kk] + c * cstride);
                 else
-                    nbv[kk - NIN][c] = (f4u)(0.f);
+                    nbv[kk][c] = (f4u)(0.f);
             }
-        if constexpr (NIN > 0) {
-            static_assert(NIN == 0 || FB == DEG, "one batch");
-            __shared__ f4a ex[4][C][64];
 #pragma unroll
-            for (int c = 0; c < C; ++c) {
-                f4a o;
-                o.x = mr[0][c];
-                o.y = mi[0][c];
-                o.z = mr[1][c];
-                o.w = mi[1][c];
-                ex[threadIdx.x >> 6][c][threadIdx.x & 63] = o;
-            }
-            exchange_barrier();
-#pragma unroll
-            for (int f = 0; f < NIN; ++f)
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    const f4a e = ex[exchange_wave(f)][c][threadIdx.x & 63];
-                    ar[0][c] += wt[f] * e.x;
-                    ai[0][c] += wt[f] * e.y;
-                    ar[1][c] += wt[f] * e.z;
-                    ai[1][c] += wt[f] * e.w;
-                }
-        }
-#pragma unroll
-        for (int kk = NIN; kk < FB; ++kk) {
+        for (int kk = 0; kk < FB; ++kk) {
             const int f = f0 + kk;
             const float w = wf[f];
             if (dxf[f] == 0) {
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
-                    const f4u e = nbv[kk - NIN][c];
+                    const f4u e = nbv[kk][c];
                     ar[0][c] += w * e.x;
                     ai[0][c] += w * e.y;
                     ar[1][c] += w * e.z;
@@ -553,7 +504,7 @@ __device__ __forceinline__ void adjoint_pair(const AdjArgs &a, int b, int nb, do
             } else {
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
-                    const f4u e = nbv[kk - NIN][c];
+                    const f4u e = nbv[kk][c];
                     float n0r = sh[f] == 0 ? e.x : e.z, n0i = sh[f] == 0 ? e.y : e.w;
                     float n1r = sh[f] == 0 ? e.z : e.x, n1i = sh[f] == 0 ? e.w : e.y;
                     n0r = (ok0[f] && sh[f] >= 0) ? n0r : 0.f;
@@ -629,8 +580,11 @@ __device__ __forceinline__ void adjoint_pair(const AdjArgs &a, int b, int nb, do
 
 // Adjoint sweep mu_{k+2} -> mu_k = mu_{k+2} + coef G'(psi_k)^T mu_{k+1} over the sweep traversal
 // (X: the lane form of gpe_internal.h), with the FP64 parameter sensitivities of the workgroup's
-// unknowns summed into partials[b].
-template <typename R, int C, int DEG, int X, int NIN>
+// unknowns summed into partials[b].  The forward sweep's exchange between the waves of a workgroup
+// loses here: FP32 spin-2 keeps three waves a SIMD without it and two with it (165 and 173 registers), and
+// the four waves of spin-1 hide its barrier worse than the forward sweep's.  us a sweep, with -> without:
+// BCC 64^3 spin-1 FP32 57.5 -> 54.0, FP64 113.7 -> 104.4; 48^3 spin-2 FP32 51.7 -> 44.8.
+template <typename R, int C, int DEG, int X>
 __global__ __launch_bounds__(256) void k_adjoint(AdjArgs a)
 {
     const int b = sweep_order(a.g, blockIdx.x, gridDim.x, a.order);
@@ -638,9 +592,9 @@ __global__ __launch_bounds__(256) void k_adjoint(AdjArgs a)
 #pragma unroll
     for (int i = 0; i < ADJ_COUNT; ++i) part[i] = 0.0;
     if constexpr (X == 1 || X == 4)
-        adjoint_single<R, C, DEG, X == 4, NIN>(a, b, gridDim.x, part);
+        adjoint_single<R, C, DEG, X == 4>(a, b, gridDim.x, part);
     else
-        adjoint_pair<C, DEG, X == 3, NIN>(a, b, gridDim.x, part);
+        adjoint_pair<C, DEG, X == 3>(a, b, gridDim.x, part);
     __shared__ double red[4][ADJ_COUNT];
     wave_sum_n<ADJ_COUNT>(part);
     if ((threadIdx.x & 63) == 0) {
@@ -757,16 +711,9 @@ __global__ __launch_bounds__(256) void k_objective(ObjArgs a)
 }
 
 template <typename R, int C, int DEG, int X>
-static hipError_t adj_n(const AdjArgs &a, hipStream_t s)
+static hipError_t adj_x(const AdjArgs &a, hipStream_t s)
 {
-    dim3 grid(a.g.blocks), block(256);
-    if constexpr (exchange_ok(DEG, C)) {
-        if (a.g.exchange) {
-            hipLaunchKernelGGL((k_adjoint<R, C, DEG, X, 2>), grid, block, 0, s, a);
-            return hipGetLastError();
-        }
-    }
-    hipLaunchKernelGGL((k_adjoint<R, C, DEG, X, 0>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_adjoint<R, C, DEG, X>), dim3(a.g.blocks), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -774,12 +721,12 @@ template <typename R, int C, int DEG>
 static hipError_t adj_form(const AdjArgs &a, hipStream_t s)
 {
     const int form = lane_form(a.g.xpl, a.g.rows);
-    if (form == 1) return adj_n<R, C, DEG, 1>(a, s);
+    if (form == 1) return adj_x<R, C, DEG, 1>(a, s);
     if constexpr (std::is_same<R, double>::value) {
-        if (form == 4) return adj_n<R, C, DEG, 4>(a, s);
+        if (form == 4) return adj_x<R, C, DEG, 4>(a, s);
     }
     if constexpr (pair_lanes_ok(std::is_same<R, double>::value, DEG, C)) {
-        return form == 2 ? adj_n<R, C, DEG, 2>(a, s) : adj_n<R, C, DEG, 3>(a, s);
+        return form == 2 ? adj_x<R, C, DEG, 2>(a, s) : adj_x<R, C, DEG, 3>(a, s);
     }
     return hipErrorInvalidValue;
 }

@@ -1,4 +1,6 @@
 """The adjoint's kept workspace on the device: given back on request, and the next call the same."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -10,13 +12,13 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("fp64", [False, True])
 def test_release_gives_the_memory_back_and_changes_no_bit(fp64):
-    import torch
     cfg = gpe.Config.centred_box("bcc", (40, 40, 40), 0.6, ncomp=3, precision=gpe.FP32, dt=2e-4, c0=60.0, c1=8.0, q=0.1)
     psi0, target = random_state(cfg.shape, 1), random_state(cfg.shape, 2)
 
     def free():
-        torch.cuda.synchronize()
-        return torch.cuda.mem_get_info()[0]
+        avail, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert gpe.load_library().hipMemGetInfo(ctypes.byref(avail), ctypes.byref(total)) == 0  # the runtime it links
+        return avail.value
 
     def run(st):
         st.set_state(psi0)
