@@ -418,20 +418,31 @@ static double lane_use(int rows, int pairs)
     return (double)slots / (64.0 * ((slots + 63) / 64));
 }
 
-// pack (FP64 sweeps, one x per lane): the rows of a tile are one group where one row per wave leaves
-// lanes idle that packed rows would fill.  Where lines are whole 128-byte lines, from 5% of the
-// lanes; otherwise a wave then starts inside cache lines that its neighbour also touches, which
-// costs more than the lanes unless more than half of them idle or the box is small.  us a sweep, one
-// row -> packed: whole lines BCC 40^3 one component 9.9 -> 7.8, FCC 40^3 spin-1 29.0 -> 24.4, C15 24^3
-// spin-2 115 -> 86, A15 48^3 147 -> 137; others C15 20^3 (31% of the lanes) 54.3 -> 40.7, A15 30^3
-// (47%) 71 -> 66, Cube 75x61x90 8.7 -> 6.4, but Z 34^3 spin-2 (53%) 184 -> 196, Z 50^3 105 -> 114, A15 39^3
-// 81 -> 84.  Full lines keep one row.
+// pack (FP64 sweeps, one x per lane): whether the rows of a tile are one group instead of one row per
+// wave.  It gains lanes, and it costs:
+//   * rows of whole 128-byte lines (8 values) start waves on them, others inside lines that the
+//     neighbouring wave touches too: spinors of large cells have the most of these;
+//   * a box of one tile has no group whose y neighbours are all inside, and a Cube of fewer than 2 waves
+//     a SIMD wants the waves rather than the lanes;
+//   * the unknowns of a cell now meet a tile of rows apart, which has to stay in an XCD's 4 MiB L2 (C15
+//     spin-2 of 200 values, 17 MB: 0.84 of one row's speed, 104 values, 9 MB: 0.94).
+// Measured at 8 rows a tile over 1016 boxes (six lattices, 1, 3 and 5 components, 14-200 values a line,
+// 8.7e4-7e6 unknowns): packed always 1.044 times the speed of one row a wave in the mean, 385 boxes of
+// them slower (to 0.64); by this rule 1.083 and 7 (to 0.94); by the best choice for each 1.087.
+constexpr double PACK_BYTES = 5.3e6;
+
+// Times the lanes of one row a wave that packing has to fill to pay.
+double pack_pays(const Geometry &g)
+{
+    const bool few = g.V == 1 && (long long)g.ny * g.nz * ((g.nx + 63) / 64) < 2000;
+    if (g.ny <= g.ty || few) return 1.9;
+    return g.nx % 8 == 0 ? 1.2 : (g.V > 12 && g.C > 1 ? 1.9 : 1.5);
+}
+
 bool pack_rows(const Geometry &g)
 {
-    const double one = lane_use(1, g.nx);
-    if (g.ty < 2 || lane_use(g.ty, g.nx) < one + 0.05) return false;
-    const long long waves = (long long)g.ny * g.nz * g.V * ((g.nx + 63) / 64);
-    return g.lx % 8 == 0 || one < 0.5 || waves <= 16384;
+    return g.ty > 1 && lane_use(g.ty, g.nx) >= pack_pays(g) * lane_use(1, g.nx) &&
+           16.0 * g.V * g.C * g.ty * g.lx <= PACK_BYTES;
 }
 
 // Segments, tiles, waves and workgroups of a traversal from nx, ny, nz, V, ty and xpl.
@@ -491,6 +502,8 @@ bool finish_geometry(Geometry &g, bool pack = false)
 // of the lanes in tiles of 8, 78% in one tile; FCC 19^3 49% and 99%).  Taller tiles have to keep
 // a plane's rows in an XCD's L2 with room for its neighbours (TILE_BYTES: C15 57^3 spin-2 588 us
 // at 8 rows, 700 at 24), and large cells' tiles to start on 128-byte boundaries (A15 41^3 49 -> 51).
+// FP64 boxes of 14-104 values a line (520 of them): 1.17 times the speed of one row a wave in tiles of 8, where the
+// best of ten heights for each would give 1.21.
 constexpr double TILE_BYTES = 2.6e6;
 
 int default_tile(const Geometry &g0, int elem_bytes, bool pack)
@@ -500,7 +513,8 @@ int default_tile(const Geometry &g0, int elem_bytes, bool pack)
         g.ty = ty;
         if (!finish_geometry(g, pack)) return 0.0;
         const int slots = g.xpl == 2 ? g.pairs : g.nx;
-        return (double)g.ny * slots / (64.0 * g.ntile * g.tyr * g.nseg);
+        const double lanes = (double)g.ny * slots / (64.0 * g.ntile * g.tyr * g.nseg);
+        return pack && g.rows > 1 ? lanes / 1.3 : lanes;  // packed lanes are worth less, in the mean by that
     };
     const int lo = std::min(8, g0.ny), hi = std::min(32, g0.ny);
     int ty = lo;

@@ -93,3 +93,25 @@ def test_bad_plans_are_refused():
     for bad in ((-1, 1, 1), (1025, 1, 1), (8, 4, 1), (8, 1, 2), (8, 1, 0)):
         assert plan(cfg, *bad)[0] == -22
     assert plan(gpe.Config(lattice="bcc", dims=(0, 8, 8)))[0] == -22
+
+
+@pytest.mark.parametrize("lat,ncomp,dims,rows", [
+    # packed rows were slower than one row a wave here (times of one row's speed)
+    ("bcc", 1, (46, 113, 112), 1),   # 0.90: 46 values in lines of 48
+    ("fcc", 1, (56, 102, 102), 1),   # 0.92: 7 of 8 lanes full without
+    ("cube", 3, (110, 192, 191), 1), # 0.96
+    ("cube", 5, (75, 30, 30), 1),    # 0.92: 1800 waves
+    ("c15", 5, (200, 11, 10), 1),    # 0.84: 17 MB between the unknowns of a cell
+    ("a15", 3, (34, 8, 7), 1),       # 0.93: one tile
+    ("z", 5, (34, 13, 13), 1),       # 0.96
+    # and faster here
+    ("fcc", 5, (40, 81, 81), 8),     # 1.18
+    ("bcc", 3, (70, 69, 70), 8),     # 1.24
+    ("c15", 1, (70, 27, 27), 8),     # 1.13
+    ("cube", 1, (40, 418, 419), 8),  # 1.17
+    ("a15", 5, (88, 28, 28), 8),     # 1.05
+    ("z", 3, (20, 20, 20), 8)])
+def test_rows_are_packed_where_that_was_faster(lat, ncomp, dims, rows):
+    cfg = gpe.Config(lattice=lat, ncomp=ncomp, precision=gpe.FP64, dims=dims)
+    rc, p = plan(cfg, 8, 1, 1)
+    assert rc == 0 and p.rows == rows
