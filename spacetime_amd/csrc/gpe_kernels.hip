@@ -1493,9 +1493,7 @@ __global__ __launch_bounds__(256) void k_pack(Geometry g, const int *__restrict_
     }
 }
 
-// One ABI value a thread: cells of one unknown, whose two sides are runs of lines already (Cube 150^3 FP64
-// in 30 us through LDS, 26 so), and FP64 levels of small cells that the caches hold, on the way in (BCC
-// 48^3 spin-1 35 us through LDS, 31 so; 96^3 210 and 247).
+// One ABI value a thread (pack_direct): no table, no barrier between a value's load and its store.
 template <typename R, bool PACK>
 __global__ __launch_bounds__(256) void k_pack_values(Geometry g, const int *__restrict__ place, const double2 *__restrict__ abi_in,
                                                      double2 *__restrict__ abi_out, const vec2_t<R> *__restrict__ dev_in,
@@ -1793,6 +1791,21 @@ hipError_t launch_phase_copy(int fp64, const void *src, void *dst, long long nel
     return hipGetLastError();
 }
 
+// Where one ABI value a thread is faster than the turn in LDS.  us a call of the smallest and of larger levels,
+// through LDS and direct:
+//   * cells of one unknown, whose two sides are runs of lines already: Cube 150^3 FP64 in 30 and 26;
+//   * levels of few workgroups, whose time is one chain of latencies: C15 6x5x6 FP64 in 14.8 and 13.1, out
+//     15.1 and 12.9.  The lines meet at 2e5-3e5 values in and 4e5-6e5 out for every cell size;
+//   * on the way in, levels of smaller cells that the caches hold, where a line's pieces meet in L2: BCC 48^3
+//     spin-1 FP64 35 and 31, 96^3 210 and 247; of 1.6e6-7e6 values A15 FP64 4-8% slower through LDS, BCC
+//     FP32 1-4%; A15 FP32 9-14% faster, Z and C15 2-59% faster.
+template <typename R, bool PACK>
+static bool pack_direct(const Geometry &g, long long values)
+{
+    if (g.V == 1 || values < (PACK ? 1 << 18 : 1 << 19)) return true;
+    return PACK && values < (8 << 20) && g.V <= (sizeof(R) == 8 ? 46 : 12);
+}
+
 // Cells per workgroup: 64 (fewer where those of a large cell fill more than 24 KiB or a
 // small box has under 128 workgroups, but 16 cells), and more, in
 // a tile of up to 40 KiB, while there are workgroups enough to hide a tile's load before its store.
@@ -1804,7 +1817,7 @@ static hipError_t pack(const Geometry &g, const Tables &tb, int ncomp, const dou
 {
     const long long cells = (long long)g.nz * g.ny * g.nx;
     const long long values = cells * g.V;
-    if (g.V == 1 || (PACK && sizeof(R) == 8 && g.V <= 12 && ncomp * values < (8 << 20))) {
+    if (pack_direct<R, PACK>(g, ncomp * values)) {
         hipLaunchKernelGGL((k_pack_values<R, PACK>), dim3(grid1(values), (unsigned)ncomp), dim3(256), 0, s, g, tb.place,
                            (const double2 *)abi_in, (double2 *)abi_out, (const vec2_t<R> *)dev_in, (vec2_t<R> *)dev_out);
         return hipGetLastError();
