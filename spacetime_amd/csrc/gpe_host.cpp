@@ -1810,7 +1810,6 @@ int gpe_release_workspace(gpe_ctx *c)
 // Members sharing (face degree, x per lane) form a group launched by one specialised kernel.
 struct EnsembleGroup {
     int deg, form;      // face degree and lane_form of every member
-    int exchange;       // their Geometry::exchange
     int first, count;   // members [first, first + count) of the sorted member list
     int blocks;         // workgroups of the group's launch
 };
@@ -1871,11 +1870,9 @@ int gpe_ensemble_create(gpe_ctx *const *members, int n, gpe_ensemble **out)
         const gpe_ctx *c = e->m[i];
         const int form = lane_form(c->gs.xpl, c->gs.rows);
         const bool solo = c->gs.blocks >= ENS_SOLO_BLOCKS;
-        const int exchange = solo ? c->gs.exchange : 0;  // a launch shared with other lattices does without
         if (i == 0 || solo || prev_solo || c->gs.deg != e->groups.back().deg || form != e->groups.back().form ||
-            exchange != e->groups.back().exchange ||
             e->groups.back().count == ENS_GROUP_MAX) {
-            e->groups.push_back(EnsembleGroup{c->gs.deg, form, exchange, i, 0, 0});
+            e->groups.push_back(EnsembleGroup{c->gs.deg, form, i, 0, 0});
             begin = 0;
         }
         prev_solo = solo;
@@ -1979,7 +1976,7 @@ int gpe_ensemble_step(gpe_ensemble *e, int nsteps, int graph_sweeps)
         a.sweep = k;
         a.sweep_base = base;
         for (int i = 0; i < gr.count; ++i) a.begin[i] = e->span[gr.first + i].first;
-        return launch_ensemble_sweep(e->fp64, e->ncomp, gr.deg, gr.form, gr.exchange, a, gr.blocks, st);
+        return launch_ensemble_sweep(e->fp64, e->ncomp, gr.deg, gr.form, a, gr.blocks, st);
     };
     auto launch_all = [&](int k, const int *base) -> hipError_t {
         for (const EnsembleGroup &gr : e->groups) {

@@ -285,10 +285,10 @@ struct EnsembleArgs {
     int begin[ENS_GROUP_MAX]; // members[i].begin
 };
 
-// All members of one launch share the component count, precision, face degree, lanes and exchange.
+// All members of one launch share the component count, precision, face degree and lanes.
 // form: lane_form of the group's traversal
-hipError_t launch_ensemble_sweep(int fp64, int ncomp, int deg, int form, int exchange, const EnsembleArgs &e,
-                                 int blocks, hipStream_t s);
+hipError_t launch_ensemble_sweep(int fp64, int ncomp, int deg, int form, const EnsembleArgs &e, int blocks,
+                                 hipStream_t s);
 hipError_t launch_advance_base(int *base, int by, hipStream_t s);
 hipError_t launch_set_base(int *base, int value, hipStream_t s);
 

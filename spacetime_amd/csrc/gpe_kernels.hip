@@ -580,8 +580,11 @@ __global__ __launch_bounds__(256) void k_sweep(SweepArgs a)
 // members sharing component count, face degree and lanes per x, so the kernel is as
 // specialised as a single run's).  Member m owns workgroups [begin_m, begin_m + blocks_m)
 // (begin_m a multiple of 8, so the XCD remap of the member's own range stays valid); its
-// arguments for parity p are m.args[p].
-template <typename R, int C, int DEG, int X, int NIN>
+// arguments for parity p are m.args[p].  Without the exchange between waves that a single run's BCC
+// sweeps make: with the arguments in memory it takes 121 registers for 94 (4 waves a SIMD for 5).  us a
+// sweep of one of two members, with -> without: FP32 spin-1 128^3 335 -> 319, spin-2 96^3 251 -> 215, FP64
+// spin-1 96^3 308 -> 282, spin-2 64^3 130 either way.
+template <typename R, int C, int DEG, int X>
 __global__ __launch_bounds__(256) void k_ensemble_sweep(EnsembleArgs e)
 {
     // parity-1 sweeps take the whole launch in reverse (members included), keeping each
@@ -601,7 +604,7 @@ __global__ __launch_bounds__(256) void k_ensemble_sweep(EnsembleArgs e)
     const SweepArgs &a = m.args[e.parity];
     const int sweep = e.sweep + (e.sweep_base ? *e.sweep_base : 0);
     const auto field = [&]() { return (const_ptr<FieldRec>)(unsigned long long)(a.fields + sweep); };
-    sweep_body<R, C, DEG, MODE_UPDATE, X, NIN>(a, field, local, m.blocks);
+    sweep_body<R, C, DEG, MODE_UPDATE, X, 0>(a, field, local, m.blocks);
 }
 
 __global__ void k_advance_base(int *base, int by)
@@ -1640,60 +1643,53 @@ hipError_t launch_aux(int fp64, int ncomp, const AuxArgs &a, hipStream_t s)
 }
 
 template <typename R, int C, int DEG, int X>
-static hipError_t ens_n(int exchange, const EnsembleArgs &e, int blocks, hipStream_t s)
+static hipError_t ens_n(const EnsembleArgs &e, int blocks, hipStream_t s)
 {
-    dim3 grid(blocks), block(256);
-    if constexpr (exchange_ok(DEG, C)) {
-        if (exchange) {
-            hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, X, 2>), grid, block, 0, s, e);
-            return hipGetLastError();
-        }
-    }
-    hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, X, 0>), grid, block, 0, s, e);
+    hipLaunchKernelGGL((k_ensemble_sweep<R, C, DEG, X>), dim3(blocks), dim3(256), 0, s, e);
     return hipGetLastError();
 }
 
 template <typename R, int C, int DEG>
-static hipError_t ens_x(int form, int exchange, const EnsembleArgs &e, int blocks, hipStream_t s)
+static hipError_t ens_x(int form, const EnsembleArgs &e, int blocks, hipStream_t s)
 {
-    if (form == 1) return ens_n<R, C, DEG, 1>(exchange, e, blocks, s);
+    if (form == 1) return ens_n<R, C, DEG, 1>(e, blocks, s);
     if constexpr (std::is_same<R, double>::value) {
-        if (form == 4) return ens_n<R, C, DEG, 4>(exchange, e, blocks, s);
+        if (form == 4) return ens_n<R, C, DEG, 4>(e, blocks, s);
     }
     if constexpr (pair_lanes_ok(std::is_same<R, double>::value, DEG, C)) {
-        if (form == 2) return ens_n<R, C, DEG, 2>(exchange, e, blocks, s);
-        if (form == 3) return ens_n<R, C, DEG, 3>(exchange, e, blocks, s);
+        if (form == 2) return ens_n<R, C, DEG, 2>(e, blocks, s);
+        if (form == 3) return ens_n<R, C, DEG, 3>(e, blocks, s);
     }
     return hipErrorInvalidValue;
 }
 
 template <typename R, int C>
-static hipError_t ens_deg(int deg, int form, int exchange, const EnsembleArgs &e, int blocks, hipStream_t s)
+static hipError_t ens_deg(int deg, int form, const EnsembleArgs &e, int blocks, hipStream_t s)
 {
     switch (deg) {
-    case 4: return ens_x<R, C, 4>(form, exchange, e, blocks, s);
-    case 6: return ens_x<R, C, 6>(form, exchange, e, blocks, s);
-    case 8: return ens_x<R, C, 8>(form, exchange, e, blocks, s);
+    case 4: return ens_x<R, C, 4>(form, e, blocks, s);
+    case 6: return ens_x<R, C, 6>(form, e, blocks, s);
+    case 8: return ens_x<R, C, 8>(form, e, blocks, s);
     default: return hipErrorInvalidValue;
     }
 }
 
 template <typename R>
-static hipError_t ens_comp(int ncomp, int deg, int form, int exchange, const EnsembleArgs &e, int blocks, hipStream_t s)
+static hipError_t ens_comp(int ncomp, int deg, int form, const EnsembleArgs &e, int blocks, hipStream_t s)
 {
     switch (ncomp) {
-    case 1: return ens_deg<R, 1>(deg, form, exchange, e, blocks, s);
-    case 3: return ens_deg<R, 3>(deg, form, exchange, e, blocks, s);
-    case 5: return ens_deg<R, 5>(deg, form, exchange, e, blocks, s);
+    case 1: return ens_deg<R, 1>(deg, form, e, blocks, s);
+    case 3: return ens_deg<R, 3>(deg, form, e, blocks, s);
+    case 5: return ens_deg<R, 5>(deg, form, e, blocks, s);
     default: return hipErrorInvalidValue;
     }
 }
 
-hipError_t launch_ensemble_sweep(int fp64, int ncomp, int deg, int form, int exchange, const EnsembleArgs &e,
-                                 int blocks, hipStream_t s)
+hipError_t launch_ensemble_sweep(int fp64, int ncomp, int deg, int form, const EnsembleArgs &e, int blocks,
+                                 hipStream_t s)
 {
-    return fp64 ? ens_comp<double>(ncomp, deg, form, exchange, e, blocks, s)
-                : ens_comp<float>(ncomp, deg, form, exchange, e, blocks, s);
+    return fp64 ? ens_comp<double>(ncomp, deg, form, e, blocks, s)
+                : ens_comp<float>(ncomp, deg, form, e, blocks, s);
 }
 
 hipError_t launch_advance_base(int *base, int by, hipStream_t s)

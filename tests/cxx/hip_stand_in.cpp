@@ -174,7 +174,7 @@ hipError_t launch_adjoint(int, int, const AdjArgs &, hipStream_t) { return hipSu
 hipError_t launch_advance_base(int *, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_set_base(int *, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_aux(int, int, const AuxArgs &, hipStream_t) { return hipSuccess; }
-hipError_t launch_ensemble_sweep(int, int, int, int, int, const EnsembleArgs &, int, hipStream_t) { return hipSuccess; }
+hipError_t launch_ensemble_sweep(int, int, int, int, const EnsembleArgs &, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_fill_tf(int, const Geometry &, const Tables &, const Physics &, int, const FillArgs &, void *, hipStream_t)
 {
     return hipSuccess;
