@@ -300,7 +300,7 @@ __device__ __forceinline__ void face_lanes(const Geometry &g, const LaneCoord &l
 // 38.1 -> 35.3, 16^3 4.4 -> 3.9.  One component loses (98 -> 123: too little work per wave for the
 // barrier) but gains 5% from the numbering alone.  Whole cells in one workgroup (12 waves) lost
 // 10% (fewer workgroups fit a CU); pairs and paths of four in A15, C15 and Z, which have no such
-// rings, gained nothing.
+// rings, gained nothing.  The reverse sweeps (k_adjoint) and the ensemble's kernel do without: both lose by it.
 // The barrier waits for LDS only (a __syncthreads would also wait for the loads in flight).  Every
 // wave of the workgroup has to arrive.
 __device__ __forceinline__ void exchange_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

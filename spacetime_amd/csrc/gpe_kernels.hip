@@ -639,9 +639,9 @@ __device__ __forceinline__ bool decode_reduce(const Geometry &g, int segs, unsig
     return true;
 }
 
-// FP64 observables of a level.  Vector instructions bind it, not bytes: spin-1 128^3 FP32 reads
-// 604 MB (92 us at the copy rate) and issues 98 M of them (159 us at 4 cycles a wave and SIMD), in
-// 241 us of kernel time; 770 us with one unknown a lane and an exchange per wave of 64.  So:
+// FP64 observables of a level.  Spin-1 128^3 FP32 issues 98 M vector instructions (159 us at 4 cycles a wave
+// and SIMD) and misses L2 for 1.18 GB, twice the level (177 us at the copy rate), which 4 waves a SIMD
+// overlap in part: 282 us of kernel time, 770 us with one unknown a lane and an exchange per wave of 64.  So:
 //   * a lane keeps its 14 sums over all the unknowns it takes and the wave exchanges them once;
 //   * the kinetic energy is summed over the faces, each once: with dv_i w_ij = dv_j w_ji (the dual
 //     volumes are solved from it) Re sum_i dv_i psi_i* sum_j w_ij (psi_j - psi_i) is
